@@ -220,7 +220,6 @@ struct mhip_nlist {
     uint32_t *idx = nullptr;      // column-major [k][nq] sorted-space neighbour indices
     float *d2 = nullptr;          // column-major [k][nq] squared distances
     float *tau = nullptr;         // k-th squared distance per slot
-    int32_t *nlt = nullptr;       // count strictly below tau per slot
     float *h = nullptr;           // smoothing length per slot (float32 copy of h64)
     double *h64 = nullptr;        // smoothing length per slot, refined in float64
     int32_t *status = nullptr;    // per slot

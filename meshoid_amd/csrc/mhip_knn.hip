@@ -37,6 +37,7 @@
 //           so neighbour sets equal the float64 kNN except for float64 ties.
 #include "../../include/meshoid_hip.h"
 #include "mhip_internal.hpp"
+#include "mhip_knn.hpp"
 #include "mhip_sortnet.hpp"
 
 namespace mhip {
@@ -45,126 +46,9 @@ constexpr int KNN_BLOCK = 256;
 constexpr int KNN_WAVES = KNN_BLOCK / WAVE;
 constexpr int QCAP = 32;                     // per-lane pending-candidate queue
 constexpr int WLCAP = 384;                   // per-wave record of candidate leaves
-constexpr float U32 = 5.9604645e-8f;         // 2^-24
-constexpr float AMBIG_REL = 12.0f * U32;     // fp32 vs fp64 ordering ambiguity of d^2
-constexpr float BAND_REL = 16.0f * U32;      // resolver band half-width
-constexpr float PRUNE_REL = 1.0f + 1e-5f;    // box-test safety factor
 constexpr int BAND_CAP = 32;
 constexpr int64_t RESOLVE_WAVES = 8192;      // resolver grid (one wavefront per ambiguous slot)
 
-struct TreeView {
-    const float *sx, *sy, *sz, *lx, *ly, *lz;
-    const float *nodes;
-    int64_t first_leaf, nleaf;
-    float box, half;  // periodic box length and half of it (0: open)
-    float slack;      // absolute box-test slack: 0 for float32 inputs, covers
-                      // the float32 residuals of float64 inputs otherwise
-    int depth;        // level of the leaves (root = level 0)
-};
-
-struct QPos {
-    float x, y, z, lx, ly, lz;
-};
-
-template <bool P64>
-MHIP_DEV QPos load_q(const TreeView &t, uint32_t p) {
-    QPos q;
-    q.x = t.sx[p];
-    q.y = t.sy[p];
-    q.z = t.sz[p];
-    q.lx = P64 ? t.lx[p] : 0.f;
-    q.ly = P64 ? t.ly[p] : 0.f;
-    q.lz = P64 ? t.lz[p] : 0.f;
-    return q;
-}
-
-// Offset c - q along one axis.  Periodic: the nearest image is formed by
-// moving whichever coordinate lies in the far half by one box length; that
-// subtraction (x - box with box/2 <= x < box) is exact (Sterbenz), so the
-// wrapped offset carries a single rounding, like an unwrapped one.
-template <bool PER>
-MHIP_DEV float axis_off(float c, float q, float box, float half) {
-    const float d = c - q;
-    if (!PER) return d;
-    const float up = (c - box) - q;  // image of c one box lower (c in the far half)
-    const float dn = c - (q - box);  // image of c one box higher (q in the far half)
-    return d > half ? up : (d < -half ? dn : d);
-}
-
-// squared distance, float32, fixed operation order (shared by every pass so
-// that the same pair always yields the same bits)
-template <bool PER, bool P64>
-MHIP_DEV float dist2(const TreeView &t, const QPos &q, float cx, float cy, float cz, float clx,
-                     float cly, float clz) {
-    float dx = axis_off<PER>(cx, q.x, t.box, t.half);
-    float dy = axis_off<PER>(cy, q.y, t.box, t.half);
-    float dz = axis_off<PER>(cz, q.z, t.box, t.half);
-    if (P64) {
-        dx = dx + (clx - q.lx);
-        dy = dy + (cly - q.ly);
-        dz = dz + (clz - q.lz);
-    }
-    return fmaf(dz, dz, fmaf(dy, dy, dx * dx));
-}
-
-template <bool PER>
-MHIP_DEV float axis_gap(float q, float lo, float hi, float box, float slack) {
-    float g = fmaxf(lo - q, q - hi);
-    if (PER) {
-        // the box one period lower / higher
-        g = fminf(g, fmaxf((lo - box) - q, q - (hi - box)));
-        g = fminf(g, fmaxf(lo - (q - box), (q - box) - hi));
-    }
-    return fmaxf(g - slack, 0.f);
-}
-
-// lower bound of the squared distance from q to any particle under node x
-template <bool PER>
-MHIP_DEV float node_d2(const TreeView &t, const QPos &q, uint32_t x) {
-    const float4 *nb = (const float4 *)(t.nodes + (int64_t)x * 8);
-    const float4 a = nb[0], b = nb[1];  // lo xyz, hi x | hi yz
-    const float dx = axis_gap<PER>(q.x, a.x, a.w, t.box, t.slack);
-    const float dy = axis_gap<PER>(q.y, a.y, b.x, t.box, t.slack);
-    const float dz = axis_gap<PER>(q.z, a.z, b.y, t.box, t.slack);
-    return fmaf(dz, dz, fmaf(dy, dy, dx * dx));
-}
-
-// next node in depth-first order after the subtree of x is finished; false
-// at the end of the traversal (children of p are 8p+1..8p+8)
-MHIP_DEV bool next_after(uint32_t &x) {
-    while (x != 0 && (x & (FANOUT - 1)) == 0) x = (x - 1) >> 3;
-    if (x == 0) return false;
-    x++;
-    return true;
-}
-
-// one leaf's candidates of this lane (per-lane gathers, 64-byte aligned)
-template <bool P64>
-MHIP_DEV void load_leaf(const TreeView &t, int64_t leaf, float (&cx)[LEAF], float (&cy)[LEAF],
-                        float (&cz)[LEAF], float (&clx)[LEAF], float (&cly)[LEAF], float (&clz)[LEAF]) {
-    const int64_t base = leaf * LEAF;
-#pragma unroll
-    for (int v = 0; v < LEAF / 4; v++) {
-        const float4 X = ((const float4 *)(t.sx + base))[v];
-        const float4 Y = ((const float4 *)(t.sy + base))[v];
-        const float4 Z = ((const float4 *)(t.sz + base))[v];
-        cx[4 * v] = X.x, cx[4 * v + 1] = X.y, cx[4 * v + 2] = X.z, cx[4 * v + 3] = X.w;
-        cy[4 * v] = Y.x, cy[4 * v + 1] = Y.y, cy[4 * v + 2] = Y.z, cy[4 * v + 3] = Y.w;
-        cz[4 * v] = Z.x, cz[4 * v + 1] = Z.y, cz[4 * v + 2] = Z.z, cz[4 * v + 3] = Z.w;
-        if (P64) {
-            const float4 LX = ((const float4 *)(t.lx + base))[v];
-            const float4 LY = ((const float4 *)(t.ly + base))[v];
-            const float4 LZ = ((const float4 *)(t.lz + base))[v];
-            clx[4 * v] = LX.x, clx[4 * v + 1] = LX.y, clx[4 * v + 2] = LX.z, clx[4 * v + 3] = LX.w;
-            cly[4 * v] = LY.x, cly[4 * v + 1] = LY.y, cly[4 * v + 2] = LY.z, cly[4 * v + 3] = LY.w;
-            clz[4 * v] = LZ.x, clz[4 * v + 1] = LZ.y, clz[4 * v + 2] = LZ.z, clz[4 * v + 3] = LZ.w;
-        } else {
-            clx[4 * v] = clx[4 * v + 1] = clx[4 * v + 2] = clx[4 * v + 3] = 0.f;
-            cly[4 * v] = cly[4 * v + 1] = cly[4 * v + 2] = cly[4 * v + 3] = 0.f;
-            clz[4 * v] = clz[4 * v + 1] = clz[4 * v + 2] = clz[4 * v + 3] = 0.f;
-        }
-    }
-}
 
 // Inserts x into the ascending list A, dropping the largest entry: slot j
 // becomes med3(A[j-1], x, A[j]).  The slots are updated in place from the top
@@ -179,41 +63,6 @@ MHIP_DEV void insert_sorted(float (&A)[KCAP], float x) {
     asm volatile("v_min_f32 %0, %1, %0" : "+v"(A[0]) : "v"(x));
 }
 
-MHIP_DEV int wave_max(int v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o));
-    return (int)uniform((uint32_t)v);
-}
-
-MHIP_DEV uint32_t wave_sum(uint32_t v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    return v;
-}
-
-struct KnnArgs {
-    TreeView t;
-    const uint32_t *qsorted;  // null: slot q is sorted particle q
-    const uint32_t *qrow;     // null: row = perm[q]
-    const uint32_t *perm;
-    int64_t nq, n;
-    int k, dim;
-    const float *seed_h;   // Newton seed per output row, null = none
-    const float *seed_r;   // search-radius bound per output row, null = none
-    int redo;              // 1: second launch, redo waves with a radius-seed miss
-    int32_t *status_out;
-    // per slot state
-    float *tau;
-    int32_t *nlt;
-    float *h_slot;
-    double *h64_slot;
-    int32_t *st_slot;
-    uint32_t *nl_idx;
-    float *nl_d2;
-    unsigned long long *stats;  // work counters, may be null
-    uint32_t *amb;              // [0] count, [1..] ambiguous slots
-    uint32_t wlcap;             // leaf-record capacity used (<= WLCAP; smaller only as a test hook)
-};
 
 MHIP_DEV int64_t slot_of_lane(int64_t *first) {
     const uint32_t b = xcd_remap(blockIdx.x, gridDim.x);
@@ -222,62 +71,6 @@ MHIP_DEV int64_t slot_of_lane(int64_t *first) {
     return wave0 + (threadIdx.x & (WAVE - 1));
 }
 
-MHIP_DEV void pad_list(const KnnArgs &a, int cnt, uint32_t qp, int64_t slot) {
-    // never leave undefined indices behind: pad with the query itself
-    for (int j = cnt; j < a.k; j++) {
-        a.nl_idx[(int64_t)j * a.nq + slot] = qp;
-        if (a.nl_d2) a.nl_d2[(int64_t)j * a.nq + slot] = INFINITY;
-    }
-}
-
-// One float64 Newton step on the smoothing length over the final member
-// list, member(j) giving the sorted index of member j < k.  The float32
-// solve below is at the float32 noise floor (relative error up to ~2.4e-7,
-// from the float32 distances); the derivative fits are sensitive to h through
-// the weights of the outermost neighbours (d ln W / d ln h = 3q / (1 - q) as
-// q -> 1), so a 2.4e-7 error of h moves second-order derivatives by up to
-// ~6e-5, and first-order derivatives of rough fields by ~4e-5, on
-// well-conditioned rows.  One step on the exact float64 pair distances
-// (float32 positions are exact in float64; float64 inputs are hi + lo) takes
-// h to ~1e-13 of the root of norm_d sum_j W(r_j / h) = k
-// (kernel_density.py:36-56).  A step beyond 1e-4 h means the float32 solve
-// did not converge; h is then kept.
-template <bool PER, bool P64, typename F>
-MHIP_DEV double refine_h64(const KnnArgs &a, const QPos &q, double hd, F member) {
-    const double qx = (double)q.x + (double)q.lx, qy = (double)q.y + (double)q.ly, qz = (double)q.z + (double)q.lz;
-    const double box = (double)a.t.box, ih = 1.0 / hd;
-    double sw = 0.0, sd = 0.0;
-    for (int j = 0; j < a.k; j++) {
-        const uint32_t p = member(j);
-        double d[3] = {(double)a.t.sx[p] - qx, (double)a.t.sy[p] - qy, (double)a.t.sz[p] - qz};
-        if (P64) {
-            d[0] += (double)a.t.lx[p];
-            d[1] += (double)a.t.ly[p];
-            d[2] += (double)a.t.lz[p];
-        }
-        if (PER) {
-#pragma unroll
-            for (int c = 0; c < 3; c++) d[c] = wrap<double>(d[c], box);
-        }
-        const double qq = sqrt(d[0] * d[0] + d[1] * d[1] + d[2] * d[2]) * ih;
-        double w, dw;
-        kernel_w_dw<double>(qq, w, dw);
-        sw += w;
-        sd += qq <= 1.0 ? dw * qq : 0.0;
-    }
-    const double norm = hsml_norm(a.dim);
-    // n(h) grows with h: dn/dh = -norm sum_j W'(q_j) q_j / h > 0
-    const double fn = norm * sw - (double)a.k, dndh = -norm * sd * ih;
-    const double hn = hd - fn / dndh;
-    return (dndh > 0.0 && fabs(hn - hd) <= 1e-4 * hd) ? hn : hd;
-}
-
-// smoothing length of one query slot (float32 copy and float64); the
-// row-order h, density and volume are formed from it by k_rows_out
-MHIP_DEV void write_h(const KnnArgs &a, int64_t slot, double h) {
-    a.h_slot[slot] = (float)h;
-    a.h64_slot[slot] = h;
-}
 
 // ---------------------------------------------------------------------------
 // smoothing length on the k nearest distances (kernel_density.py:36-56 root):
@@ -672,9 +465,6 @@ __global__ __launch_bounds__(KNN_BLOCK) void k_knn_main(KnnArgs a) {
         return;
     }
     if (tau1 <= tau * (1.0f + AMBIG_REL)) st |= ST_AMBIGUOUS;
-    int nlt = 0;
-#pragma unroll
-    for (int j = 0; j < KCAP - 1; j++) nlt += (A[j] >= 0.f && A[j] < tau);
     const float seed = a.seed_h ? a.seed_h[row] : 0.f;
     int n_newton = 0;
     const float h = hsml_solve<KCAP>(A, a.k, a.dim, seed, st, n_newton);
@@ -690,7 +480,6 @@ __global__ __launch_bounds__(KNN_BLOCK) void k_knn_main(KnnArgs a) {
     }
     if (live) {
         a.tau[slot] = tau;
-        a.nlt[slot] = nlt;
     }
     double h64 = (double)h;
     // members: a candidate at or below tau passed its lane's queue filter
@@ -1104,7 +893,7 @@ static int nl_reserve(mhip_ctx *ctx, mhip_nlist *nl, int64_t nq, int k) {
     int rc = 0;
     if (nl->cap < nq || nl->k < k) {
         void **arr[] = {(void **)&nl->qsorted, (void **)&nl->qrow, (void **)&nl->tau,
-                        (void **)&nl->nlt,     (void **)&nl->h,    (void **)&nl->status};
+                        (void **)&nl->h,       (void **)&nl->status};
         for (auto p : arr)
             if ((rc = nl_grow(ctx, p, nq * 4))) return rc;
         if ((rc = nl_grow(ctx, (void **)&nl->rowrec, nq * 16))) return rc;
@@ -1195,7 +984,6 @@ int knn_run(mhip_ctx *ctx, const mhip_index *ix, const int64_t *qidx, int64_t nq
     a.redo = 0;
     a.status_out = status_out;
     a.tau = nl->tau;
-    a.nlt = nl->nlt;
     a.h_slot = nl->h;
     a.h64_slot = nl->h64;
     a.st_slot = nl->status;
@@ -1210,22 +998,28 @@ int knn_run(mhip_ctx *ctx, const mhip_index *ix, const int64_t *qidx, int64_t nq
     hipLaunchKernelGGL(k_amb_reset, dim3(1), dim3(64), 0, s, nl->amb);
     const int need = k + 1;
     ProfRegion pr1(ctx, "knn_main");
-    if (need <= 5)
-        launch_main<5>(a, per, p64, g, s);
-    else if (need <= 9)
-        launch_main<9>(a, per, p64, g, s);
-    else if (need <= 17)
-        launch_main<17>(a, per, p64, g, s);
-    else if (need <= 21)
-        launch_main<21>(a, per, p64, g, s);
-    else if (need <= 33)
-        launch_main<33>(a, per, p64, g, s);
-    else if (need <= 65)
-        launch_main<65>(a, per, p64, g, s);
-    else if (need <= 101)
-        launch_main<101>(a, per, p64, g, s);
-    else
-        launch_main<129>(a, per, p64, g, s);
+    // seeds and the leaf-record test hook belong to the main kernel
+    const bool wave = !seed_h && !seed_r && !(flags & MHIP_KNN_SMALL_RECORD) && knn_wave_serves(ix->n, nq, k);
+    if (wave) {
+        if ((rc = knn_wave_launch(ctx, a, per, p64))) return rc;
+    } else {
+        if (need <= 5)
+            launch_main<5>(a, per, p64, g, s);
+        else if (need <= 9)
+            launch_main<9>(a, per, p64, g, s);
+        else if (need <= 17)
+            launch_main<17>(a, per, p64, g, s);
+        else if (need <= 21)
+            launch_main<21>(a, per, p64, g, s);
+        else if (need <= 33)
+            launch_main<33>(a, per, p64, g, s);
+        else if (need <= 65)
+            launch_main<65>(a, per, p64, g, s);
+        else if (need <= 101)
+            launch_main<101>(a, per, p64, g, s);
+        else
+            launch_main<129>(a, per, p64, g, s);
+    }
     if (seed_r) {
         // second launch: waves with a radius-seed miss are recomputed plainly
         KnnArgs r = a;
@@ -1310,10 +1104,10 @@ __global__ __launch_bounds__(256) void k_export(const uint32_t *__restrict__ idx
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void k_nl_subset(
     const uint32_t *__restrict__ fidx, const float *__restrict__ fd2, const float *__restrict__ ftau,
-    const int32_t *__restrict__ fnlt, const float *__restrict__ fh, const double *__restrict__ fh64,
+    const float *__restrict__ fh, const double *__restrict__ fh64,
     const int32_t *__restrict__ fst, int64_t nfull, const uint32_t *__restrict__ qsorted,
     const uint32_t *__restrict__ qrow, int64_t nq, int k, int dim, const double *__restrict__ m_rows,
-    uint32_t *__restrict__ idx, float *__restrict__ d2, float *__restrict__ tau, int32_t *__restrict__ nlt,
+    uint32_t *__restrict__ idx, float *__restrict__ d2, float *__restrict__ tau,
     float *__restrict__ hs, double *__restrict__ hs64, int32_t *__restrict__ st, float *__restrict__ h_out,
     float *__restrict__ rho_out, float *__restrict__ vol_out, int32_t *__restrict__ status_out) {
     const int64_t s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
@@ -1325,7 +1119,6 @@ __global__ __launch_bounds__(256) void k_nl_subset(
     }
     const double h = fh64[f];
     tau[s] = ftau[f];
-    nlt[s] = fnlt[f];
     hs[s] = fh[f];
     hs64[s] = h;
     st[s] = fst[f];
@@ -1358,9 +1151,9 @@ int nlist_subset(mhip_ctx *ctx, const mhip_nlist *full, const int64_t *qidx, int
     if ((rc = query_setup(ctx, ix, qidx, nq, nl))) return rc;
     ProfRegion pr(ctx, "nlist_subset");
     hipLaunchKernelGGL(k_nl_subset, dim3((unsigned)((nq + 255) / 256)), dim3(256), 0, ctx->stream, full->idx,
-                       full->has_d2 ? full->d2 : nullptr, full->tau, full->nlt, full->h, full->h64, full->status,
+                       full->has_d2 ? full->d2 : nullptr, full->tau, full->h, full->h64, full->status,
                        full->nq, nl->qsorted, nl->qrow, nq, k, ix->dim, m_rows, nl->idx,
-                       full->has_d2 ? nl->d2 : nullptr, nl->tau, nl->nlt, nl->h, nl->h64, nl->status, h_out, rho_out,
+                       full->has_d2 ? nl->d2 : nullptr, nl->tau, nl->h, nl->h64, nl->status, h_out, rho_out,
                        vol_out, status_out);
     return check_hip(ctx, hipGetLastError(), "subset launch");
 }

@@ -1,0 +1,257 @@
+// Shared by the kNN kernels (mhip_knn.hip: one lane per query; mhip_knn_wave.hip:
+// one wavefront per query): tree view, float32 distances and box gaps, float64
+// refinement of the smoothing length.
+#pragma once
+#include "mhip_internal.hpp"
+
+namespace mhip {
+
+constexpr float U32 = 5.9604645e-8f;         // 2^-24
+constexpr float AMBIG_REL = 12.0f * U32;     // fp32 vs fp64 ordering ambiguity of d^2
+constexpr float BAND_REL = 16.0f * U32;      // resolver band half-width
+constexpr float PRUNE_REL = 1.0f + 1e-5f;    // box-test safety factor
+
+struct TreeView {
+    const float *sx, *sy, *sz, *lx, *ly, *lz;
+    const float *nodes;
+    int64_t first_leaf, nleaf;
+    float box, half;  // periodic box length and half of it (0: open)
+    float slack;      // absolute box-test slack: 0 for float32 inputs, covers
+                      // the float32 residuals of float64 inputs otherwise
+    int depth;        // level of the leaves (root = level 0)
+};
+
+struct QPos {
+    float x, y, z, lx, ly, lz;
+};
+
+template <bool P64>
+MHIP_DEV QPos load_q(const TreeView &t, uint32_t p) {
+    QPos q;
+    q.x = t.sx[p];
+    q.y = t.sy[p];
+    q.z = t.sz[p];
+    q.lx = P64 ? t.lx[p] : 0.f;
+    q.ly = P64 ? t.ly[p] : 0.f;
+    q.lz = P64 ? t.lz[p] : 0.f;
+    return q;
+}
+
+// Offset c - q along one axis.  Periodic: the nearest image is formed by
+// moving whichever coordinate lies in the far half by one box length; that
+// subtraction (x - box with box/2 <= x < box) is exact (Sterbenz), so the
+// wrapped offset carries a single rounding, like an unwrapped one.
+template <bool PER>
+MHIP_DEV float axis_off(float c, float q, float box, float half) {
+    const float d = c - q;
+    if (!PER) return d;
+    const float up = (c - box) - q;  // image of c one box lower (c in the far half)
+    const float dn = c - (q - box);  // image of c one box higher (q in the far half)
+    return d > half ? up : (d < -half ? dn : d);
+}
+
+// squared distance, float32, fixed operation order (shared by every pass so
+// that the same pair always yields the same bits)
+template <bool PER, bool P64>
+MHIP_DEV float dist2(const TreeView &t, const QPos &q, float cx, float cy, float cz, float clx,
+                     float cly, float clz) {
+    float dx = axis_off<PER>(cx, q.x, t.box, t.half);
+    float dy = axis_off<PER>(cy, q.y, t.box, t.half);
+    float dz = axis_off<PER>(cz, q.z, t.box, t.half);
+    if (P64) {
+        dx = dx + (clx - q.lx);
+        dy = dy + (cly - q.ly);
+        dz = dz + (clz - q.lz);
+    }
+    return fmaf(dz, dz, fmaf(dy, dy, dx * dx));
+}
+
+template <bool PER>
+MHIP_DEV float axis_gap(float q, float lo, float hi, float box, float slack) {
+    float g = fmaxf(lo - q, q - hi);
+    if (PER) {
+        // the box one period lower / higher
+        g = fminf(g, fmaxf((lo - box) - q, q - (hi - box)));
+        g = fminf(g, fmaxf(lo - (q - box), (q - box) - hi));
+    }
+    return fmaxf(g - slack, 0.f);
+}
+
+// lower bound of the squared distance from q to any particle under node x
+template <bool PER>
+MHIP_DEV float node_d2(const TreeView &t, const QPos &q, uint32_t x) {
+    const float4 *nb = (const float4 *)(t.nodes + (int64_t)x * 8);
+    const float4 a = nb[0], b = nb[1];  // lo xyz, hi x | hi yz
+    const float dx = axis_gap<PER>(q.x, a.x, a.w, t.box, t.slack);
+    const float dy = axis_gap<PER>(q.y, a.y, b.x, t.box, t.slack);
+    const float dz = axis_gap<PER>(q.z, a.z, b.y, t.box, t.slack);
+    return fmaf(dz, dz, fmaf(dy, dy, dx * dx));
+}
+
+// next node in depth-first order after the subtree of x is finished; false
+// at the end of the traversal (children of p are 8p+1..8p+8)
+MHIP_DEV bool next_after(uint32_t &x) {
+    while (x != 0 && (x & (FANOUT - 1)) == 0) x = (x - 1) >> 3;
+    if (x == 0) return false;
+    x++;
+    return true;
+}
+
+// one leaf's candidates of this lane (per-lane gathers, 64-byte aligned)
+template <bool P64>
+MHIP_DEV void load_leaf(const TreeView &t, int64_t leaf, float (&cx)[LEAF], float (&cy)[LEAF],
+                        float (&cz)[LEAF], float (&clx)[LEAF], float (&cly)[LEAF], float (&clz)[LEAF]) {
+    const int64_t base = leaf * LEAF;
+#pragma unroll
+    for (int v = 0; v < LEAF / 4; v++) {
+        const float4 X = ((const float4 *)(t.sx + base))[v];
+        const float4 Y = ((const float4 *)(t.sy + base))[v];
+        const float4 Z = ((const float4 *)(t.sz + base))[v];
+        cx[4 * v] = X.x, cx[4 * v + 1] = X.y, cx[4 * v + 2] = X.z, cx[4 * v + 3] = X.w;
+        cy[4 * v] = Y.x, cy[4 * v + 1] = Y.y, cy[4 * v + 2] = Y.z, cy[4 * v + 3] = Y.w;
+        cz[4 * v] = Z.x, cz[4 * v + 1] = Z.y, cz[4 * v + 2] = Z.z, cz[4 * v + 3] = Z.w;
+        if (P64) {
+            const float4 LX = ((const float4 *)(t.lx + base))[v];
+            const float4 LY = ((const float4 *)(t.ly + base))[v];
+            const float4 LZ = ((const float4 *)(t.lz + base))[v];
+            clx[4 * v] = LX.x, clx[4 * v + 1] = LX.y, clx[4 * v + 2] = LX.z, clx[4 * v + 3] = LX.w;
+            cly[4 * v] = LY.x, cly[4 * v + 1] = LY.y, cly[4 * v + 2] = LY.z, cly[4 * v + 3] = LY.w;
+            clz[4 * v] = LZ.x, clz[4 * v + 1] = LZ.y, clz[4 * v + 2] = LZ.z, clz[4 * v + 3] = LZ.w;
+        } else {
+            clx[4 * v] = clx[4 * v + 1] = clx[4 * v + 2] = clx[4 * v + 3] = 0.f;
+            cly[4 * v] = cly[4 * v + 1] = cly[4 * v + 2] = cly[4 * v + 3] = 0.f;
+            clz[4 * v] = clz[4 * v + 1] = clz[4 * v + 2] = clz[4 * v + 3] = 0.f;
+        }
+    }
+}
+
+MHIP_DEV int wave_max(int v) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o));
+    return (int)uniform((uint32_t)v);
+}
+
+MHIP_DEV uint32_t wave_sum(uint32_t v) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+    return v;
+}
+
+struct KnnArgs {
+    TreeView t;
+    const uint32_t *qsorted;  // null: slot q is sorted particle q
+    const uint32_t *qrow;     // null: row = perm[q]
+    const uint32_t *perm;
+    int64_t nq, n;
+    int k, dim;
+    const float *seed_h;   // Newton seed per output row, null = none
+    const float *seed_r;   // search-radius bound per output row, null = none
+    int redo;              // 1: second launch, redo waves with a radius-seed miss
+    int32_t *status_out;
+    // per slot state
+    float *tau;
+    float *h_slot;
+    double *h64_slot;
+    int32_t *st_slot;
+    uint32_t *nl_idx;
+    float *nl_d2;
+    unsigned long long *stats;  // work counters, may be null
+    uint32_t *amb;              // [0] count, [1..] ambiguous slots
+    uint32_t wlcap;             // leaf-record capacity used (<= WLCAP; smaller only as a test hook)
+};
+
+MHIP_DEV void pad_list(const KnnArgs &a, int cnt, uint32_t qp, int64_t slot) {
+    // never leave undefined indices behind: pad with the query itself
+    for (int j = cnt; j < a.k; j++) {
+        a.nl_idx[(int64_t)j * a.nq + slot] = qp;
+        if (a.nl_d2) a.nl_d2[(int64_t)j * a.nq + slot] = INFINITY;
+    }
+}
+
+// |d| from r2 = |d|^2 (float64): the hardware reciprocal square root and one
+// Newton step on the root give ~1e-16 relative error without the correctly
+// rounded expansion's scaling and fix-up instructions.  Tiny r2 (float64
+// inputs at pathological scales, where the estimate would meet denormals)
+// take sqrt.
+MHIP_DEV double pair_dist(double r2) {
+    if (r2 < 1e-280) return sqrt(r2);
+    const double y = __builtin_amdgcn_rsq(r2);
+    const double r = r2 * y;
+    const double res = fma(-r, r, r2);
+    return fma(0.5 * y, res, r);
+}
+
+// float64 offset of member p from the query: exact for float32 positions,
+// hi + lo for float64 inputs, minimum image when periodic
+template <bool PER, bool P64>
+MHIP_DEV double member_dist(const TreeView &t, const QPos &q, uint32_t p) {
+    double d[3] = {(double)t.sx[p] - ((double)q.x + (double)q.lx), (double)t.sy[p] - ((double)q.y + (double)q.ly),
+                   (double)t.sz[p] - ((double)q.z + (double)q.lz)};
+    if (P64) {
+        d[0] += (double)t.lx[p];
+        d[1] += (double)t.ly[p];
+        d[2] += (double)t.lz[p];
+    }
+    if (PER) {
+        const double box = (double)t.box;
+#pragma unroll
+        for (int c = 0; c < 3; c++) d[c] = wrap<double>(d[c], box);
+    }
+    return pair_dist(d[0] * d[0] + d[1] * d[1] + d[2] * d[2]);
+}
+
+// One float64 step on the smoothing length over the final member list.  The
+// float32 solve before it is at the float32 noise floor (relative error up to
+// ~3e-7, from the float32 distances); the derivative fits are sensitive to h
+// through the weights of the outermost neighbours (d ln W / d ln h =
+// 3q / (1 - q) as q -> 1), so a 2.4e-7 error of h moves second-order
+// derivatives by up to ~6e-5.  The spline as truncated powers, W = 2 a^3 - b^3
+// with a = (1 - q)_+ and b = (1 - 2q)_+, gives W' = -6 (a^2 - b^2) and
+// W'' = 12 a - 24 b without branches, so Halley's step (cubic: third
+// derivatives of W are bounded) costs two more operations per neighbour than
+// Newton's and leaves h at the rounding level of the float64 sums instead of
+// at ~(3e-7)^2.
+struct HsmlSums {
+    double w = 0.0, d1 = 0.0, d2 = 0.0;  // sums of W / 2, -W' q / 6, W'' q^2 / 12
+    MHIP_DEV void add(double q) {
+        const double a = fmax(1.0 - q, 0.0), b = fmax(fma(-2.0, q, 1.0), 0.0);
+        const double aa = a * a, bb = b * b, qc = fmin(q, 1.0);
+        w += fma(-0.5 * b, bb, a * aa);
+        const double t = (aa - bb) * qc;
+        d1 += t;
+        d2 = fma(fma(-2.0, b, a) * qc, qc, d2);
+    }
+};
+
+// the step from hd; a step beyond 1e-4 h means the float32 solve did not
+// converge: h is then kept
+MHIP_DEV double hsml_step64(const HsmlSums &s, double hd, int k, int dim) {
+    const double norm = hsml_norm(dim);
+    // n(h) = norm sum W(r_j / h) grows with h; p = h n'(h), c = h^2 n''(h)
+    const double f = norm * (2.0 * s.w) - (double)k;
+    const double p = norm * 6.0 * s.d1, c = norm * 12.0 * (s.d2 - s.d1);
+    const double rel = 2.0 * f * p / (2.0 * p * p - f * c);
+    return (p > 0.0 && fabs(rel) <= 1e-4) ? hd - hd * rel : hd;
+}
+
+// the whole step by one lane, member(j) giving the sorted index of member j < k
+template <bool PER, bool P64, typename F>
+MHIP_DEV double refine_h64(const KnnArgs &a, const QPos &q, double hd, F member) {
+    const double ih = 1.0 / hd;
+    HsmlSums s;
+    for (int j = 0; j < a.k; j++) s.add(member_dist<PER, P64>(a.t, q, member(j)) * ih);
+    return hsml_step64(s, hd, a.k, a.dim);
+}
+
+// smoothing length of one query slot (float32 copy and float64); the
+// row-order h, density and volume are formed from it by k_rows_out
+MHIP_DEV void write_h(const KnnArgs &a, int64_t slot, double h) {
+    a.h_slot[slot] = (float)h;
+    a.h64_slot[slot] = h;
+}
+
+// one wavefront per query (mhip_knn_wave.hip)
+bool knn_wave_serves(int64_t n, int64_t nq, int k);
+int knn_wave_launch(mhip_ctx *ctx, const KnnArgs &a, bool per, bool p64);
+
+}  // namespace mhip
