@@ -45,7 +45,10 @@ namespace mhip {
 constexpr int KNN_BLOCK = 256;
 constexpr int KNN_WAVES = KNN_BLOCK / WAVE;
 constexpr int QCAP = 32;                     // per-lane pending-candidate queue
-constexpr int WLCAP = 384;                   // per-wave record of candidate leaves
+constexpr int WLCAP = 128;                   // per-wave record of candidate leaves
+constexpr int WLWORDS = WLCAP / 32;
+static_assert(WLWORDS == 4, "the member pass reads the masks as two pairs");
+constexpr uint32_t INF_BITS = 0x7f800000u;   // +inf
 constexpr int BAND_CAP = 32;
 constexpr int64_t RESOLVE_WAVES = 8192;      // resolver grid (one wavefront per ambiguous slot)
 
@@ -64,6 +67,31 @@ MHIP_DEV void insert_sorted(float (&A)[KCAP], float x) {
 }
 
 
+// LDS rows are ROW_STEP bytes apart (one float per lane)
+constexpr uint32_t ROW_STEP = WAVE * 4;
+
+// LDS byte address of a shared variable, and a store there
+MHIP_DEV uint32_t lds_address(uint32_t *p) { return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint32_t *)p; }
+MHIP_DEV void lds_store(uint32_t addr, uint32_t v) { *(__attribute__((address_space(3))) uint32_t *)(uintptr_t)addr = v; }
+
+// row address ra of the lanes with a < b (or a <= b) moves on by one row: the
+// compare writes EXEC, the addition runs under it, and the wavefront's EXEC
+// (all) comes back.  Two vector instructions per candidate; a compare into a
+// mask, a select and an addition are three, and a row counter with the
+// address formed from it four.
+MHIP_DEV void advance_lt(uint32_t &ra, float a, float b, uint64_t all) {
+    asm volatile("v_cmpx_lt_f32 vcc, %1, %2\n\tv_add_u32 %0, %3, %0\n\ts_mov_b64 exec, %4"
+                 : "+v"(ra)
+                 : "v"(a), "v"(b), "s"(ROW_STEP), "s"(all)
+                 : "vcc");
+}
+MHIP_DEV void advance_le(uint32_t &ra, float a, float b, uint64_t all) {
+    asm volatile("v_cmpx_le_f32 vcc, %1, %2\n\tv_add_u32 %0, %3, %0\n\ts_mov_b64 exec, %4"
+                 : "+v"(ra)
+                 : "v"(a), "v"(b), "s"(ROW_STEP), "s"(all)
+                 : "vcc");
+}
+
 MHIP_DEV int64_t slot_of_lane(int64_t *first) {
     const uint32_t b = xcd_remap(blockIdx.x, gridDim.x);
     const int64_t wave0 = ((int64_t)b * KNN_WAVES + (threadIdx.x >> 6)) * WAVE;
@@ -74,11 +102,15 @@ MHIP_DEV int64_t slot_of_lane(int64_t *first) {
 
 // ---------------------------------------------------------------------------
 // smoothing length on the k nearest distances (kernel_density.py:36-56 root):
-// norm * sum_j W(r_j/h) = k, bracket [r_1, c_d r_{k-1}].  Safeguarded Newton
-// with compensated float32 sums; the bracket is the fallback.  On return
-// A[0..KCAP-2] hold the distances (sentinel slots +inf), not their squares:
-// the list is not needed afterwards, and reusing its registers keeps the
-// kernel's register count at that of the traversal.
+// norm * sum_j W(r_j/h) = k, bracket [r_1, c_d r_{k-1}].  Safeguarded Newton in
+// float32; the bracket is the fallback.  On return A[0..KCAP-2] hold the
+// distances (sentinel slots: larger than any), not their squares: the list is
+// not needed afterwards, and reusing its registers keeps the kernel's register
+// count at that of the traversal.  W as truncated powers (see HsmlSums): 11
+// instructions per neighbour and iteration, against ~30 with the two branches
+// of the spline and compensated sums.  The float64 step that follows is cubic,
+// so h needs to be good to ~1e-5 only: a Newton step below 1e-3 h ends the
+// solve (n(h) is C^2, the error left is of the order of the step squared).
 // ---------------------------------------------------------------------------
 template <int KCAP>
 MHIP_DEV float hsml_solve(float (&A)[KCAP], int k, int dim, float seed, int32_t &st, int &iters) {
@@ -88,7 +120,7 @@ MHIP_DEV float hsml_solve(float (&A)[KCAP], int k, int dim, float seed, int32_t 
     float lo = 0.f, rmax = 0.f;
 #pragma unroll
     for (int j = 0; j < KCAP - 1; j++) {
-        r[j] = A[j] >= 0.f ? __builtin_sqrtf(A[j]) : INFINITY;
+        r[j] = A[j] >= 0.f ? __builtin_amdgcn_sqrtf(A[j]) : 3e38f;
         if (j == e + 1) lo = r[j];
         if (j == KCAP - 2) rmax = r[j];
     }
@@ -105,38 +137,32 @@ MHIP_DEV float hsml_solve(float (&A)[KCAP], int k, int dim, float seed, int32_t 
     const float kf = (float)k;
     int it = 0;
     for (; it < 40; it++) {
-        const float ih = 1.0f / h;
-        float s = 0.f, c = 0.f, ds = 0.f;
+        const float ih = __builtin_amdgcn_rcpf(h);
+        float s = 0.f, ds = 0.f;  // sums of W / 2 and of -W' q / 6
 #pragma unroll
         for (int j = 0; j < KCAP - 1; j++) {
-            float q = r[j] * ih, w, dw;
-            kernel_w_dw(q, w, dw);
-            float y = w - c, tt = s + y;
-            c = (tt - s) - y;
-            s = tt;
-            ds += q <= 1.0f ? dw * q : 0.0f;
+            const float q = fminf(r[j] * ih, 1.0f);
+            const float a = 1.0f - q, b = fmaxf(fmaf(-2.0f, q, 1.0f), 0.f);
+            const float aa = a * a, bb = b * b;
+            s = fmaf(a, aa, s);
+            s = fmaf(-0.5f * b, bb, s);
+            ds = fmaf(aa - bb, q, ds);
             // keep the terms in order: evaluating all k kernel values ahead
             // of the sums would hold them all in registers at once
-            asm volatile("" : "+v"(s), "+v"(c), "+v"(ds));
+            asm volatile("" : "+v"(s), "+v"(ds));
         }
-        const float f = norm * s - kf;
+        const float f = fmaf(2.0f * norm, s, -kf);
         if (f == 0.f) break;
         if (f > 0.f)
             hi = h;
         else
             lo = h;
-        const float dndh = -norm * ds * ih;
-        const float step = f / dndh;
-        // n(h) is C^2 (W is C^2 at q = 1/2 and q = 1), so Newton converges
-        // quadratically: after a step below 3e-4 h the error of h - step is
-        // at the float32 noise floor (~3e-7 h with the compensated sums), and
-        // the float64 Newton step over the final members that follows
-        // (refine_h64) takes it to ~2e-13 h.  Such a step ends the
-        // solve even when it rounds onto the bracket end that h itself has
-        // just become (otherwise a converged lane would bisect the whole
-        // bracket again and hold its wavefront for ~15 more iterations).  A
-        // collapsed bracket also ends the solve.
-        if (fabsf(step) <= 3e-4f * h) {
+        const float step = f * __builtin_amdgcn_rcpf(norm * 6.0f * ds * ih);
+        // such a step ends the solve even when it rounds onto the bracket end
+        // that h itself has just become (otherwise a converged lane would
+        // bisect the whole bracket again and hold its wavefront).  A collapsed
+        // bracket also ends it.
+        if (fabsf(step) <= HSML_STEP * h) {
             h = fminf(fmaxf(h - step, lo), hi);
             break;
         }
@@ -215,14 +241,13 @@ MHIP_DEV uint32_t expand_mask(const TreeView &t, const QBox &b, uint32_t x, floa
     return m;
 }
 
-// the set bit of m nearest to position o (m != 0); ties go upwards
-MHIP_DEV uint32_t pick_nearest(uint32_t m, uint32_t o) {
-    const uint32_t up = m >> o;
-    const uint32_t down = m & ((1u << o) - 1u);
-    if (!down) return o + __builtin_ctz(up);
-    const uint32_t cd = 31u - __builtin_clz(down);
+// the set bit of m nearest to position o <= 63 (m != 0); ties go upwards
+MHIP_DEV uint32_t pick_nearest64(uint64_t m, int o) {
+    const uint64_t up = m >> o, down = m & ((1ull << o) - 1ull);
+    if (!down) return o + __builtin_ctzll(up);
+    const uint32_t cd = 63u - __builtin_clzll(down);
     if (!up) return cd;
-    const uint32_t cu = o + __builtin_ctz(up);
+    const uint32_t cu = o + __builtin_ctzll(up);
     return cu - o <= o - cd ? cu : cd;
 }
 
@@ -255,6 +280,7 @@ __global__ __launch_bounds__(KNN_BLOCK) void k_knn_main(KnnArgs a) {
     constexpr bool STAGE = KCAP <= LROWS;
     __shared__ uint32_t s_buf[KNN_WAVES][QROWS][WAVE];
     __shared__ uint32_t s_wl[KNN_WAVES][WLCAP];
+    __shared__ uint32_t s_stk[KNN_WAVES][MAX_DEPTH / 2 + 1][3];
     const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x >> 6;
     int64_t wave0;
     const int64_t slot = slot_of_lane(&wave0);
@@ -293,151 +319,228 @@ __global__ __launch_bounds__(KNN_BLOCK) void k_knn_main(KnnArgs a) {
 #pragma unroll
     for (int j = 0; j < KCAP; j++) A[j] = j < e ? -1.0f : tau0;
     float cx[LEAF], cy[LEAF], cz[LEAF], clx[LEAF], cly[LEAF], clz[LEAF];
-    uint32_t n_ins = 0, n_leaf = 0, n_nodes = 0;
-    uint32_t need_lane = 0, parent_max = 0;  // work counters (stats only)
+    uint32_t n_ins = 0, n_leaf = 0, n_nodes = 0;  // work counters
 
-    // (1) the leaves holding this wave's own queries first (they fill every
-    // list with a nearby bound), then (2) a wave-uniform depth-first traversal
-    // without a stack: expanding a node tests all 8 children against every
-    // lane's bound at once and keeps the survivors as an 8-bit mask per level;
-    // children nearest (in index) to the path of the wave's middle query are
-    // taken first.  Every candidate of a leaf is written to its lane's LDS queue
-    // row qn, and qn advances when the candidate is under the lane's current
-    // (k+1)-th distance; the queues drain into the sorted lists in batches.
-    // Leaves where some lane queued a candidate are recorded for (3).
+    // lists of at least LEAF slots take whole runs of LEAF candidates through
+    // sorting networks
+    // (longer lists, which only seeded searches and sets of 2^30 particles
+    // bring here, insert one by one)
+    constexpr bool NET = KCAP >= LEAF && KCAP <= 65;
+    // fewer queued rows than this are inserted one by one: a step costs about
+    // KCAP + 8 instructions, sorting and merging a run of 16 about 300 (KCAP
+    // 33) or 230 (KCAP 17, 21)
+    constexpr int NETMIN = 8;
+    float t1 = tau0;               // this lane's (k+1)-th distance when its queue was last drained
+    float bound = t1 * PRUNE_REL;  // of it: box tests
+    float bmax = INFINITY;         // the wavefront's largest bound
+    // this lane's queue: LDS byte addresses of its first and next row
+    const uint32_t rows0 = lds_address(&s_buf[w][0][lane]);
+    uint32_t qa = rows0;
+    bool pad = false;              // the last, NaN-padded leaf has been scanned since the last drain
+    uint32_t nwl = 0;              // recorded leaves
+    uint32_t mw[WLWORDS];          // bit r: this lane queued a candidate of recorded leaf r
+#pragma unroll
+    for (int i = 0; i < WLWORDS; i++) mw[i] = 0u;
+    const uint32_t first_leaf = (uint32_t)t.first_leaf, nleaf = (uint32_t)t.nleaf;
+    const uint32_t last_leaf = nleaf - 1;
+    const int depth = t.depth;
+
+    // (1) the leaves holding the wave's own queries, and EXT more on either
+    // side along the curve, fill the lists (two leaves more than that take
+    // tighten the outer queries' bounds, which decide how many rows the later
+    // drains insert); then (2) the rest of the tree, inside out from the
+    // middle query's leaf: its ancestor two levels up, then the rest of that
+    // node's ancestor two levels up, ...  A node's 64 grandchildren
+    // (contiguous in the heap numbering) are tested by the 64 lanes at once
+    // against the box of all queries and the largest bound; the survivors are
+    // then tested one by one by every lane against its own bound of the
+    // moment.  A block's leaves go in three classes of distance to the
+    // queries' box, each from the curve's position outwards.
+    // One loop holds every stage, so that the scan and the drain exist once.
     const uint32_t p_first = uniform(__shfl(qp, 0));
     const uint32_t p_last = uniform(__shfl(qp, WAVE - 1));
-    const int64_t l0 = p_first / LEAF;
-    const int64_t l1 = min<int64_t>(p_last / LEAF, l0 + 7);
-    float t1 = A[KCAP - 1];
-    float bound = t1 * PRUNE_REL;
-    int qn = 0;
-    uint32_t nwl = 0;  // recorded leaves (uniform)
-    const uint32_t first_leaf = (uint32_t)t.first_leaf;
-    const int depth = t.depth;
-    const uint32_t lc = uniform(__shfl(qp, WAVE / 2 - 1)) / LEAF;
-    MaskStack ms;
-    int lvl = 0;
-    uint32_t x = 0, off = 0;  // node whose children (level lvl + 1) are pending; its offset in its level
-    int64_t L = l0;           // next own leaf
-    bool walking = false, done = false;
-    if (KCAP == 33 && e == 0) {
-        // k = 32: the own leaves fill the lists through sorting networks, one
-        // leaf at a time (its 16 distances sorted in registers, then merged
-        // into the 33-slot list; the merge's other 16 inputs are +inf),
-        // instead of one queued insertion step per candidate (64 steps of 34
-        // instructions for four own leaves)
-        for (int64_t li = l0; li <= l1; li++) {
-            load_leaf_uniform<P64>(sx, sy, sz, lx, ly, lz, li, cx, cy, cz, clx, cly, clz);
-            float S[32];
+    constexpr uint32_t EXT = NET ? 2 : 0;
+    uint32_t l0 = p_first / LEAF;
+    const uint32_t l1 = min(min(p_last / LEAF, l0 + 7) + EXT, last_leaf);
+    l0 = l0 > EXT ? l0 - EXT : 0;
+    uint32_t L = l0;  // next of these leaves
+    float wlo[3] = {qb.lx, qb.ly, qb.lz}, whi[3] = {qb.hx, qb.hy, qb.hz};
 #pragma unroll
-            for (int i = 0; i < LEAF; i++) {
-                const float d2 = dist2<PER, P64>(t, q, cx[i], cy[i], cz[i], clx[i], cly[i], clz[i]);
-                S[i] = fminf(d2, INFINITY);  // padding (NaN) -> +inf
-            }
-            oddeven_sort<LEAF>(*reinterpret_cast<float(*)[LEAF]>(&S[0]));
-#pragma unroll
-            for (int i = LEAF; i < 32; i++) S[i] = INFINITY;
-            merge_into<32>(*reinterpret_cast<float(*)[33]>(&A[0]), S);
-            if (nwl < a.wlcap && lane == 0) s_wl[w][nwl] = (uint32_t)li;
-            nwl++;
-            n_leaf++;
-        }
-        L = l1 + 1;
-        t1 = A[KCAP - 1];
-        bound = t1 * PRUNE_REL;
+    for (int c = 0; c < 3; c++) {
+        wlo[c] = wave_min_f(wlo[c]);
+        whi[c] = wave_max_f(whi[c]);
     }
-    // batches: scan leaves until some queue is nearly full (the sorted lists
-    // are not touched there), then drain every queue into its list
-    while (true) {
-        while (true) {
-            int64_t li = -1;
-            if (L <= l1) {
-                li = L++;
-            } else if (depth > 0) {
-                if (!walking) {
-                    walking = true;
-                    ms.put(0, expand_mask<PER>(t, qb, 0u, bound));
-                    n_nodes += FANOUT;
+    const uint32_t lc = uniform(__shfl(qp, WAVE / 2 - 1)) / LEAF;
+    uint32_t own = first_leaf + lc;   // ancestor of the middle leaf whose subtree is done
+    int lev = depth;                  // its level
+    uint32_t lbase = 0;               // current block of leaves (heap number),
+    uint64_t lmask = 0;               // those of the current class still to visit,
+    float g = NAN;                    // this lane's leaf's distance (NaN: none, or visited)
+    int cls = 3, lpos = 0;            // next class; the curve's position in the block
+    uint32_t fbase = 0;               // current group of inner nodes,
+    uint64_t fmask = 0;               // those still to visit,
+    int flev = 0, f = 0;              // their level, stacked groups
+    for (int r = 0; r < QROWS; r++) s_buf[w][r][lane] = INF_BITS;
+    bool done = false, fill = true;
+    while (!done) {
+        uint32_t li = 0;
+        if (L <= l1) {
+            li = L++;
+        } else {
+            while (true) {
+                uint32_t y;
+                bool leaf = false;
+                uint32_t eb;  // group to expand, its nodes, their level
+                int ecnt = 64, elev;
+                uint64_t skip = 0;
+                if (lmask) {
+                    const uint32_t b = pick_nearest64(lmask, lpos);
+                    lmask &= ~(1ull << b);
+                    y = lbase + b;
+                    leaf = true;
+                } else if (cls < 3) {
+                    const float part = cls == 0 ? 0.06f : (cls == 1 ? 0.25f : 1.0f);
+                    const bool sel = g <= part * bmax;
+                    lmask = __ballot(sel);
+                    g = sel ? NAN : g;
+                    cls++;
+                    continue;
+                } else if (fmask) {
+                    y = fbase + __builtin_ctzll(fmask);
+                    fmask &= fmask - 1;
+                } else if (f > 0) {
+                    f--;
+                    flev -= 2;
+                    __builtin_amdgcn_wave_barrier();
+                    fbase = uniform(s_stk[w][f][0]);
+                    fmask = (uint64_t)uniform(s_stk[w][f][1]) | (uint64_t)uniform(s_stk[w][f][2]) << 32;
+                    continue;
+                } else if (lev == 0) {
+                    done = true;
+                    break;
+                } else {
+                    y = 0;
                 }
-                while (true) {
-                    const uint32_t m = ms.get(lvl);
-                    if (m == 0u) {
-                        if (lvl == 0) break;
-                        lvl--;
-                        x = (x - 1) >> 3;
-                        off >>= 3;
-                        continue;
-                    }
-                    // the child on (or nearest to) the middle query's path first
-                    const uint32_t anc = lc >> (3 * (depth - 1 - lvl));
-                    const uint32_t base = FANOUT * off;
-                    const uint32_t o = anc < base ? 0u : (anc > base + 7 ? 7u : anc - base);
-                    const uint32_t c = pick_nearest(m, o);
-                    ms.clear(lvl, c);
-                    const uint32_t y = FANOUT * x + 1 + c;
-                    if (lvl + 1 < depth) {
-                        lvl++;
-                        x = y;
-                        off = base + c;
-                        ms.put(lvl, expand_mask<PER>(t, qb, y, bound));
-                        n_nodes += FANOUT;
-                        if (a.stats && lvl + 1 == depth) {
-                            // work counters: leaves this lane itself needs
-                            int pc = 0;
-                            for (int cc = 0; cc < FANOUT; cc++) {
-                                const int64_t lf = (int64_t)(FANOUT * y + 1 + cc - first_leaf);
-                                pc += box_gap2_u<PER>(t, qb, FANOUT * y + 1 + cc) <= bound &&
-                                      !(lf >= l0 && lf <= l1) && lf < t.nleaf;
-                            }
-                            need_lane += pc;
-                            parent_max += wave_max(pc);
-                        }
-                        continue;
-                    }
-                    const int64_t cand = (int64_t)(y - first_leaf);
-                    // own leaves are done; empty leaves pass the box test
-                    // only while some list is not full
-                    if ((cand >= l0 && cand <= l1) || cand >= t.nleaf) continue;
-                    li = cand;
+                if (y != 0 && !__any(box_gap2_u<PER>(t, qb, y) <= bound)) continue;
+                if (leaf) {
+                    li = y - first_leaf;
                     break;
                 }
+                if (y != 0) {
+                    eb = 64u * y + 9u;
+                    elev = flev + 2;
+                    if (elev != depth) {
+                        if (lane == 0) {
+                            s_stk[w][f][0] = fbase;
+                            s_stk[w][f][1] = (uint32_t)fmask;
+                            s_stk[w][f][2] = (uint32_t)(fmask >> 32);
+                        }
+                        __builtin_amdgcn_wave_barrier();
+                        f++;
+                    }
+                } else {
+                    // up: the group that holds own
+                    const uint32_t par = (own - 1) >> 3;
+                    const bool two = lev >= 2;
+                    const uint32_t top = two ? (par - 1) >> 3 : par;
+                    eb = two ? 64u * top + 9u : 8u * top + 1u;
+                    ecnt = two ? 64 : 8;
+                    elev = lev;
+                    skip = 1ull << (own - eb);
+                    own = top;
+                    lev -= two ? 2 : 1;
+                }
+                // the group's boxes against the box of all queries
+                n_nodes += WAVE;
+                const float4 *nb = (const float4 *)(t.nodes + (int64_t)(eb + min(lane, ecnt - 1)) * 8);
+                const float4 u = nb[0], v = nb[1];  // lo xyz, hi x | hi yz
+                const float gx = axis_gap_u<PER>(wlo[0], whi[0], u.x, u.w, t.box);
+                const float gy = axis_gap_u<PER>(wlo[1], whi[1], u.y, v.x, t.box);
+                const float gz = axis_gap_u<PER>(wlo[2], whi[2], u.z, v.y, t.box);
+                const float gap = fmaf(gz, gz, fmaf(gy, gy, gx * gx));
+                if (elev == depth) {
+                    const uint32_t l = eb + lane - first_leaf;
+                    g = lane < ecnt && l < nleaf && !(l >= l0 && l <= l1) ? gap : NAN;
+                    cls = 0;
+                    lbase = eb;
+                    const int o = (int)min<int64_t>(63, max<int64_t>(0, (int64_t)lc - (int64_t)(eb - first_leaf)));
+                    lpos = o;
+                } else {
+                    fbase = eb;
+                    flev = elev;
+                    fmask = __ballot(lane < ecnt && gap <= bmax) & ~skip;
+                }
             }
-            if (li < 0) {
-                done = true;
-                break;
-            }
+        }
+        if (!done) {
+            // every candidate of the leaf is written to its lane's next queue
+            // row, and the row advances when it is under the lane's (k+1)-th
+            // distance; leaves where some lane queued a candidate are recorded
             n_leaf++;
             load_leaf_uniform<P64>(sx, sy, sz, lx, ly, lz, li, cx, cy, cz, clx, cly, clz);
-            const int before = qn;
+            const uint32_t before = qa;
+            const uint64_t all = __builtin_amdgcn_read_exec();
 #pragma unroll
             for (int i = 0; i < LEAF; i++) {
                 const float d2 = dist2<PER, P64>(t, q, cx[i], cy[i], cz[i], clx[i], cly[i], clz[i]);
-                // qn <= QCAP - LEAF when a leaf starts, so the row stays in range
-                s_buf[w][qn][lane] = __float_as_uint(d2);
-                qn += d2 < t1;
+                // at most QCAP - LEAF rows are in use when a leaf starts, so
+                // the row stays in range
+                lds_store(qa, __float_as_uint(d2));
+                advance_lt(qa, d2, t1, all);
             }
-            if (__any(qn > before)) {
-                if (nwl < a.wlcap && lane == 0) s_wl[w][nwl] = (uint32_t)li;
+            if (li == last_leaf) pad = true;
+            if (__any(qa > before)) {
+                if (nwl < a.wlcap) {
+                    if (lane == 0) s_wl[w][nwl] = li;
+                    const uint32_t bit = qa > before ? 1u << (nwl & 31u) : 0u;
+#pragma unroll
+                    for (int i = 0; i < WLWORDS; i++)
+                        if ((nwl >> 5) == (uint32_t)i) mw[i] |= bit;
+                }
                 nwl++;
             }
-            if (__any(qn > QCAP - LEAF)) break;
         }
-        const int nd = wave_max(qn);
-        for (int i = 0; i < nd; i++) {
-            // rows below QCAP are always in range; rows at or past qn are stale
-            const float r = __uint_as_float(s_buf[w][i][lane]);
-            const float v = i < qn ? r : INFINITY;
-            // rows that no lane's list takes any more are skipped
-            if (__any(v < A[KCAP - 1])) {
-                insert_sorted<KCAP>(A, v);
-                n_ins++;
+        // the queues drain when one may not take another leaf, after the fill
+        // and at the end.  Rows past a lane's qn hold +inf, or at row qn a
+        // candidate that was not under the lane's (k+1)-th distance: neither
+        // changes a list.
+        if (done || (fill && L > l1) || __any(qa > rows0 + (QCAP - LEAF) * ROW_STEP)) {
+            fill = fill && L <= l1;
+            const int nd = wave_max((int)(qa - rows0)) / (int)ROW_STEP;
+            if (pad) {
+                for (int i = 0; i < QROWS; i++)
+                    s_buf[w][i][lane] = __float_as_uint(fminf(__uint_as_float(s_buf[w][i][lane]), INFINITY));
+                pad = false;
             }
+            int i = 0;
+            if constexpr (NET) {
+                while (nd - i >= NETMIN && i + LEAF <= QROWS) {
+                    float S[LEAF];
+#pragma unroll
+                    for (int r = 0; r < LEAF; r++) S[r] = __uint_as_float(s_buf[w][i + r][lane]);
+#pragma unroll
+                    for (int r = 0; r < LEAF; r++) s_buf[w][i + r][lane] = INF_BITS;
+                    oddeven_sort<LEAF>(S);
+                    merge_sorted<KCAP, LEAF>(A, S);
+                    i += LEAF;
+                    n_ins += LEAF;
+                }
+            }
+            for (; i < nd; i++) {
+                const float v = __uint_as_float(s_buf[w][i][lane]);
+                s_buf[w][i][lane] = INF_BITS;
+                // rows that no lane's list takes any more are skipped
+                if (__any(v < A[KCAP - 1])) {
+                    insert_sorted<KCAP>(A, v);
+                    n_ins++;
+                }
+            }
+            s_buf[w][min(nd, QROWS - 1)][lane] = INF_BITS;
+            qa = rows0;
+            t1 = A[KCAP - 1];
+            bound = t1 * PRUNE_REL;
+            bmax = wave_max_f(bound);
         }
-        qn = 0;
-        t1 = A[KCAP - 1];
-        bound = t1 * PRUNE_REL;
-        if (done) break;
     }
     __builtin_amdgcn_wave_barrier();
     if (a.stats && lane == 0) {
@@ -446,14 +549,6 @@ __global__ __launch_bounds__(KNN_BLOCK) void k_knn_main(KnnArgs a) {
         atomicAdd(a.stats + STAT_P1_INSERTS, (unsigned long long)n_ins);
         atomicAdd(a.stats + STAT_P2_LEAVES, (unsigned long long)nwl);
         atomicAdd(a.stats + STAT_WAVES, 1ull);
-        atomicAdd(a.stats + STAT_PARENT_MAX, (unsigned long long)parent_max);
-    }
-    if (a.stats) {
-        const uint32_t tot = wave_sum(need_lane), mx = (uint32_t)wave_max((int)need_lane);
-        if (lane == 0) {
-            atomicAdd(a.stats + STAT_LANE_NEED, (unsigned long long)tot);
-            atomicAdd(a.stats + STAT_MAXLANE_NEED, (unsigned long long)mx);
-        }
     }
 
     // (3) epilogue
@@ -494,98 +589,125 @@ __global__ __launch_bounds__(KNN_BLOCK) void k_knn_main(KnnArgs a) {
         // 64 recorded leaves at a time: a step scans one leaf per lane (its
         // particles loaded by the lane itself), so the wave pays for the
         // busiest lane, not for every leaf some lane needs.
+        // Ambiguous lanes take nothing: the resolver writes their rows.
         int cnt = 0;
+        uint32_t ra = rows0;  // staged rows: LDS address of the next
         uint32_t nscan = 0;
         const float tb = tau * PRUNE_REL;
-        auto collect = [&](uint32_t nrec) {
-        for (uint32_t r0 = 0; r0 < nrec; r0 += 64) {
-            const uint32_t nr = min(64u, nrec - r0);
-            uint32_t nlo = 0, nhi = 0;
-            for (uint32_t r = 0; r < nr; r++) {
-                const uint32_t li = uniform(s_wl[w][r0 + r]);
-                if (box_gap2_u<PER>(t, qb, first_leaf + li) <= tb) {
-                    if (r < 32)
-                        nlo |= 1u << r;
-                    else
-                        nhi |= 1u << (r - 32);
-                }
-            }
-            while (__any((nlo | nhi) != 0u)) {
-                const bool act = (nlo | nhi) != 0u;
-                const uint32_t r = nlo ? (uint32_t)__builtin_ctz(nlo) : (nhi ? 32u + (uint32_t)__builtin_ctz(nhi) : 0u);
-                if (nlo)
-                    nlo &= nlo - 1u;
-                else
-                    nhi &= nhi - 1u;
-                const uint32_t li = s_wl[w][r0 + r];
-                nscan++;
-                load_leaf<P64>(t, li, cx, cy, cz, clx, cly, clz);
-#pragma unroll
-                for (int i = 0; i < LEAF; i++) {
-                    const float d2 = dist2<PER, P64>(t, q, cx[i], cy[i], cz[i], clx[i], cly[i], clz[i]);
-                    const bool take = act & (d2 <= tau) & (cnt < a.k);
-                    if (a.nl_d2 && take && live) a.nl_d2[(int64_t)cnt * a.nq + slot] = d2;
-                    if (STAGE) {
-                        // row cnt <= k < LROWS; the row is kept only on a hit
-                        s_buf[w][cnt][lane] = li * LEAF + i;
-                    } else if (take && live) {
-                        a.nl_idx[(int64_t)cnt * a.nq + slot] = li * LEAF + i;
+        const float take = st & ST_AMBIGUOUS ? -1.0f : tau;
+        // a wavefront whose record overflowed (queries spread over a large
+        // region) walks the tree again, pruned by every lane's final radius,
+        // and collects in batches of wlcap leaves
+        const bool over = nwl > a.wlcap;
+        MaskStack ws;
+        int wl = 0;
+        uint32_t wx = 0, nrec = nwl;
+        if (over) ws.put(0, expand_mask<PER>(t, qb, 0u, tb));
+        bool more = true;
+        while (more) {
+            more = over;
+            if (over) {
+                nrec = 0;
+                __builtin_amdgcn_wave_barrier();
+                while (nrec < a.wlcap) {
+                    const uint32_t m = ws.get(wl);
+                    if (m == 0u) {
+                        if (wl == 0) {
+                            more = false;
+                            break;
+                        }
+                        wl--;
+                        wx = (wx - 1) >> 3;
+                        continue;
                     }
-                    cnt += take;
+                    const uint32_t c = (uint32_t)__builtin_ctz(m);
+                    ws.clear(wl, c);
+                    const uint32_t y = FANOUT * wx + 1 + c;
+                    if (wl + 1 < depth) {
+                        wl++;
+                        wx = y;
+                        ws.put(wl, expand_mask<PER>(t, qb, y, tb));
+                        continue;
+                    }
+                    const int64_t cand = (int64_t)(y - first_leaf);
+                    if (cand >= t.nleaf) continue;
+                    if (lane == 0) s_wl[w][nrec] = (uint32_t)cand;
+                    nrec++;
+                }
+                __builtin_amdgcn_wave_barrier();
+            }
+#pragma unroll 1
+            for (uint32_t r0 = 0; r0 < nrec; r0 += 64) {
+                const uint32_t nr = min(64u, nrec - r0);
+                uint32_t nlo = 0, nhi = 0;
+                for (uint32_t r = 0; r < nr; r++) {
+                    const uint32_t li = uniform(s_wl[w][r0 + r]);
+                    if (box_gap2_u<PER>(t, qb, first_leaf + li) <= tb) {
+                        if (r < 32)
+                            nlo |= 1u << r;
+                        else
+                            nhi |= 1u << (r - 32);
+                    }
+                }
+                if (!over) {
+                    // a lane that queued no candidate of a leaf has no member there
+                    nlo &= r0 == 0 ? mw[0] : mw[2];
+                    nhi &= r0 == 0 ? mw[1] : mw[3];
+                }
+                while (__any((nlo | nhi) != 0u)) {
+                    const bool act = (nlo | nhi) != 0u;
+                    const uint32_t r =
+                        nlo ? (uint32_t)__builtin_ctz(nlo) : (nhi ? 32u + (uint32_t)__builtin_ctz(nhi) : 0u);
+                    if (nlo)
+                        nlo &= nlo - 1u;
+                    else
+                        nhi &= nhi - 1u;
+                    const uint32_t li = s_wl[w][r0 + r];
+                    nscan++;
+                    load_leaf<P64>(t, li, cx, cy, cz, clx, cly, clz);
+                    const float lim = act ? take : -1.0f;
+                    if (STAGE) {
+                        const uint64_t all = __builtin_amdgcn_read_exec();
+#pragma unroll
+                        for (int i = 0; i < LEAF; i++) {
+                            const float d2 = dist2<PER, P64>(t, q, cx[i], cy[i], cz[i], clx[i], cly[i], clz[i]);
+                            // at most k members, so at most row k < LROWS; a
+                            // row is kept only on a hit
+                            lds_store(ra, li * LEAF + i);
+                            advance_le(ra, d2, lim, all);
+                        }
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < LEAF; i++) {
+                            const float d2 = dist2<PER, P64>(t, q, cx[i], cy[i], cz[i], clx[i], cly[i], clz[i]);
+                            const bool hit = d2 <= lim;
+                            if (hit && live) {
+                                a.nl_idx[(int64_t)cnt * a.nq + slot] = li * LEAF + i;
+                                if (a.nl_d2) a.nl_d2[(int64_t)cnt * a.nq + slot] = d2;
+                            }
+                            cnt += hit;
+                        }
+                    }
                 }
             }
         }
-        };
-        if (nwl <= a.wlcap) {
-            collect(nwl);
-        } else {
-            // the leaf record overflowed (a wavefront whose queries spread
-            // over a large region): walk the tree again, pruned by every
-            // lane's final radius, and collect in batches of wlcap leaves
-            MaskStack ws;
-            int wl = 0;
-            uint32_t wx = 0, nrec = 0;
-            ws.put(0, expand_mask<PER>(t, qb, 0u, tb));
-            while (true) {
-                const uint32_t m = ws.get(wl);
-                if (m == 0u) {
-                    if (wl == 0) break;
-                    wl--;
-                    wx = (wx - 1) >> 3;
-                    continue;
-                }
-                const uint32_t c = (uint32_t)__builtin_ctz(m);
-                ws.clear(wl, c);
-                const uint32_t y = FANOUT * wx + 1 + c;
-                if (wl + 1 < depth) {
-                    wl++;
-                    wx = y;
-                    ws.put(wl, expand_mask<PER>(t, qb, y, tb));
-                    continue;
-                }
-                const int64_t cand = (int64_t)(y - first_leaf);
-                if (cand >= t.nleaf) continue;
-                if (lane == 0) s_wl[w][nrec] = (uint32_t)cand;
-                if (++nrec == a.wlcap) {
-                    __builtin_amdgcn_wave_barrier();
-                    collect(nrec);
-                    nrec = 0;
-                    __builtin_amdgcn_wave_barrier();
-                }
-            }
-            __builtin_amdgcn_wave_barrier();
-            collect(nrec);
-            if (a.stats && lane == 0) atomicAdd(a.stats + STAT_OVERFLOW_WAVES, 1ull);
-        }
+        if (over && a.stats && lane == 0) atomicAdd(a.stats + STAT_OVERFLOW_WAVES, 1ull);
+        if (STAGE) cnt = (int)((ra - rows0) / ROW_STEP);
         if (a.stats && lane == 0) atomicAdd(a.stats + STAT_P2_NODES, (unsigned long long)nscan);
         if (STAGE && live) {
             for (int j = 0; j < a.k; j++) a.nl_idx[(int64_t)j * a.nq + slot] = j < cnt ? s_buf[w][j][lane] : qp;
+            if (a.nl_d2) {
+                for (int j = 0; j < a.k; j++) {
+                    const uint32_t p = j < cnt ? s_buf[w][j][lane] : qp;
+                    const float d2 = dist2<PER, P64>(t, q, sx[p], sy[p], sz[p], P64 ? lx[p] : 0.f, P64 ? ly[p] : 0.f,
+                                                     P64 ? lz[p] : 0.f);
+                    a.nl_d2[(int64_t)j * a.nq + slot] = j < cnt ? d2 : INFINITY;
+                }
+            }
         }
         if (live && cnt != a.k) {
-            st |= ST_COUNT;
+            st |= ST_COUNT;  // (the resolver takes it back from rows it completes)
             if (!STAGE) pad_list(a, cnt, qp, slot);
-            else if (a.nl_d2)
-                for (int j = cnt; j < a.k; j++) a.nl_d2[(int64_t)j * a.nq + slot] = INFINITY;
         }
         // float64 refinement over the members just collected; ambiguous rows
         // (whose capped collection may hold the wrong ties) are refined by

@@ -9,6 +9,7 @@ namespace mhip {
 constexpr float U32 = 5.9604645e-8f;         // 2^-24
 constexpr float AMBIG_REL = 12.0f * U32;     // fp32 vs fp64 ordering ambiguity of d^2
 constexpr float BAND_REL = 16.0f * U32;      // resolver band half-width
+constexpr float HSML_STEP = 1e-3f;           // a relative float32 Newton step that ends the solve for h
 constexpr float PRUNE_REL = 1.0f + 1e-5f;    // box-test safety factor
 
 struct TreeView {
@@ -125,6 +126,24 @@ MHIP_DEV void load_leaf(const TreeView &t, int64_t leaf, float (&cx)[LEAF], floa
     }
 }
 
+// wavefront minimum / maximum on the DPP network: rows of 16, then the row
+// broadcasts; the result is in lane 63
+template <int CTRL, int ROWS>
+MHIP_DEV float dpp_f(float old, float x) {
+    return __int_as_float(
+        __builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(x), CTRL, ROWS, 0xf, false));
+}
+MHIP_DEV float wave_min_f(float x) {
+    x = fminf(x, dpp_f<0x111, 0xf>(x, x));
+    x = fminf(x, dpp_f<0x112, 0xf>(x, x));
+    x = fminf(x, dpp_f<0x114, 0xf>(x, x));
+    x = fminf(x, dpp_f<0x118, 0xf>(x, x));
+    x = fminf(x, dpp_f<0x142, 0xa>(x, x));
+    x = fminf(x, dpp_f<0x143, 0xc>(x, x));
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), 63));
+}
+MHIP_DEV float wave_max_f(float x) { return -wave_min_f(-x); }
+
 MHIP_DEV int wave_max(int v) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o));
@@ -201,16 +220,14 @@ MHIP_DEV double member_dist(const TreeView &t, const QPos &q, uint32_t p) {
 }
 
 // One float64 step on the smoothing length over the final member list.  The
-// float32 solve before it is at the float32 noise floor (relative error up to
-// ~3e-7, from the float32 distances); the derivative fits are sensitive to h
-// through the weights of the outermost neighbours (d ln W / d ln h =
+// float32 solve before it leaves a relative error of ~1e-6 to 1e-5; the
+// derivative fits are sensitive to h through the weights of the outermost neighbours (d ln W / d ln h =
 // 3q / (1 - q) as q -> 1), so a 2.4e-7 error of h moves second-order
 // derivatives by up to ~6e-5.  The spline as truncated powers, W = 2 a^3 - b^3
 // with a = (1 - q)_+ and b = (1 - 2q)_+, gives W' = -6 (a^2 - b^2) and
 // W'' = 12 a - 24 b without branches, so Halley's step (cubic: third
 // derivatives of W are bounded) costs two more operations per neighbour than
-// Newton's and leaves h at the rounding level of the float64 sums instead of
-// at ~(3e-7)^2.
+// Newton's and leaves h at the rounding level of the float64 sums.
 struct HsmlSums {
     double w = 0.0, d1 = 0.0, d2 = 0.0;  // sums of W / 2, -W' q / 6, W'' q^2 / 12
     MHIP_DEV void add(double q) {

@@ -30,25 +30,8 @@ namespace mhip {
 constexpr int KW_WAVES = 4;  // wavefronts per block
 constexpr int KW_LEAFQ = 68;  // leaf queue: a block of 64 and up to 3 left over
 
-// ---- reductions on the DPP network.  Over the wavefront: rows of 16, then
-// the row broadcasts, result in lane 63; over each row: rotations, result in
-// every lane
-template <int CTRL, int ROWS>
-MHIP_DEV float dpp_f(float old, float x) {
-    return __int_as_float(
-        __builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(x), CTRL, ROWS, 0xf, false));
-}
-MHIP_DEV float wave_min_f(float x) {
-    x = fminf(x, dpp_f<0x111, 0xf>(x, x));
-    x = fminf(x, dpp_f<0x112, 0xf>(x, x));
-    x = fminf(x, dpp_f<0x114, 0xf>(x, x));
-    x = fminf(x, dpp_f<0x118, 0xf>(x, x));
-    x = fminf(x, dpp_f<0x142, 0xa>(x, x));
-    x = fminf(x, dpp_f<0x143, 0xc>(x, x));
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), 63));
-}
-MHIP_DEV float wave_max_f(float x) { return -wave_min_f(-x); }
-
+// ---- reductions over each row of 16 lanes by DPP rotations, result in every
+// lane of the row
 template <int N>
 MHIP_DEV float ror_f(float x) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x120 + N, 0xf, 0xf, true));
@@ -459,7 +442,7 @@ MHIP_DEV void row_hsml(const KnnArgs &a, bool on, int64_t slot, uint32_t qp, flo
         bool done = f == 0.f;
         if (done) {
             hn = h;
-        } else if (fabsf(stp) <= 3e-4f * h) {  // as the main kernel: a step this small ends the solve
+        } else if (fabsf(stp) <= HSML_STEP * h) {  // as the main kernel: a step this small ends the solve
             hn = fminf(fmaxf(hn, lo), hi);
             done = true;
         } else {
