@@ -141,7 +141,7 @@ enum : int {
     STAT_NN_EXACT,        // points re-ranked in float64
     STAT_NEWTON,          // smoothing-length iterations (sum over query lanes)
     STAT_NEWTON_WMAX,     // per wavefront, the largest iteration count of a lane (sum)
-    STAT_OVERFLOW_WAVES,  // wavefronts whose leaf record overflowed (members by a second walk)
+    STAT_OVERFLOW_WAVES,  // wavefronts left to the one-wavefront-per-query kernel
     STAT_COUNT
 };
 static_assert(STAT_COUNT <= 16, "the work-counter buffer holds 16 entries");
@@ -224,6 +224,7 @@ struct mhip_nlist {
     double *h64 = nullptr;        // smoothing length per slot, refined in float64
     int32_t *status = nullptr;    // per slot
     uint32_t *amb = nullptr;      // [0] count, [1..] slots flagged ambiguous (for the resolver)
+    uint32_t *defer = nullptr;    // [0] count, [1..] wavefronts left to the one-wavefront-per-query kernel
     int masked = 0;               // qsorted/qrow valid (query rows are a subset/reordering)
     int has_d2 = 0;               // d2 filled (needed for export)
     const mhip_index *index = nullptr;

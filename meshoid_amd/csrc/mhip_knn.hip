@@ -6,35 +6,36 @@
 //                                                src/meshoid/kernel_density.py:14-57
 //   density = des_ngb*m/(volnorm*h^dim)          src/meshoid/Meshoid.py:169-170
 //
-// Design (one lane per query; 64 consecutive queries in Hilbert order per
-// wavefront; the tree is a complete 8-ary tree in heap numbering, root 0,
-// children of x at 8x+1..8x+8, leaves of 16 particles on the last level):
-//   main    Every lane keeps the k+1 smallest float32 squared distances of
-//           its query sorted in VGPRs; an insertion is one in-place v_med3
-//           per slot.  (1) The leaves holding the wave's own queries are
-//           scanned first.  (2) A wave-uniform depth-first walk without a
-//           stack: expanding a node tests its 8 children (one contiguous
-//           block of boxes, scalar loads) against every lane's bound and
-//           keeps the survivors as an 8-bit mask per level in SGPRs; the
-//           child nearest (in index) to the path of the wave's middle query
-//           goes first.  (3) A leaf's 16 candidates (scalar loads) go to each
-//           lane's LDS queue row qn; qn advances when the candidate is under
-//           the lane's (k+1)-th distance.  Queues drain into the sorted lists
-//           in uniform counted loops.  Leaves where some lane queued a
-//           candidate are recorded.  (4) Epilogue: smoothing length
-//           (safeguarded float32 Newton, then one float64 Newton step over
-//           the final members), density, volume,
-//           and the member set {d2 <= tau}: each lane tests the recorded
-//           leaves against its own final radius and scans only those, one
-//           leaf per lane per step (per-lane loads); the indices are staged
-//           in LDS and written as whole rows.  Queries whose k-th and
-//           (k+1)-th distances are closer than float32 rounding can order
-//           are flagged.  A wavefront whose leaf record overflows walks
-//           the tree again with every lane's final radius and collects the
-//           members in batches of recorded leaves.
-//   resolve for flagged queries only: members in the rounding band around tau
-//           are re-ranked with float64 distances from the caller's positions,
-//           so neighbour sets equal the float64 kNN except for float64 ties.
+// Two kernels: one lane per query (here) and one wavefront per query
+// (mhip_knn_wave.hip); knn_wave_serves there says which takes a set.
+//
+// One lane per query (64 consecutive queries in Hilbert order per wavefront;
+// the tree is a complete 8-ary tree in heap numbering, root 0, children of x
+// at 8x+1..8x+8, leaves of 16 particles on the last level).  Every lane keeps
+// the k+1 smallest float32 squared distances of its query sorted in VGPRs.
+//   (1) The leaves holding the wave's own queries and two on either side are
+//       scanned first; then a walk inside out over groups of 64 nodes.
+//   (2) A leaf's 16 candidates (scalar loads) go to each lane's LDS queue
+//       row, which advances when the candidate is under the lane's (k+1)-th
+//       distance.  Queues drain 16 rows at a time through sorting networks
+//       (few rows: one in-place v_med3 per slot and row).  Leaves where some
+//       lane queued a candidate are recorded, with the lanes that did.
+//   (3) Epilogue: smoothing length (safeguarded float32 Newton, then one
+//       float64 step over the final members), density, volume, and the member
+//       set {d2 <= tau}: each lane scans the recorded leaves that it queued
+//       from and that its final radius reaches, one leaf per lane per step
+//       (per-lane loads); the indices are staged in LDS and written as whole
+//       rows.  Queries whose k-th and (k+1)-th distances float32 cannot order
+//       are re-ranked with float64 distances from the caller's positions, so
+//       neighbour sets equal the float64 kNN except for float64 ties.
+//   Wavefronts whose queries spread over a large region, and in periodic sets
+//   those whose balls reach a face of the box, are left to the other kernel.
+// It is bound by vector instructions: 27.9k a wavefront at 2^24 clustered
+// particles, k = 32 (70 leaves x 143, 20 runs of 16 through the networks x
+// 306, 3.5 smoothing-length iterations x 415, 16 member steps x 157), the
+// vector units 90% busy; 14.5 ms, against 20.0 ms and 43.3k with one insertion
+// step per queued row, 8 child boxes tested by all lanes per node and
+// compensated branches in the smoothing length.
 #include "../../include/meshoid_hip.h"
 #include "mhip_internal.hpp"
 #include "mhip_knn.hpp"
@@ -48,6 +49,9 @@ constexpr int QCAP = 32;                     // per-lane pending-candidate queue
 constexpr int WLCAP = 128;                   // per-wave record of candidate leaves
 constexpr int WLWORDS = WLCAP / 32;
 static_assert(WLWORDS == 4, "the member pass reads the masks as two pairs");
+// leaves after which a wavefront gives up (its queries lie far apart; ~70 are
+// scanned by one whose queries do not)
+constexpr uint32_t LEAFMAX = 224;
 constexpr uint32_t INF_BITS = 0x7f800000u;   // +inf
 constexpr int BAND_CAP = 32;
 constexpr int64_t RESOLVE_WAVES = 8192;      // resolver grid (one wavefront per ambiguous slot)
@@ -109,8 +113,8 @@ MHIP_DEV int64_t slot_of_lane(int64_t *first) {
 // count at that of the traversal.  W as truncated powers (see HsmlSums): 11
 // instructions per neighbour and iteration, against ~30 with the two branches
 // of the spline and compensated sums.  The float64 step that follows is cubic,
-// so h needs to be good to ~1e-5 only: a Newton step below 1e-3 h ends the
-// solve (n(h) is C^2, the error left is of the order of the step squared).
+// so h needs to be good to ~1e-5 only: a step below HSML_STEP h ends the solve
+// (n(h) is C^2, the error left is about twice the step squared).
 // ---------------------------------------------------------------------------
 template <int KCAP>
 MHIP_DEV float hsml_solve(float (&A)[KCAP], int k, int dim, float seed, int32_t &st, int &iters) {
@@ -127,7 +131,7 @@ MHIP_DEV float hsml_solve(float (&A)[KCAP], int k, int dim, float seed, int32_t 
     float hi = (float)hsml_bound_coeff(dim) * rmax;
     iters = 0;
     if (!(hi > 0.f)) return 0.f;  // all k at distance 0: the reference returns 0
-    float h = rmax;
+    float h = fmaxf(HSML_START * rmax, lo);
     if (seed > 0.f) {
         if (seed > lo && seed < hi)
             h = seed;
@@ -151,22 +155,21 @@ MHIP_DEV float hsml_solve(float (&A)[KCAP], int k, int dim, float seed, int32_t 
             // of the sums would hold them all in registers at once
             asm volatile("" : "+v"(s), "+v"(ds));
         }
-        const float f = fmaf(2.0f * norm, s, -kf);
-        if (f == 0.f) break;
-        if (f > 0.f)
+        const float n = 2.0f * norm * s;
+        if (n == kf) break;
+        if (n > kf)
             hi = h;
         else
             lo = h;
-        const float step = f * __builtin_amdgcn_rcpf(norm * 6.0f * ds * ih);
+        float hn = hsml_step(h, n, norm * 6.0f * ds, kf);
         // such a step ends the solve even when it rounds onto the bracket end
         // that h itself has just become (otherwise a converged lane would
         // bisect the whole bracket again and hold its wavefront).  A collapsed
         // bracket also ends it.
-        if (fabsf(step) <= HSML_STEP * h) {
-            h = fminf(fmaxf(h - step, lo), hi);
+        if (fabsf(hn - h) <= HSML_STEP * h) {
+            h = fminf(fmaxf(hn, lo), hi);
             break;
         }
-        float hn = h - step;
         if (!(hn > lo && hn < hi)) hn = 0.5f * (lo + hi);
         if (hi - lo <= 2.5e-7f * h) {
             h = hn;
@@ -274,13 +277,14 @@ struct MaskStack {
 constexpr int LROWS = 33;                          // staged member rows (k <= 32)
 constexpr int QROWS = QCAP > LROWS ? QCAP : LROWS;  // per-lane LDS rows
 
-template <int KCAP, bool PER, bool P64>
+template <int KCAP, bool P64>
 __global__ __launch_bounds__(KNN_BLOCK) void k_knn_main(KnnArgs a) {
     // members are staged in LDS and written as whole rows when they fit
     constexpr bool STAGE = KCAP <= LROWS;
     __shared__ uint32_t s_buf[KNN_WAVES][QROWS][WAVE];
     __shared__ uint32_t s_wl[KNN_WAVES][WLCAP];
     __shared__ uint32_t s_stk[KNN_WAVES][MAX_DEPTH / 2 + 1][3];
+    __shared__ uint32_t s_walk[KNN_WAVES][8];
     const int lane = threadIdx.x & (WAVE - 1), w = threadIdx.x >> 6;
     int64_t wave0;
     const int64_t slot = slot_of_lane(&wave0);
@@ -323,8 +327,8 @@ __global__ __launch_bounds__(KNN_BLOCK) void k_knn_main(KnnArgs a) {
 
     // lists of at least LEAF slots take whole runs of LEAF candidates through
     // sorting networks
-    // (longer lists, which only seeded searches and sets of 2^30 particles
-    // bring here, insert one by one)
+    // (longer lists have no registers left for it: k = 100 gains nothing, k =
+    // 128 spills)
     constexpr bool NET = KCAP >= LEAF && KCAP <= 65;
     // fewer queued rows than this are inserted one by one: a step costs about
     // KCAP + 8 instructions, sorting and merging a run of 16 about 300 (KCAP
@@ -371,92 +375,113 @@ __global__ __launch_bounds__(KNN_BLOCK) void k_knn_main(KnnArgs a) {
         whi[c] = wave_max_f(whi[c]);
     }
     const uint32_t lc = uniform(__shfl(qp, WAVE / 2 - 1)) / LEAF;
-    uint32_t own = first_leaf + lc;   // ancestor of the middle leaf whose subtree is done
-    int lev = depth;                  // its level
     uint32_t lbase = 0;               // current block of leaves (heap number),
     uint64_t lmask = 0;               // those of the current class still to visit,
     float g = NAN;                    // this lane's leaf's distance (NaN: none, or visited)
     int cls = 3, lpos = 0;            // next class; the curve's position in the block
-    uint32_t fbase = 0;               // current group of inner nodes,
-    uint64_t fmask = 0;               // those still to visit,
-    int flev = 0, f = 0;              // their level, stacked groups
+    // the walk above the leaves is needed once per block of leaves: it lives
+    // in LDS, the scalar registers being short (48 hold a leaf's candidates)
+    struct Walk {
+        uint32_t own;        // ancestor of the middle leaf whose subtree is done,
+        int lev;             // its level
+        uint32_t base, mlo, mhi;  // current group of inner nodes, those still to visit,
+        int flev, f;         // their level, stacked groups
+    };
+    if (lane == 0) {
+        s_walk[w][0] = first_leaf + lc;
+        s_walk[w][1] = (uint32_t)depth;
+        s_walk[w][2] = s_walk[w][3] = s_walk[w][4] = s_walk[w][5] = s_walk[w][6] = 0u;
+    }
+    __builtin_amdgcn_wave_barrier();
     for (int r = 0; r < QROWS; r++) s_buf[w][r][lane] = INF_BITS;
-    bool done = false, fill = true;
+    bool done = false, fill = true, defer = false;
     while (!done) {
         uint32_t li = 0;
         if (L <= l1) {
             li = L++;
         } else {
             while (true) {
-                uint32_t y;
-                bool leaf = false;
-                uint32_t eb;  // group to expand, its nodes, their level
-                int ecnt = 64, elev;
-                uint64_t skip = 0;
                 if (lmask) {
                     const uint32_t b = pick_nearest64(lmask, lpos);
                     lmask &= ~(1ull << b);
-                    y = lbase + b;
-                    leaf = true;
-                } else if (cls < 3) {
+                    if (!__any(box_gap2_u<false>(t, qb, lbase + b) <= bound)) continue;
+                    li = lbase + b - first_leaf;
+                    break;
+                }
+                if (cls < 3) {
                     const float part = cls == 0 ? 0.06f : (cls == 1 ? 0.25f : 1.0f);
                     const bool sel = g <= part * bmax;
                     lmask = __ballot(sel);
                     g = sel ? NAN : g;
                     cls++;
                     continue;
-                } else if (fmask) {
-                    y = fbase + __builtin_ctzll(fmask);
-                    fmask &= fmask - 1;
-                } else if (f > 0) {
-                    f--;
-                    flev -= 2;
-                    __builtin_amdgcn_wave_barrier();
-                    fbase = uniform(s_stk[w][f][0]);
-                    fmask = (uint64_t)uniform(s_stk[w][f][1]) | (uint64_t)uniform(s_stk[w][f][2]) << 32;
-                    continue;
-                } else if (lev == 0) {
+                }
+                // the next group of nodes
+                __builtin_amdgcn_wave_barrier();
+                Walk k;
+                k.own = uniform(s_walk[w][0]);
+                k.lev = (int)uniform(s_walk[w][1]);
+                k.base = uniform(s_walk[w][2]);
+                uint64_t fmask = (uint64_t)uniform(s_walk[w][3]) | (uint64_t)uniform(s_walk[w][4]) << 32;
+                k.flev = (int)uniform(s_walk[w][5]);
+                k.f = (int)uniform(s_walk[w][6]);
+                uint32_t y = 0;  // inner node to expand
+                while (true) {
+                    if (fmask) {
+                        y = k.base + __builtin_ctzll(fmask);
+                        fmask &= fmask - 1;
+                        if (__any(box_gap2_u<false>(t, qb, y) <= bound)) break;
+                        y = 0;
+                    } else if (k.f > 0) {
+                        k.f--;
+                        k.flev -= 2;
+                        k.base = uniform(s_stk[w][k.f][0]);
+                        fmask = (uint64_t)uniform(s_stk[w][k.f][1]) | (uint64_t)uniform(s_stk[w][k.f][2]) << 32;
+                    } else {
+                        break;
+                    }
+                }
+                if (y == 0 && k.lev == 0) {
                     done = true;
                     break;
-                } else {
-                    y = 0;
                 }
-                if (y != 0 && !__any(box_gap2_u<PER>(t, qb, y) <= bound)) continue;
-                if (leaf) {
-                    li = y - first_leaf;
+                if (n_leaf > LEAFMAX) {
+                    defer = true;
                     break;
                 }
+                uint32_t eb;  // group to expand, its nodes, their level
+                int ecnt = 64, elev;
+                uint64_t skip = 0;
                 if (y != 0) {
                     eb = 64u * y + 9u;
-                    elev = flev + 2;
+                    elev = k.flev + 2;
                     if (elev != depth) {
                         if (lane == 0) {
-                            s_stk[w][f][0] = fbase;
-                            s_stk[w][f][1] = (uint32_t)fmask;
-                            s_stk[w][f][2] = (uint32_t)(fmask >> 32);
+                            s_stk[w][k.f][0] = k.base;
+                            s_stk[w][k.f][1] = (uint32_t)fmask;
+                            s_stk[w][k.f][2] = (uint32_t)(fmask >> 32);
                         }
-                        __builtin_amdgcn_wave_barrier();
-                        f++;
+                        k.f++;
                     }
                 } else {
                     // up: the group that holds own
-                    const uint32_t par = (own - 1) >> 3;
-                    const bool two = lev >= 2;
+                    const uint32_t par = (k.own - 1) >> 3;
+                    const bool two = k.lev >= 2;
                     const uint32_t top = two ? (par - 1) >> 3 : par;
                     eb = two ? 64u * top + 9u : 8u * top + 1u;
                     ecnt = two ? 64 : 8;
-                    elev = lev;
-                    skip = 1ull << (own - eb);
-                    own = top;
-                    lev -= two ? 2 : 1;
+                    elev = k.lev;
+                    skip = 1ull << (k.own - eb);
+                    k.own = top;
+                    k.lev -= two ? 2 : 1;
                 }
                 // the group's boxes against the box of all queries
                 n_nodes += WAVE;
                 const float4 *nb = (const float4 *)(t.nodes + (int64_t)(eb + min(lane, ecnt - 1)) * 8);
                 const float4 u = nb[0], v = nb[1];  // lo xyz, hi x | hi yz
-                const float gx = axis_gap_u<PER>(wlo[0], whi[0], u.x, u.w, t.box);
-                const float gy = axis_gap_u<PER>(wlo[1], whi[1], u.y, v.x, t.box);
-                const float gz = axis_gap_u<PER>(wlo[2], whi[2], u.z, v.y, t.box);
+                const float gx = axis_gap_u<false>(wlo[0], whi[0], u.x, u.w, t.box);
+                const float gy = axis_gap_u<false>(wlo[1], whi[1], u.y, v.x, t.box);
+                const float gz = axis_gap_u<false>(wlo[2], whi[2], u.z, v.y, t.box);
                 const float gap = fmaf(gz, gz, fmaf(gy, gy, gx * gx));
                 if (elev == depth) {
                     const uint32_t l = eb + lane - first_leaf;
@@ -466,11 +491,22 @@ __global__ __launch_bounds__(KNN_BLOCK) void k_knn_main(KnnArgs a) {
                     const int o = (int)min<int64_t>(63, max<int64_t>(0, (int64_t)lc - (int64_t)(eb - first_leaf)));
                     lpos = o;
                 } else {
-                    fbase = eb;
-                    flev = elev;
+                    k.base = eb;
+                    k.flev = elev;
                     fmask = __ballot(lane < ecnt && gap <= bmax) & ~skip;
                 }
+                if (lane == 0) {
+                    s_walk[w][0] = k.own;
+                    s_walk[w][1] = (uint32_t)k.lev;
+                    s_walk[w][2] = k.base;
+                    s_walk[w][3] = (uint32_t)fmask;
+                    s_walk[w][4] = (uint32_t)(fmask >> 32);
+                    s_walk[w][5] = (uint32_t)k.flev;
+                    s_walk[w][6] = (uint32_t)k.f;
+                }
+                __builtin_amdgcn_wave_barrier();
             }
+            if (defer) break;
         }
         if (!done) {
             // every candidate of the leaf is written to its lane's next queue
@@ -482,7 +518,7 @@ __global__ __launch_bounds__(KNN_BLOCK) void k_knn_main(KnnArgs a) {
             const uint64_t all = __builtin_amdgcn_read_exec();
 #pragma unroll
             for (int i = 0; i < LEAF; i++) {
-                const float d2 = dist2<PER, P64>(t, q, cx[i], cy[i], cz[i], clx[i], cly[i], clz[i]);
+                const float d2 = dist2<false, P64>(t, q, cx[i], cy[i], cz[i], clx[i], cly[i], clz[i]);
                 // at most QCAP - LEAF rows are in use when a leaf starts, so
                 // the row stays in range
                 lds_store(qa, __float_as_uint(d2));
@@ -490,13 +526,15 @@ __global__ __launch_bounds__(KNN_BLOCK) void k_knn_main(KnnArgs a) {
             }
             if (li == last_leaf) pad = true;
             if (__any(qa > before)) {
-                if (nwl < a.wlcap) {
-                    if (lane == 0) s_wl[w][nwl] = li;
-                    const uint32_t bit = qa > before ? 1u << (nwl & 31u) : 0u;
-#pragma unroll
-                    for (int i = 0; i < WLWORDS; i++)
-                        if ((nwl >> 5) == (uint32_t)i) mw[i] |= bit;
+                if (nwl == a.wlcap) {
+                    defer = true;
+                    break;
                 }
+                if (lane == 0) s_wl[w][nwl] = li;
+                const uint32_t bit = qa > before ? 1u << (nwl & 31u) : 0u;
+#pragma unroll
+                for (int i = 0; i < WLWORDS; i++)
+                    if ((nwl >> 5) == (uint32_t)i) mw[i] |= bit;
                 nwl++;
             }
         }
@@ -505,7 +543,7 @@ __global__ __launch_bounds__(KNN_BLOCK) void k_knn_main(KnnArgs a) {
         // candidate that was not under the lane's (k+1)-th distance: neither
         // changes a list.
         if (done || (fill && L > l1) || __any(qa > rows0 + (QCAP - LEAF) * ROW_STEP)) {
-            fill = fill && L <= l1;
+            const bool filled = fill && L > l1;
             const int nd = wave_max((int)(qa - rows0)) / (int)ROW_STEP;
             if (pad) {
                 for (int i = 0; i < QROWS; i++)
@@ -540,7 +578,39 @@ __global__ __launch_bounds__(KNN_BLOCK) void k_knn_main(KnnArgs a) {
             t1 = A[KCAP - 1];
             bound = t1 * PRUNE_REL;
             bmax = wave_max_f(bound);
+            if (filled) {
+                fill = false;
+                if (t.box > 0.f) {
+                    // Periodic: no query's ball may reach a face of the box
+                    // (no neighbour is then an image, and plain offsets and
+                    // box gaps serve)
+                    const float r = __builtin_amdgcn_sqrtf(t1) * 1.001f + t.slack;
+                    const float qx[3] = {q.x, q.y, q.z};
+                    bool inner = r < t.half;
+#pragma unroll
+                    for (int c = 0; c < 3; c++)
+                        inner = inner && (c >= a.dim || (qx[c] - r > 0.f && qx[c] + r < t.box));
+                    if (__any(!inner)) {
+                        defer = true;
+                        break;
+                    }
+                }
+            }
         }
+    }
+    if (defer) {
+        // queries spread over a large region (more leaves than the record
+        // holds, or than a wavefront should scan), or near a periodic face:
+        // left to the one-wavefront-per-query kernel
+        if (lane == 0) {
+            a.defer[1 + atomicAdd(a.defer, 1u)] = (uint32_t)(wave0 / WAVE);
+            if (a.stats) {
+                atomicAdd(a.stats + STAT_OVERFLOW_WAVES, 1ull);
+                atomicAdd(a.stats + STAT_WAVES, 1ull);
+            }
+        }
+        if (live) a.st_slot[slot] = 0;
+        return;
     }
     __builtin_amdgcn_wave_barrier();
     if (a.stats && lane == 0) {
@@ -595,103 +665,58 @@ __global__ __launch_bounds__(KNN_BLOCK) void k_knn_main(KnnArgs a) {
         uint32_t nscan = 0;
         const float tb = tau * PRUNE_REL;
         const float take = st & ST_AMBIGUOUS ? -1.0f : tau;
-        // a wavefront whose record overflowed (queries spread over a large
-        // region) walks the tree again, pruned by every lane's final radius,
-        // and collects in batches of wlcap leaves
-        const bool over = nwl > a.wlcap;
-        MaskStack ws;
-        int wl = 0;
-        uint32_t wx = 0, nrec = nwl;
-        if (over) ws.put(0, expand_mask<PER>(t, qb, 0u, tb));
-        bool more = true;
-        while (more) {
-            more = over;
-            if (over) {
-                nrec = 0;
-                __builtin_amdgcn_wave_barrier();
-                while (nrec < a.wlcap) {
-                    const uint32_t m = ws.get(wl);
-                    if (m == 0u) {
-                        if (wl == 0) {
-                            more = false;
-                            break;
-                        }
-                        wl--;
-                        wx = (wx - 1) >> 3;
-                        continue;
-                    }
-                    const uint32_t c = (uint32_t)__builtin_ctz(m);
-                    ws.clear(wl, c);
-                    const uint32_t y = FANOUT * wx + 1 + c;
-                    if (wl + 1 < depth) {
-                        wl++;
-                        wx = y;
-                        ws.put(wl, expand_mask<PER>(t, qb, y, tb));
-                        continue;
-                    }
-                    const int64_t cand = (int64_t)(y - first_leaf);
-                    if (cand >= t.nleaf) continue;
-                    if (lane == 0) s_wl[w][nrec] = (uint32_t)cand;
-                    nrec++;
-                }
-                __builtin_amdgcn_wave_barrier();
-            }
 #pragma unroll 1
-            for (uint32_t r0 = 0; r0 < nrec; r0 += 64) {
-                const uint32_t nr = min(64u, nrec - r0);
-                uint32_t nlo = 0, nhi = 0;
-                for (uint32_t r = 0; r < nr; r++) {
-                    const uint32_t li = uniform(s_wl[w][r0 + r]);
-                    if (box_gap2_u<PER>(t, qb, first_leaf + li) <= tb) {
-                        if (r < 32)
-                            nlo |= 1u << r;
-                        else
-                            nhi |= 1u << (r - 32);
-                    }
-                }
-                if (!over) {
-                    // a lane that queued no candidate of a leaf has no member there
-                    nlo &= r0 == 0 ? mw[0] : mw[2];
-                    nhi &= r0 == 0 ? mw[1] : mw[3];
-                }
-                while (__any((nlo | nhi) != 0u)) {
-                    const bool act = (nlo | nhi) != 0u;
-                    const uint32_t r =
-                        nlo ? (uint32_t)__builtin_ctz(nlo) : (nhi ? 32u + (uint32_t)__builtin_ctz(nhi) : 0u);
-                    if (nlo)
-                        nlo &= nlo - 1u;
+        for (uint32_t r0 = 0; r0 < nwl; r0 += 64) {
+            const uint32_t nr = min(64u, nwl - r0);
+            uint32_t nlo = 0, nhi = 0;
+            for (uint32_t r = 0; r < nr; r++) {
+                const uint32_t li = uniform(s_wl[w][r0 + r]);
+                if (box_gap2_u<false>(t, qb, first_leaf + li) <= tb) {
+                    if (r < 32)
+                        nlo |= 1u << r;
                     else
-                        nhi &= nhi - 1u;
-                    const uint32_t li = s_wl[w][r0 + r];
-                    nscan++;
-                    load_leaf<P64>(t, li, cx, cy, cz, clx, cly, clz);
-                    const float lim = act ? take : -1.0f;
-                    if (STAGE) {
-                        const uint64_t all = __builtin_amdgcn_read_exec();
+                        nhi |= 1u << (r - 32);
+                }
+            }
+            // a lane that queued no candidate of a leaf has no member there
+            nlo &= r0 == 0 ? mw[0] : mw[2];
+            nhi &= r0 == 0 ? mw[1] : mw[3];
+            while (__any((nlo | nhi) != 0u)) {
+                const bool act = (nlo | nhi) != 0u;
+                const uint32_t r =
+                    nlo ? (uint32_t)__builtin_ctz(nlo) : (nhi ? 32u + (uint32_t)__builtin_ctz(nhi) : 0u);
+                if (nlo)
+                    nlo &= nlo - 1u;
+                else
+                    nhi &= nhi - 1u;
+                const uint32_t li = s_wl[w][r0 + r];
+                nscan++;
+                load_leaf<P64>(t, li, cx, cy, cz, clx, cly, clz);
+                const float lim = act ? take : -1.0f;
+                if (STAGE) {
+                    const uint64_t all = __builtin_amdgcn_read_exec();
 #pragma unroll
-                        for (int i = 0; i < LEAF; i++) {
-                            const float d2 = dist2<PER, P64>(t, q, cx[i], cy[i], cz[i], clx[i], cly[i], clz[i]);
-                            // at most k members, so at most row k < LROWS; a
-                            // row is kept only on a hit
-                            lds_store(ra, li * LEAF + i);
-                            advance_le(ra, d2, lim, all);
-                        }
-                    } else {
+                    for (int i = 0; i < LEAF; i++) {
+                        const float d2 = dist2<false, P64>(t, q, cx[i], cy[i], cz[i], clx[i], cly[i], clz[i]);
+                        // at most k members, so at most row k < LROWS; a
+                        // row is kept only on a hit
+                        lds_store(ra, li * LEAF + i);
+                        advance_le(ra, d2, lim, all);
+                    }
+                } else {
 #pragma unroll
-                        for (int i = 0; i < LEAF; i++) {
-                            const float d2 = dist2<PER, P64>(t, q, cx[i], cy[i], cz[i], clx[i], cly[i], clz[i]);
-                            const bool hit = d2 <= lim;
-                            if (hit && live) {
-                                a.nl_idx[(int64_t)cnt * a.nq + slot] = li * LEAF + i;
-                                if (a.nl_d2) a.nl_d2[(int64_t)cnt * a.nq + slot] = d2;
-                            }
-                            cnt += hit;
+                    for (int i = 0; i < LEAF; i++) {
+                        const float d2 = dist2<false, P64>(t, q, cx[i], cy[i], cz[i], clx[i], cly[i], clz[i]);
+                        const bool hit = d2 <= lim;
+                        if (hit && live) {
+                            a.nl_idx[(int64_t)cnt * a.nq + slot] = li * LEAF + i;
+                            if (a.nl_d2) a.nl_d2[(int64_t)cnt * a.nq + slot] = d2;
                         }
+                        cnt += hit;
                     }
                 }
             }
         }
-        if (over && a.stats && lane == 0) atomicAdd(a.stats + STAT_OVERFLOW_WAVES, 1ull);
         if (STAGE) cnt = (int)((ra - rows0) / ROW_STEP);
         if (a.stats && lane == 0) atomicAdd(a.stats + STAT_P2_NODES, (unsigned long long)nscan);
         if (STAGE && live) {
@@ -699,7 +724,7 @@ __global__ __launch_bounds__(KNN_BLOCK) void k_knn_main(KnnArgs a) {
             if (a.nl_d2) {
                 for (int j = 0; j < a.k; j++) {
                     const uint32_t p = j < cnt ? s_buf[w][j][lane] : qp;
-                    const float d2 = dist2<PER, P64>(t, q, sx[p], sy[p], sz[p], P64 ? lx[p] : 0.f, P64 ? ly[p] : 0.f,
+                    const float d2 = dist2<false, P64>(t, q, sx[p], sy[p], sz[p], P64 ? lx[p] : 0.f, P64 ? ly[p] : 0.f,
                                                      P64 ? lz[p] : 0.f);
                     a.nl_d2[(int64_t)j * a.nq + slot] = j < cnt ? d2 : INFINITY;
                 }
@@ -714,9 +739,9 @@ __global__ __launch_bounds__(KNN_BLOCK) void k_knn_main(KnnArgs a) {
         // the resolver once it has rebuilt them
         if (live && cnt == a.k && h > 0.f && !(st & (ST_HSML_NOCONV | ST_AMBIGUOUS))) {
             if (STAGE)
-                h64 = refine_h64<PER, P64>(a, q, h64, [&](int j) { return s_buf[w][j][lane]; });
+                h64 = refine_h64<false, P64>(a, q, h64, [&](int j) { return s_buf[w][j][lane]; });
             else
-                h64 = refine_h64<PER, P64>(a, q, h64, [&](int j) { return a.nl_idx[(int64_t)j * a.nq + slot]; });
+                h64 = refine_h64<false, P64>(a, q, h64, [&](int j) { return a.nl_idx[(int64_t)j * a.nq + slot]; });
         }
     }
     if (live) {
@@ -902,10 +927,10 @@ MHIP_DEV void resolve_slot(const KnnArgs &a, const PT *__restrict__ pos_in, int6
     a.st_slot[slot] = st;
 }
 
-// empties the list of ambiguous slots (a kernel, so graph capture records no
-// memset node)
-__global__ void k_amb_reset(uint32_t *__restrict__ amb) {
-    if (threadIdx.x == 0) amb[0] = 0u;
+// empties the lists of ambiguous slots and of deferred wavefronts (a kernel,
+// so graph capture records no memset node)
+__global__ void k_lists_reset(uint32_t *__restrict__ amb, uint32_t *__restrict__ defer) {
+    if (threadIdx.x == 0) amb[0] = defer[0] = 0u;
 }
 
 // the list of ambiguous slots, one wavefront per slot (a grid-stride loop
@@ -997,18 +1022,23 @@ static int nl_grow(mhip_ctx *ctx, void **p, size_t bytes) {
 }
 
 template <int KCAP>
-static void launch_main(const KnnArgs &a, bool per, bool p64, dim3 g, hipStream_t s) {
-    if (per) {
-        if (p64)
-            hipLaunchKernelGGL((k_knn_main<KCAP, true, true>), g, dim3(KNN_BLOCK), 0, s, a);
-        else
-            hipLaunchKernelGGL((k_knn_main<KCAP, true, false>), g, dim3(KNN_BLOCK), 0, s, a);
-    } else {
-        if (p64)
-            hipLaunchKernelGGL((k_knn_main<KCAP, false, true>), g, dim3(KNN_BLOCK), 0, s, a);
-        else
-            hipLaunchKernelGGL((k_knn_main<KCAP, false, false>), g, dim3(KNN_BLOCK), 0, s, a);
-    }
+static void launch_main(const KnnArgs &a, bool p64, dim3 g, hipStream_t s) {
+    if (p64)
+        hipLaunchKernelGGL((k_knn_main<KCAP, true>), g, dim3(KNN_BLOCK), 0, s, a);
+    else
+        hipLaunchKernelGGL((k_knn_main<KCAP, false>), g, dim3(KNN_BLOCK), 0, s, a);
+}
+
+static void launch_main_k(const KnnArgs &a, bool p64, dim3 g, hipStream_t s) {
+    const int need = a.k + 1;
+    if (need <= 5) launch_main<5>(a, p64, g, s);
+    else if (need <= 9) launch_main<9>(a, p64, g, s);
+    else if (need <= 17) launch_main<17>(a, p64, g, s);
+    else if (need <= 21) launch_main<21>(a, p64, g, s);
+    else if (need <= 33) launch_main<33>(a, p64, g, s);
+    else if (need <= 65) launch_main<65>(a, p64, g, s);
+    else if (need <= 101) launch_main<101>(a, p64, g, s);
+    else launch_main<129>(a, p64, g, s);
 }
 
 static int nl_reserve(mhip_ctx *ctx, mhip_nlist *nl, int64_t nq, int k) {
@@ -1020,6 +1050,7 @@ static int nl_reserve(mhip_ctx *ctx, mhip_nlist *nl, int64_t nq, int k) {
             if ((rc = nl_grow(ctx, p, nq * 4))) return rc;
         if ((rc = nl_grow(ctx, (void **)&nl->rowrec, nq * 16))) return rc;
         if ((rc = nl_grow(ctx, (void **)&nl->amb, (nq + 1) * 4))) return rc;
+        if ((rc = nl_grow(ctx, (void **)&nl->defer, (nq / WAVE + 2) * 4))) return rc;
         if ((rc = nl_grow(ctx, (void **)&nl->h64, nq * 8))) return rc;
         if ((rc = nl_grow(ctx, (void **)&nl->idx, (size_t)nq * k * 4))) return rc;
         if ((rc = nl_grow(ctx, (void **)&nl->d2, (size_t)nq * k * 4))) return rc;
@@ -1113,55 +1144,27 @@ int knn_run(mhip_ctx *ctx, const mhip_index *ix, const int64_t *qidx, int64_t nq
     a.nl_d2 = nl->has_d2 ? nl->d2 : nullptr;
     a.stats = ctx->prof >= 2 ? ctx->stats : nullptr;
     a.amb = nl->amb;
+    a.defer = nl->defer;
     a.wlcap = (flags & MHIP_KNN_SMALL_RECORD) ? 8u : (uint32_t)WLCAP;
     const bool p64 = ix->pos_f64 != 0;
     const dim3 g((unsigned)((nq + KNN_BLOCK - 1) / KNN_BLOCK));
     hipStream_t s = ctx->stream;
-    hipLaunchKernelGGL(k_amb_reset, dim3(1), dim3(64), 0, s, nl->amb);
-    const int need = k + 1;
+    hipLaunchKernelGGL(k_lists_reset, dim3(1), dim3(64), 0, s, nl->amb, nl->defer);
     ProfRegion pr1(ctx, "knn_main");
-    // seeds and the leaf-record test hook belong to the main kernel
-    const bool wave = !seed_h && !seed_r && !(flags & MHIP_KNN_SMALL_RECORD) && knn_wave_serves(ix->n, nq, k);
+    // seeds and the test hooks belong to the main kernel
+    const bool wave = !seed_h && !seed_r && !(flags & (MHIP_KNN_SMALL_RECORD | MHIP_KNN_LANE)) &&
+                      knn_wave_serves(ix->n, nq, k, ix->dim, per);
     if (wave) {
-        if ((rc = knn_wave_launch(ctx, a, per, p64))) return rc;
+        if ((rc = knn_wave_launch(ctx, a, per, p64, false))) return rc;
     } else {
-        if (need <= 5)
-            launch_main<5>(a, per, p64, g, s);
-        else if (need <= 9)
-            launch_main<9>(a, per, p64, g, s);
-        else if (need <= 17)
-            launch_main<17>(a, per, p64, g, s);
-        else if (need <= 21)
-            launch_main<21>(a, per, p64, g, s);
-        else if (need <= 33)
-            launch_main<33>(a, per, p64, g, s);
-        else if (need <= 65)
-            launch_main<65>(a, per, p64, g, s);
-        else if (need <= 101)
-            launch_main<101>(a, per, p64, g, s);
-        else
-            launch_main<129>(a, per, p64, g, s);
-    }
-    if (seed_r) {
-        // second launch: waves with a radius-seed miss are recomputed plainly
-        KnnArgs r = a;
-        r.redo = 1;
-        if (need <= 5)
-            launch_main<5>(r, per, p64, g, s);
-        else if (need <= 9)
-            launch_main<9>(r, per, p64, g, s);
-        else if (need <= 17)
-            launch_main<17>(r, per, p64, g, s);
-        else if (need <= 21)
-            launch_main<21>(r, per, p64, g, s);
-        else if (need <= 33)
-            launch_main<33>(r, per, p64, g, s);
-        else if (need <= 65)
-            launch_main<65>(r, per, p64, g, s);
-        else if (need <= 101)
-            launch_main<101>(r, per, p64, g, s);
-        else
-            launch_main<129>(r, per, p64, g, s);
+        launch_main_k(a, p64, g, s);
+        if (seed_r) {
+            // second launch: waves with a radius-seed miss are recomputed plainly
+            KnnArgs r = a;
+            r.redo = 1;
+            launch_main_k(r, p64, g, s);
+        }
+        if ((rc = knn_wave_launch(ctx, a, per, p64, true))) return rc;
     }
     pr1.end();
     ProfRegion pr3(ctx, "knn_resolve");

@@ -9,7 +9,8 @@ namespace mhip {
 constexpr float U32 = 5.9604645e-8f;         // 2^-24
 constexpr float AMBIG_REL = 12.0f * U32;     // fp32 vs fp64 ordering ambiguity of d^2
 constexpr float BAND_REL = 16.0f * U32;      // resolver band half-width
-constexpr float HSML_STEP = 1e-3f;           // a relative float32 Newton step that ends the solve for h
+constexpr float HSML_STEP = 2e-3f;           // a relative float32 step that ends the solve for h
+constexpr float HSML_START = 0.92f;          // first guess of h / r_k (its median is 0.91)
 constexpr float PRUNE_REL = 1.0f + 1e-5f;    // box-test safety factor
 
 struct TreeView {
@@ -176,6 +177,7 @@ struct KnnArgs {
     float *nl_d2;
     unsigned long long *stats;  // work counters, may be null
     uint32_t *amb;              // [0] count, [1..] ambiguous slots
+    uint32_t *defer;            // [0] count, [1..] wavefronts (64 slots) left to the one-wavefront-per-query kernel
     uint32_t wlcap;             // leaf-record capacity used (<= WLCAP; smaller only as a test hook)
 };
 
@@ -260,6 +262,13 @@ MHIP_DEV double refine_h64(const KnnArgs &a, const QPos &q, double hd, F member)
     return hsml_step64(s, hd, a.k, a.dim);
 }
 
+// Newton's step in the logarithms, ln n against ln h (n(h) is close to a power
+// law between neighbours): p = h n'(h)
+MHIP_DEV float hsml_step(float h, float n, float p, float kf) {
+    return h * __builtin_amdgcn_exp2f(__builtin_amdgcn_logf(kf * __builtin_amdgcn_rcpf(n)) * n *
+                                      __builtin_amdgcn_rcpf(p));
+}
+
 // smoothing length of one query slot (float32 copy and float64); the
 // row-order h, density and volume are formed from it by k_rows_out
 MHIP_DEV void write_h(const KnnArgs &a, int64_t slot, double h) {
@@ -267,8 +276,10 @@ MHIP_DEV void write_h(const KnnArgs &a, int64_t slot, double h) {
     a.h64_slot[slot] = h;
 }
 
-// one wavefront per query (mhip_knn_wave.hip)
-bool knn_wave_serves(int64_t n, int64_t nq, int k);
-int knn_wave_launch(mhip_ctx *ctx, const KnnArgs &a, bool per, bool p64);
+// one wavefront per query (mhip_knn_wave.hip): whether it is the faster kernel
+// for the whole set; its launch over every slot, or (deferred) over the
+// wavefronts in a.defer
+bool knn_wave_serves(int64_t n, int64_t nq, int k, int dim, bool per);
+int knn_wave_launch(mhip_ctx *ctx, const KnnArgs &a, bool per, bool p64, bool deferred);
 
 }  // namespace mhip

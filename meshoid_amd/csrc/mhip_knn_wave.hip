@@ -21,6 +21,7 @@
 //           per lane and wave-wide sums.
 // The same float32 distances, box tests and ambiguity rule as the main
 // kernel, so the member sets are the same; ambiguous rows go to the resolver.
+#include <algorithm>
 #include <type_traits>
 
 #include "mhip_knn.hpp"
@@ -28,6 +29,7 @@
 namespace mhip {
 
 constexpr int KW_WAVES = 4;  // wavefronts per block
+constexpr int64_t KW_LIST_OPEN = 2048, KW_LIST_PER = 65536;  // grids over deferred wavefronts
 constexpr int KW_LEAFQ = 68;  // leaf queue: a block of 64 and up to 3 left over
 
 // ---- reductions over each row of 16 lanes by DPP rotations, result in every
@@ -70,9 +72,12 @@ MHIP_DEV int lane_rank(uint64_t m) {  // set bits of m below this lane
 // keeps the compiler from moving them across)
 MHIP_DEV void lds_order() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
 
-// element p of an array of fewer than 2^30 floats, through a 32-bit byte
-// offset from a scalar base
-MHIP_DEV float ld32(const float *b, uint32_t p) { return *(const float *)((const char *)b + (size_t)(uint32_t)(p << 2)); }
+// element p of a float array: with fewer than 2^30 of them (OFF = uint32_t)
+// through a 32-bit byte offset from a scalar base
+template <typename OFF>
+MHIP_DEV float ld32(const float *b, uint32_t p) {
+    return *(const float *)((const char *)b + (size_t)((OFF)p << 2));
+}
 
 template <int NR>
 MHIP_DEV int count_le(const float (&v)[NR], float t, int nr) {
@@ -122,7 +127,7 @@ MHIP_DEV float threshold(const float (&v)[NR], float top, int n, int nr, int lo_
 // of squared distance and sorted index); s_lq: its leaf queue; s_stk: its walk stack.  Members go to
 // s_out[j * ncol + col], j < k; returns the row's status bits, tau = the k-th
 // squared distance.
-template <int NR, bool PER, bool P64>
+template <int NR, bool PER, bool P64, typename OFF>
 MHIP_DEV int32_t wave_search(const KnnArgs &a, int64_t slot, uint32_t qp, uint2 *s_c, uint32_t *s_lq,
                              uint32_t (*s_stk)[4], uint32_t *s_out, int col, int ncol, float &tau_out) {
     constexpr int CAP = 64 * NR;
@@ -211,8 +216,9 @@ MHIP_DEV int32_t wave_search(const KnnArgs &a, int64_t slot, uint32_t qp, uint2 
     };
     auto dist = [&](uint32_t p, auto per) {
         constexpr bool WRAP = decltype(per)::value;
-        return dist2<WRAP, P64>(t, q, ld32(t.sx, p), ld32(t.sy, p), ld32(t.sz, p), P64 ? ld32(t.lx, p) : 0.f,
-                                P64 ? ld32(t.ly, p) : 0.f, P64 ? ld32(t.lz, p) : 0.f);
+        return dist2<WRAP, P64>(t, q, ld32<OFF>(t.sx, p), ld32<OFF>(t.sy, p), ld32<OFF>(t.sz, p),
+                                P64 ? ld32<OFF>(t.lx, p) : 0.f, P64 ? ld32<OFF>(t.ly, p) : 0.f,
+                                P64 ? ld32<OFF>(t.lz, p) : 0.f);
     };
 
     // fill: the leaves around the query's own (more than k + 1 candidates)
@@ -330,9 +336,10 @@ MHIP_DEV int32_t wave_search(const KnnArgs &a, int64_t slot, uint32_t qp, uint2 
         // a ball that does not reach the box's faces meets no image: offsets
         // beyond half the box are then beyond the bound either way
         const float r = __builtin_sqrtf(bound) * 1.001f + t.slack;
-        const float lo = fminf(q.x, fminf(q.y, a.dim == 3 ? q.z : q.y));
-        const float hi = fmaxf(q.x, fmaxf(q.y, q.z));
-        const bool inner = a.dim > 1 && lo - r > 0.f && hi + r < t.box && r < t.half;
+        const float qx[3] = {q.x, q.y, q.z};
+        bool inner = r < t.half;
+#pragma unroll
+        for (int c = 0; c < 3; c++) inner = inner && (c >= a.dim || (qx[c] - r > 0.f && qx[c] + r < t.box));
         if (__any(!inner)) walk(std::true_type());
         else walk(std::false_type());
     } else {
@@ -387,7 +394,8 @@ MHIP_DEV int32_t wave_search(const KnnArgs &a, int64_t slot, uint32_t qp, uint2 
 // lanes, MPL members per lane (16 MPL >= k): float64 distances of the members,
 // safeguarded float32 Newton, one float64 step (hsml_step64).  The same
 // control flow as the main kernel's solve.
-template <int MPL, bool PER, bool P64>
+// SEED: a Newton seed per row (a.seed_h) may be given.
+template <int MPL, bool PER, bool P64, bool SEED>
 MHIP_DEV void row_hsml(const KnnArgs &a, bool on, int64_t slot, uint32_t qp, float tau, int32_t st,
                        const uint32_t *s_out, int col, int ncol) {
     const int rl = threadIdx.x & 15;
@@ -419,7 +427,12 @@ MHIP_DEV void row_hsml(const KnnArgs &a, bool on, int64_t slot, uint32_t qp, flo
     const float norm = (float)hsml_norm(a.dim), kf = (float)k;
     float hi = (float)hsml_bound_coeff(a.dim) * rmax;
     bool run = on && !(st & ST_COUNT) && hi > 0.f;
-    float h = run ? rmax : 0.f;
+    float h = run ? fmaxf(HSML_START * rmax, lo) : 0.f;
+    if (SEED && run && a.seed_h) {
+        const float seed = a.seed_h[a.qrow ? a.qrow[slot] : a.perm[slot]];
+        if (seed > lo && seed < hi) h = seed;
+        else if (seed > 0.f) st |= ST_SEED_MISS;
+    }
     for (int it = 0; it < 40 && __any(run); it++) {
         const float ih = __builtin_amdgcn_rcpf(h);
         float s = 0.f, ds = 0.f;
@@ -434,15 +447,14 @@ MHIP_DEV void row_hsml(const KnnArgs &a, bool on, int64_t slot, uint32_t qp, flo
         }
         s = row_sum(s);
         ds = row_sum(ds);
-        const float f = norm * s - kf;
-        if (f > 0.f) hi = h;
+        const float n = norm * s;
+        if (n > kf) hi = h;
         else lo = h;
-        const float stp = f * __builtin_amdgcn_rcpf(norm * 6.0f * ds * ih);
-        float hn = h - stp;
-        bool done = f == 0.f;
+        float hn = hsml_step(h, n, norm * 6.0f * ds, kf);
+        bool done = n == kf;
         if (done) {
             hn = h;
-        } else if (fabsf(stp) <= HSML_STEP * h) {  // as the main kernel: a step this small ends the solve
+        } else if (fabsf(hn - h) <= HSML_STEP * h) {  // as the main kernel: a step this small ends the solve
             hn = fminf(fmaxf(hn, lo), hi);
             done = true;
         } else {
@@ -471,77 +483,127 @@ MHIP_DEV void row_hsml(const KnnArgs &a, bool on, int64_t slot, uint32_t qp, flo
 }
 
 // each wavefront serves PW consecutive slots; the block's rows of the member
-// list (4 PW slots wide) are staged in LDS and written together
-template <int NR, bool PER, bool P64, int PW>
-__global__ __launch_bounds__(64 * KW_WAVES) void k_knn_wave(KnnArgs a) {
+// list (4 PW slots wide) are staged in LDS and written together.  The slots
+// are all slots (KW_ALL) or those of the wavefronts in a.defer, whose number
+// only the device knows: block b serves part first + b of the list (KW_LIST),
+// or every gridDim.x-th from there (KW_LOOP: the compiler keeps the loop's
+// invariants in registers, 4 wavefronts a SIMD instead of 7).
+enum { KW_ALL, KW_LIST, KW_LOOP };
+template <int NR, bool PER, bool P64, int PW, int MODE, typename OFF>
+__global__ __launch_bounds__(64 * KW_WAVES) void k_knn_wave(KnnArgs a, uint32_t first) {
+    constexpr bool LIST = MODE != KW_ALL;
     constexpr int NCOL = KW_WAVES * PW;
     constexpr int KMAX = NR > 4 ? 128 : 64;
+    static_assert(WAVE % NCOL == 0, "a deferred wavefront's slots are whole blocks of them");
     __shared__ uint2 s_c[KW_WAVES][64 * NR];
     __shared__ uint32_t s_lq[KW_WAVES][KW_LEAFQ];
     __shared__ uint32_t s_stk[KW_WAVES][MAX_DEPTH / 2 + 1][4];
     __shared__ uint32_t s_out[KMAX * NCOL];
     const int w = threadIdx.x >> 6, row = (threadIdx.x & 63) >> 4;
-    const int64_t slot0 = (int64_t)xcd_remap(blockIdx.x, gridDim.x) * NCOL;
-    // the slot of this lane's row in the smoothing-length stage
-    float tau = 0.f;
-    int32_t st = 0;
-    uint32_t qr = 0;
-    bool on = false;
-    for (int i = 0; i < PW; i++) {
-        const int col = w * PW + i;
+    auto serve = [&](int64_t slot0) {
+        // the slot of this lane's row in the smoothing-length stage
+        float tau = 0.f;
+        int32_t st = 0;
+        uint32_t qr = 0;
+        bool on = false;
+        for (int i = 0; i < PW; i++) {
+            const int col = w * PW + i;
+            const int64_t slot = slot0 + col;
+            if (slot >= a.nq) break;
+            const uint32_t qp = uniform(a.qsorted ? a.qsorted[slot] : (uint32_t)slot);
+            float tq;
+            const int32_t sq = wave_search<NR, PER, P64, OFF>(a, slot, qp, s_c[w], s_lq[w], s_stk[w], s_out, col,
+                                                              NCOL, tq);
+            if (row == i) {
+                tau = tq;
+                st = sq;
+                qr = qp;
+                on = true;
+            }
+        }
+        const int col = w * PW + min(row, PW - 1);
         const int64_t slot = slot0 + col;
-        if (slot >= a.nq) break;
-        const uint32_t qp = uniform(a.qsorted ? a.qsorted[slot] : (uint32_t)slot);
-        float tq;
-        const int32_t sq = wave_search<NR, PER, P64>(a, slot, qp, s_c[w], s_lq[w], s_stk[w], s_out, col, NCOL, tq);
-        if (row == i) {
-            tau = tq;
-            st = sq;
-            qr = qp;
-            on = true;
+        if (__any(on)) {
+            // rows without a query repeat the wavefront's first
+            if (!on) qr = (uint32_t)__shfl((int)qr, 0);
+            const int c = on ? col : w * PW;
+            if (a.k <= 32) row_hsml<2, PER, P64, LIST>(a, on, slot, qr, tau, st, s_out, c, NCOL);
+            else row_hsml<(NR > 4 ? 8 : 4), PER, P64, LIST>(a, on, slot, qr, tau, st, s_out, c, NCOL);
+        }
+        __syncthreads();
+        for (int e = threadIdx.x; e < a.k * NCOL; e += 64 * KW_WAVES) {
+            const int64_t s = slot0 + e % NCOL;
+            if (s < a.nq) a.nl_idx[(int64_t)(e / NCOL) * a.nq + s] = s_out[e];
+        }
+    };
+    constexpr uint32_t PARTS = WAVE / NCOL;
+    auto part = [&](uint32_t b) { return (int64_t)a.defer[1 + b / PARTS] * WAVE + b % PARTS * NCOL; };
+    if constexpr (MODE == KW_ALL) {
+        serve((int64_t)xcd_remap(blockIdx.x, gridDim.x) * NCOL);
+    } else if constexpr (MODE == KW_LIST) {
+        const uint32_t b = first + blockIdx.x;
+        if (b < a.defer[0] * PARTS) serve(part(b));
+    } else {
+        const uint32_t total = a.defer[0] * PARTS;
+        for (uint32_t b = first + blockIdx.x; b < total; b += gridDim.x) {
+            serve(part(b));
+            __syncthreads();  // the next slots reuse s_out
         }
     }
-    const int col = w * PW + min(row, PW - 1);
-    const int64_t slot = slot0 + col;
-    if (__any(on)) {
-        // rows without a query repeat the wavefront's first
-        if (!on) qr = (uint32_t)__shfl((int)qr, 0);
-        const int c = on ? col : w * PW;
-        if (a.k <= 32) row_hsml<2, PER, P64>(a, on, slot, qr, tau, st, s_out, c, NCOL);
-        else row_hsml<(NR > 4 ? 8 : 4), PER, P64>(a, on, slot, qr, tau, st, s_out, c, NCOL);
-    }
-    __syncthreads();
-    for (int e = threadIdx.x; e < a.k * NCOL; e += 64 * KW_WAVES) {
-        const int64_t s = slot0 + e % NCOL;
-        if (s < a.nq) a.nl_idx[(int64_t)(e / NCOL) * a.nq + s] = s_out[e];
-    }
 }
 
-bool knn_wave_serves(int64_t n, int64_t nq, int k) {
+// Where the lines lie (ms of the whole search, one lane / one wavefront per
+// query): k = 32 open 3D float32, 65536 particles 0.200 / 0.135, 10^5 0.212 /
+// 0.212, 3 10^5 0.369 / 0.560; 2D 32768 0.078 / 0.069, 65536 0.076 / 0.104;
+// k = 64 3D 3 10^5 0.69 / 0.68, 10^6 1.85 / 2.31; periodic float64 k = 32
+// 3 10^5 0.77 / 0.68, 10^6 1.90 / 2.28 (wavefronts near the faces come here
+// anyway); k = 100 10^6 3.31 / 2.84, clustered 2^22 16.0 / 13.7.  Few queries
+// in a large set lie far apart and share no leaves.
+bool knn_wave_serves(int64_t n, int64_t nq, int k, int dim, bool per) {
     if (n >= (int64_t)1 << 30) return false;  // 32-bit byte offsets
-    return k > 32 || n <= 100000 || nq < n / 4;
+    if (k > 64 || nq < n / 4) return true;
+    int64_t most = dim == 3 ? 100000 : 45000;
+    if (k > 32) most *= 3;
+    if (per) most *= 3;
+    return n <= most;
 }
 
-template <int NR, int PW>
-static void launch_wave(const KnnArgs &a, bool per, bool p64, hipStream_t s) {
-    const int64_t nb = (a.nq + KW_WAVES * PW - 1) / (KW_WAVES * PW);
-    const dim3 g((unsigned)nb), b(64 * KW_WAVES);
-    if (per && p64) hipLaunchKernelGGL((k_knn_wave<NR, true, true, PW>), g, b, 0, s, a);
-    else if (per) hipLaunchKernelGGL((k_knn_wave<NR, true, false, PW>), g, b, 0, s, a);
-    else if (p64) hipLaunchKernelGGL((k_knn_wave<NR, false, true, PW>), g, b, 0, s, a);
-    else hipLaunchKernelGGL((k_knn_wave<NR, false, false, PW>), g, b, 0, s, a);
+template <int NR, int PW, int MODE, typename OFF>
+static void launch_wave(const KnnArgs &a, bool per, bool p64, int64_t blocks, int64_t first, hipStream_t s) {
+    const dim3 g((unsigned)blocks), b(64 * KW_WAVES);
+    const uint32_t f = (uint32_t)first;
+    if (per && p64) hipLaunchKernelGGL((k_knn_wave<NR, true, true, PW, MODE, OFF>), g, b, 0, s, a, f);
+    else if (per) hipLaunchKernelGGL((k_knn_wave<NR, true, false, PW, MODE, OFF>), g, b, 0, s, a, f);
+    else if (p64) hipLaunchKernelGGL((k_knn_wave<NR, false, true, PW, MODE, OFF>), g, b, 0, s, a, f);
+    else hipLaunchKernelGGL((k_knn_wave<NR, false, false, PW, MODE, OFF>), g, b, 0, s, a, f);
 }
 
-int knn_wave_launch(mhip_ctx *ctx, const KnnArgs &a, bool per, bool p64) {
-    hipStream_t s = ctx->stream;
-    const bool few = a.nq <= 32768;
-    if (a.k <= 64) {
-        if (few) launch_wave<4, 1>(a, per, p64, s);
-        else launch_wave<4, 4>(a, per, p64, s);
+template <int NR>
+static void launch_wave_k(const KnnArgs &a, bool per, bool p64, bool deferred, hipStream_t s) {
+    const int64_t nb = (a.nq + 4 * KW_WAVES - 1) / (4 * KW_WAVES);  // blocks of four slots a wavefront
+    if (deferred) {
+        const int64_t nb = (a.nq + WAVE - 1) / WAVE * (WAVE / (4 * KW_WAVES));  // parts of whole wavefronts
+        // most of the list on a grid that needs no loop: in an open set it is
+        // short, in a periodic one it holds the wavefronts near the faces
+        const int64_t n1 = std::min<int64_t>(nb, per ? KW_LIST_PER : KW_LIST_OPEN);
+        if (a.n >= (int64_t)1 << 30) {
+            launch_wave<NR, 4, KW_LOOP, uint64_t>(a, per, p64, std::min(nb, KW_LIST_OPEN), 0, s);
+            return;
+        }
+        launch_wave<NR, 4, KW_LIST, uint32_t>(a, per, p64, n1, 0, s);
+        if (nb > n1) launch_wave<NR, 4, KW_LOOP, uint32_t>(a, per, p64, std::min(nb - n1, KW_LIST_OPEN), n1, s);
+    } else if (a.nq <= 32768) {
+        // one slot per wavefront while there are fewer wavefronts than the
+        // chip holds, else four
+        launch_wave<NR, 1, KW_ALL, uint32_t>(a, per, p64, (a.nq + KW_WAVES - 1) / KW_WAVES, 0, s);
     } else {
-        if (few) launch_wave<6, 1>(a, per, p64, s);
-        else launch_wave<6, 4>(a, per, p64, s);
+        launch_wave<NR, 4, KW_ALL, uint32_t>(a, per, p64, nb, 0, s);
     }
+}
+
+int knn_wave_launch(mhip_ctx *ctx, const KnnArgs &a, bool per, bool p64, bool deferred) {
+    if (a.k <= 64) launch_wave_k<4>(a, per, p64, deferred, ctx->stream);
+    else launch_wave_k<6>(a, per, p64, deferred, ctx->stream);
     return check_hip(ctx, hipGetLastError(), "knn launch");
 }
 

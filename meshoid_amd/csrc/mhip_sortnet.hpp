@@ -68,7 +68,7 @@ MHIP_HD void oddeven_sort(float (&v)[N]) {
 template <int K, int NS>
 MHIP_HD void merge_sorted(float (&A)[K], const float (&S)[NS]) {
     static_assert(NS <= K, "the list must hold the new values");
-    constexpr int P = K <= 1 ? 1 : K <= 2 ? 2 : K <= 4 ? 4 : K <= 8 ? 8 : K <= 16 ? 16 : K <= 32 ? 32 : K <= 64 ? 64 : 128;
+    constexpr int P = K <= 1 ? 1 : K <= 2 ? 2 : K <= 4 ? 4 : K <= 8 ? 8 : K <= 16 ? 16 : K <= 32 ? 32 : K <= 64 ? 64 : K <= 128 ? 128 : 256;
     static_assert(K <= P, "list too long");
     constexpr int V = P - K;
 #pragma unroll

@@ -36,7 +36,7 @@ def test_wave_search_equals_lane_search(n, k, dim, box, f64, masked):
     p = torch.from_numpy(pos if f64 else np.minimum(pos, 0.99999).astype(np.float32)).cuda()
     ix = engine.SpatialIndex().build(p, box)
     q = torch.from_numpy(rng.permutation(n)[: max(1, n // 5)].astype(np.int64)).cuda() if masked else None
-    out = [engine.knn_hsml(ix, k, qidx=q, small_record=lane) for lane in (False, True)]
+    out = [engine.knn_hsml(ix, k, qidx=q, lane=lane) for lane in (False, True)]
     (na, da), (nb, db) = (o["nlist"].export(f64=True) for o in out)
     fa, fb = (o["nlist"].export()[1] for o in out)
     assert torch.equal(out[0]["status"], out[1]["status"])
