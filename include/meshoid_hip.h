@@ -84,6 +84,14 @@ int mhip_index_create(mhip_index **out);
 int mhip_index_build(mhip_ctx *ctx, mhip_index *ix, const void *pos, int pos_f64, int64_t n,
                      int dim, double boxsize);
 int mhip_index_destroy(mhip_index *ix);
+/* Device memory of the index from the caller (e.g. a caching allocator's):
+ * bytes that n particles need, and the memory, which the caller keeps until
+ * the index is destroyed or given other memory (ptr NULL: the library
+ * allocates again); the index has to be built anew, and a build that needs
+ * more fails with MHIP_ERR_VALUE.  The caller orders its reuse after the
+ * work queued on every stream that used the index. */
+int64_t mhip_index_bytes(int64_t n, int pos_f64);
+int mhip_index_storage(mhip_index *ix, void *ptr, int64_t bytes);
 /* host-side copy of n, dim, boxsize and the bounding box (lo xyz, hi xyz) */
 int mhip_index_info(const mhip_index *ix, int64_t *n, int *dim, double *boxsize, float *bbox6);
 /* the index's particle order: perm_out uint32[n] (device), the original row
@@ -114,6 +122,10 @@ int mhip_index_order(mhip_ctx *ctx, const mhip_index *ix, uint32_t *perm_out);
  */
 int mhip_nlist_create(mhip_nlist **out);
 int mhip_nlist_destroy(mhip_nlist *nl);
+/* device memory of the list from the caller, as mhip_index_storage; masked:
+ * query rows are given (qidx, or a subset of another list) */
+int64_t mhip_nlist_bytes(int64_t nq, int k, int masked, int flags);
+int mhip_nlist_storage(mhip_nlist *nl, void *ptr, int64_t bytes);
 int mhip_knn_hsml(mhip_ctx *ctx, const mhip_index *ix, const int64_t *qidx, int64_t nq, int k,
                   const double *m_rows, const float *seed_h, const float *seed_r, float *h_out,
                   float *rho_out, float *vol_out, int32_t *status_out, int flags, mhip_nlist *nl);
@@ -125,6 +137,15 @@ int mhip_knn_hsml(mhip_ctx *ctx, const mhip_index *ix, const int64_t *qidx, int6
  * may be NULL.  Needs a list built with MHIP_KNN_KEEP_DIST.
  */
 int mhip_nlist_export(mhip_ctx *ctx, const mhip_nlist *nl, int32_t *ngb_out, float *dist_out);
+
+/*
+ * The list's rows in float64, in row order: h (HsmlIter's root), density =
+ * k m / (V_d h^d) and volume = m / density (src/meshoid/Meshoid.py:165-170),
+ * double[nq], and the MHIP_ST_* bits, int32[nq]; any may be NULL.  m_rows
+ * float64[nq] mass of each row, NULL = 1.
+ */
+int mhip_nlist_rows64(mhip_ctx *ctx, const mhip_nlist *nl, const double *m_rows, double *h_out,
+                      double *rho_out, double *vol_out, int32_t *status_out);
 
 /*
  * The same rows with float64 distances, recomputed from the positions the
@@ -162,6 +183,10 @@ int mhip_nlist_hsml(mhip_ctx *ctx, const mhip_nlist *nl, double *h_out);
  */
 int mhip_apply_D(mhip_ctx *ctx, const mhip_nlist *nl, const void *f, int f_f64, int64_t nf_rows,
                  int K, int order, int weighted, float *out_d1, float *out_d2, int32_t *status);
+/* the same; any int32[1] (device, may be NULL): the OR of all rows' status */
+int mhip_apply_D_any(mhip_ctx *ctx, const mhip_nlist *nl, const void *f, int f_f64, int64_t nf_rows,
+                     int K, int order, int weighted, float *out_d1, float *out_d2, int32_t *status,
+                     int32_t *any);
 
 /*
  * gradient_weights(pos, ngb, kernel_radius, indices, boxsize, weighted, order)

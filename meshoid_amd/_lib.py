@@ -35,7 +35,8 @@ EXPORTED = [
     "mhip_batch_tuning", "mhip_batch_force",
     "mhip_index_order", "mhip_nearest", "mhip_unique_inverse", "mhip_reconstruct", "mhip_nlist_subset",
     "mhip_surface_density", "mhip_grid_density", "mhip_radtransfer", "mhip_nlist_export_f64",
-    "mhip_nlist_hsml", "mhip_integrate_noalloc",
+    "mhip_nlist_hsml", "mhip_integrate_noalloc", "mhip_index_bytes", "mhip_index_storage",
+    "mhip_nlist_bytes", "mhip_nlist_storage", "mhip_nlist_rows64", "mhip_apply_D_any",
 ]
 
 if not os.path.exists(LIB_PATH):
@@ -69,6 +70,12 @@ _SIGS = {
     "mhip_nlist_export_f64": ([_p, _p, _p, _p], _i),
     "mhip_nlist_hsml": ([_p, _p, _p], _i),
     "mhip_apply_D": ([_p, _p, _p, _i, _i64, _i, _i, _i, _p, _p, _p], _i),
+    "mhip_apply_D_any": ([_p, _p, _p, _i, _i64, _i, _i, _i, _p, _p, _p, _p], _i),
+    "mhip_index_bytes": ([_i64, _i], _i64),
+    "mhip_index_storage": ([_p, _p, _i64], _i),
+    "mhip_nlist_bytes": ([_i64, _i, _i, _i], _i64),
+    "mhip_nlist_storage": ([_p, _p, _i64], _i),
+    "mhip_nlist_rows64": ([_p, _p, _p, _p, _p, _p, _p], _i),
     "mhip_gradient_weights": ([_p, _p, _i, _i64, _i, _p, _i64, _i, _p, _p, _d, _i, _i, _p, _p],
                               _i),
     "mhip_hsml_iter": ([_p, _p, _i, _i64, _i, _i, _d, _p, _p], _i),

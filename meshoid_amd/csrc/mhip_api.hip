@@ -42,6 +42,25 @@ void *scratch(mhip_ctx *ctx, size_t bytes, int *rc) {
     return ctx->scratch;
 }
 
+int block_reserve(mhip_ctx *ctx, Block &b, size_t need, const char *what) {
+    if (need <= b.bytes) return 0;
+    if (b.ext) return fail(ctx, MHIP_ERR_VALUE, std::string(what) + ": the storage given is too small");
+    if (b.p) (void)hipFree(b.p);
+    b.p = nullptr;
+    b.bytes = 0;
+    const int rc = check_hip(ctx, hipMalloc((void **)&b.p, need), "hipMalloc (index or neighbour list)");
+    if (!rc) b.bytes = need;
+    return rc;
+}
+
+// the caller's memory instead of the library's own (null: the library's again)
+static void block_storage(Block &b, void *p, int64_t bytes) {
+    if (b.p && !b.ext) (void)hipFree(b.p);
+    b.p = (char *)p;
+    b.bytes = p ? (size_t)bytes : 0;
+    b.ext = p != nullptr;
+}
+
 }  // namespace mhip
 
 using namespace mhip;
@@ -185,10 +204,35 @@ int mhip_index_create(mhip_index **out) {
 
 int mhip_index_destroy(mhip_index *ix) {
     if (!ix) return MHIP_OK;
-    void *arrs[] = {ix->sx, ix->sy, ix->sz, ix->lx, ix->ly, ix->lz, ix->perm, ix->iperm, ix->nodes};
-    for (void *p : arrs)
-        if (p) hipFree(p);
+    block_storage(ix->mem, nullptr, 0);
     delete ix;
+    return MHIP_OK;
+}
+
+int64_t mhip_index_bytes(int64_t n, int pos_f64) {
+    if (n < 1) return 0;
+    mhip_index ix;
+    return (int64_t)index_layout(&ix, n, pos_f64 ? 1 : 0, nullptr);
+}
+
+int mhip_index_storage(mhip_index *ix, void *ptr, int64_t bytes) {
+    if (!ix || bytes < 0) return MHIP_ERR_VALUE;
+    ix->n = 0;  // what was built is gone
+    block_storage(ix->mem, ptr, bytes);
+    return MHIP_OK;
+}
+
+int64_t mhip_nlist_bytes(int64_t nq, int k, int masked, int flags) {
+    if (nq < 1 || k < 1) return 0;
+    mhip_nlist nl;
+    return (int64_t)nlist_layout(&nl, nq, k, masked != 0, (flags & MHIP_KNN_KEEP_DIST) != 0, nullptr);
+}
+
+int mhip_nlist_storage(mhip_nlist *nl, void *ptr, int64_t bytes) {
+    if (!nl || bytes < 0) return MHIP_ERR_VALUE;
+    nl->nq = 0;
+    nl->index = nullptr;
+    block_storage(nl->mem, ptr, bytes);
     return MHIP_OK;
 }
 
@@ -228,9 +272,7 @@ int mhip_nlist_create(mhip_nlist **out) {
 
 int mhip_nlist_destroy(mhip_nlist *nl) {
     if (!nl) return MHIP_OK;
-    void *arrs[] = {nl->qsorted, nl->qrow, nl->rowrec, nl->idx, nl->d2, nl->tau, nl->h, nl->h64, nl->status, nl->amb, nl->defer};
-    for (void *p : arrs)
-        if (p) hipFree(p);
+    block_storage(nl->mem, nullptr, 0);
     delete nl;
     return MHIP_OK;
 }
@@ -293,6 +335,14 @@ int mhip_nlist_hsml(mhip_ctx *ctx, const mhip_nlist *nl, double *h_out) {
     return nlist_hsml(ctx, nl, h_out);
 }
 
+int mhip_nlist_rows64(mhip_ctx *ctx, const mhip_nlist *nl, const double *m_rows, double *h_out, double *rho_out,
+                      double *vol_out, int32_t *status_out) {
+    if (!ctx) return MHIP_ERR_VALUE;
+    MHIP_NEED(nl, "null neighbour list");
+    hipSetDevice(ctx->device);
+    return nlist_rows64(ctx, nl, m_rows, h_out, rho_out, vol_out, status_out);
+}
+
 int mhip_nlist_export_f64(mhip_ctx *ctx, const mhip_nlist *nl, int32_t *ngb_out, double *dist_out) {
     if (!ctx) return MHIP_ERR_VALUE;
     MHIP_NEED(nl, "null neighbour list");
@@ -300,14 +350,19 @@ int mhip_nlist_export_f64(mhip_ctx *ctx, const mhip_nlist *nl, int32_t *ngb_out,
     return nlist_export64(ctx, nl, ngb_out, dist_out);
 }
 
-int mhip_apply_D(mhip_ctx *ctx, const mhip_nlist *nl, const void *f, int f_f64, int64_t nf_rows, int K,
-                 int order, int weighted, float *out_d1, float *out_d2, int32_t *status) {
+int mhip_apply_D_any(mhip_ctx *ctx, const mhip_nlist *nl, const void *f, int f_f64, int64_t nf_rows, int K,
+                     int order, int weighted, float *out_d1, float *out_d2, int32_t *status, int32_t *any) {
     if (!ctx) return MHIP_ERR_VALUE;
     MHIP_NEED(nl && f, "null neighbour list or field");
     MHIP_NEED(nf_rows >= 0, "negative field length");
     hipSetDevice(ctx->device);
     return apply_ops(ctx, nl, f, f_f64 ? 1 : 0, nf_rows, K, order, weighted ? 1 : 0, out_d1, out_d2,
-                     status);
+                     status, any);
+}
+
+int mhip_apply_D(mhip_ctx *ctx, const mhip_nlist *nl, const void *f, int f_f64, int64_t nf_rows, int K,
+                 int order, int weighted, float *out_d1, float *out_d2, int32_t *status) {
+    return mhip_apply_D_any(ctx, nl, f, f_f64, nf_rows, K, order, weighted, out_d1, out_d2, status, nullptr);
 }
 
 int mhip_gradient_weights(mhip_ctx *ctx, const void *pos, int pos_f64, int64_t n, int dim, const int32_t *ngb,

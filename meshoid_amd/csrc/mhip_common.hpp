@@ -187,8 +187,33 @@ struct __align__(16) RowRec {
 };
 }  // namespace mhip
 
+namespace mhip {
+// One stretch of device memory behind an object's arrays: the library's own
+// (kept and grown) or the caller's (mhip_*_storage), e.g. from the caller's
+// caching allocator.  A device allocation and its release cost 0.1 to 3 ms
+// each at 2^22 particles, and the release waits for the device.
+struct Block {
+    char *p = nullptr;
+    size_t bytes = 0;
+    bool ext = false;
+};
+// successive arrays of a block, 256-byte aligned (p null: sizes only)
+struct Carve {
+    char *p;
+    size_t off = 0;
+    template <typename T>
+    T *take(int64_t n) {
+        off = (off + 255) & ~(size_t)255;
+        T *r = p ? (T *)(p + off) : nullptr;
+        off += (size_t)n * sizeof(T);
+        return r;
+    }
+};
+}  // namespace mhip
+
 struct mhip_index {
-    int64_t n = 0, npad = 0, cap = 0;
+    mhip::Block mem;
+    int64_t n = 0, npad = 0;
     int dim = 3;
     double box = -1.0;  // > 0: periodic in [0, box)^dim
     int pos_f64 = 0;
@@ -206,13 +231,13 @@ struct mhip_index {
     int depth = 0;
     int64_t nleaf = 0, first_leaf = 0, nnodes = 0;
     float *nodes = nullptr;
-    int64_t node_cap = 0;
     float bbox[6] = {};
     float frame[4] = {};  // sort-key quantisation: origin xyz, scale (cells per unit, 2^21 - 1 over the extent)
 };
 
 struct mhip_nlist {
-    int64_t nq = 0, cap = 0;
+    mhip::Block mem;
+    int64_t nq = 0;
     int k = 0;
     uint32_t *qsorted = nullptr;  // sorted-space particle index of each query slot
     uint32_t *qrow = nullptr;     // output row of each query slot

@@ -72,8 +72,10 @@ __global__ __launch_bounds__(256) void k_pack_xyzf(const float *__restrict__ sx,
 __global__ __launch_bounds__(256) void k_pack_xyzf_rows(const float *__restrict__ sx, const float *__restrict__ sy,
                                                        const float *__restrict__ sz, const float *__restrict__ f,
                                                        int64_t nf_rows, const uint32_t *__restrict__ perm,
-                                                       int64_t n, int64_t npad, float4 *__restrict__ out) {
+                                                       int64_t n, int64_t npad, float4 *__restrict__ out,
+                                                       int32_t *__restrict__ any) {
     const int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (p == 0 && any) *any = 0;  // the derivative kernel's status word
     if (p >= npad) return;
     const uint32_t o = p < n ? perm[p] : 0xffffffffu;
     out[p] = make_float4(sx[p], sy[p], sz[p], o < nf_rows ? f[o] : NAN);
@@ -228,6 +230,7 @@ MHIP_DEV void apply_row(const ApplyArgs &a, int64_t s, int fb, int fe, int gl = 
         }
     }
     if (a.status && gl == 0) a.status[row] = a.or_status ? (a.status[row] | st) : st;
+    if (a.any && gl == 0 && st) atomicOr(a.any, st);
 }
 
 // apply_row for the common case of one float32 field, 3D, first order,
@@ -320,6 +323,7 @@ MHIP_DEV void apply_row_packed1(const ApplyArgs &a, int64_t s, int gl) {
         for (int i = 0; i < 3; i++) o[i] = ok ? (float)B[i] : NAN;
     }
     if (a.status) a.status[row] = a.or_status ? (a.status[row] | st) : st;
+    if (a.any && st) atomicOr(a.any, st);
 }
 
 // lanes per query: 2 for first-order fits (measured at 2^24, k = 32, with the
@@ -703,6 +707,7 @@ void apply_args_fill(const mhip_nlist *nl, const void *fs, int K, float *out1, i
     a->out2 = nullptr;
     a->status = status;
     a->or_status = or_status;
+    a->any = nullptr;
 }
 
 template <int DIM, int ORDER, typename FT>
@@ -730,7 +735,7 @@ static void dispatch_apply(const ApplyArgs &a, int dim, int order, dim3 g, hipSt
 }
 
 int apply_ops(mhip_ctx *ctx, const mhip_nlist *nl, const void *f, int f_f64, int64_t nf_rows, int K,
-              int order, int weighted, float *out1, float *out2, int32_t *status) {
+              int order, int weighted, float *out1, float *out2, int32_t *status, int32_t *any) {
     const mhip_index *ix = nl->index;
     if (!ix || nl->nq < 1) return fail(ctx, -1, "neighbour list is empty");
     if (order != 1 && order != 2) return fail(ctx, -1, "order must be 1 or 2");
@@ -751,13 +756,13 @@ int apply_ops(mhip_ctx *ctx, const mhip_nlist *nl, const void *f, int f_f64, int
     ProfRegion prp(ctx, "apply_permute_fields");
     if (packed1)
         hipLaunchKernelGGL(k_pack_xyzf_rows, gp, dim3(256), 0, ctx->stream, ix->sx, ix->sy, ix->sz,
-                           (const float *)f, nf_rows, ix->perm, ix->n, ix->npad, xyzf);
+                           (const float *)f, nf_rows, ix->perm, ix->n, ix->npad, xyzf, any);
     else if (f_f64)
         hipLaunchKernelGGL(k_permute_fields<double>, gp, dim3(256), 0, ctx->stream, (const double *)f,
-                           nf_rows, K, ix->perm, ix->n, ix->npad, (double *)fs);
+                           nf_rows, K, ix->perm, ix->n, ix->npad, (double *)fs, any);
     else
         hipLaunchKernelGGL(k_permute_fields<float>, gp, dim3(256), 0, ctx->stream, (const float *)f,
-                           nf_rows, K, ix->perm, ix->n, ix->npad, (float *)fs);
+                           nf_rows, K, ix->perm, ix->n, ix->npad, (float *)fs, any);
     if (pack && !packed1)
         hipLaunchKernelGGL(k_pack_xyzf, gp, dim3(256), 0, ctx->stream, ix->sx, ix->sy, ix->sz, (const float *)fs,
                            ix->npad, xyzf);
@@ -788,6 +793,7 @@ int apply_ops(mhip_ctx *ctx, const mhip_nlist *nl, const void *f, int f_f64, int
     a.out2 = out2;
     a.status = status;
     a.or_status = 0;
+    a.any = any;
     prp.end();
     ProfRegion pra(ctx, order == 1 ? "apply_D1" : "apply_D2");
     if (packed1) {

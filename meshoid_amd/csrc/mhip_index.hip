@@ -462,13 +462,39 @@ __global__ __launch_bounds__(256) void k_node_boxes(float *__restrict__ nodes, i
     o[1] = make_float4(hi[1], hi[2], 0.f, 0.f);
 }
 
-static int grow(mhip_ctx *ctx, void **p, size_t bytes) {
-    if (*p) {
-        hipFree(*p);
-        *p = nullptr;
+// leaves and depth of the complete 8-ary tree over n particles
+struct TreeShape {
+    int64_t npad, nleaf, nslots, first_leaf, nodes;
+    int depth;
+};
+static TreeShape tree_shape(int64_t n) {
+    TreeShape t;
+    t.npad = (n + LEAF - 1) / LEAF * LEAF;
+    t.nleaf = t.npad / LEAF;
+    t.depth = 0;
+    t.nslots = 1;
+    while (t.nslots < t.nleaf) {
+        t.nslots *= FANOUT;
+        t.depth++;
     }
-    if (bytes == 0) return 0;
-    return check_hip(ctx, hipMalloc(p, bytes), "hipMalloc (index)");
+    t.first_leaf = (t.nslots - 1) / (FANOUT - 1);
+    t.nodes = t.first_leaf + t.nslots;
+    return t;
+}
+
+size_t index_layout(mhip_index *ix, int64_t n, int pos_f64, char *base) {
+    const TreeShape t = tree_shape(n);
+    Carve c{base};
+    ix->sx = c.take<float>(t.npad);
+    ix->sy = c.take<float>(t.npad);
+    ix->sz = c.take<float>(t.npad);
+    ix->lx = pos_f64 ? c.take<float>(t.npad) : nullptr;
+    ix->ly = pos_f64 ? c.take<float>(t.npad) : nullptr;
+    ix->lz = pos_f64 ? c.take<float>(t.npad) : nullptr;
+    ix->perm = c.take<uint32_t>(t.npad);
+    ix->iperm = c.take<uint32_t>(t.npad);
+    ix->nodes = c.take<float>(t.nodes * 8);
+    return c.off;
 }
 
 int index_build(mhip_ctx *ctx, const void *pos, int pos_f64, int64_t n, int dim, double box,
@@ -476,32 +502,13 @@ int index_build(mhip_ctx *ctx, const void *pos, int pos_f64, int64_t n, int dim,
     if (n < 1) return fail(ctx, -1, "index needs at least one particle");
     if (n >= (int64_t)0xffffffff) return fail(ctx, -4, "more than 2^32-2 particles");
     if (dim < 1 || dim > 3) return fail(ctx, -5, "dim must be 1, 2 or 3");
-    const int64_t npad = (n + LEAF - 1) / LEAF * LEAF;
-    const int64_t nleaf = npad / LEAF;
+    const TreeShape ts = tree_shape(n);
+    const int64_t npad = ts.npad, nleaf = ts.nleaf, nslots = ts.nslots, first_leaf = ts.first_leaf, tot = ts.nodes;
+    const int depth = ts.depth;
     int rc = 0;
-    // complete 8-ary tree over the leaves
-    int depth = 0;
-    int64_t nslots = 1;
-    while (nslots < nleaf) {
-        nslots *= FANOUT;
-        depth++;
-    }
     if (depth > MAX_DEPTH) return fail(ctx, -4, "tree too deep");
-    const int64_t first_leaf = (nslots - 1) / (FANOUT - 1);
-    const int64_t tot = first_leaf + nslots;
-    if (ix->cap < npad || (pos_f64 && !ix->lx)) {
-        void **arrs[6] = {(void **)&ix->sx, (void **)&ix->sy, (void **)&ix->sz,
-                          (void **)&ix->lx, (void **)&ix->ly, (void **)&ix->lz};
-        for (int a = 0; a < 6; a++)
-            if ((rc = grow(ctx, arrs[a], (a < 3 || pos_f64) ? npad * sizeof(float) : 0))) return rc;
-        if ((rc = grow(ctx, (void **)&ix->perm, npad * sizeof(uint32_t)))) return rc;
-        if ((rc = grow(ctx, (void **)&ix->iperm, npad * sizeof(uint32_t)))) return rc;
-        ix->cap = npad;
-    }
-    if (ix->node_cap < tot) {
-        if ((rc = grow(ctx, (void **)&ix->nodes, tot * 8 * sizeof(float)))) return rc;
-        ix->node_cap = tot;
-    }
+    if ((rc = block_reserve(ctx, ix->mem, index_layout(ix, n, pos_f64, nullptr), "index"))) return rc;
+    index_layout(ix, n, pos_f64, ix->mem.p);
     ix->iperm_ok = 0;
     ix->n = n;
     ix->npad = npad;

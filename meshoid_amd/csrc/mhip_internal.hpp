@@ -11,6 +11,13 @@ int fail(mhip_ctx *ctx, int code, const std::string &msg);
 int check_hip(mhip_ctx *ctx, hipError_t e, const char *what);
 void *scratch(mhip_ctx *ctx, size_t bytes, int *rc);
 
+// at least need bytes behind b (the caller's storage cannot grow)
+int block_reserve(mhip_ctx *ctx, Block &b, size_t need, const char *what);
+// arrays of an index / a neighbour list within base (null: sizes only);
+// returns the bytes they take
+size_t index_layout(mhip_index *ix, int64_t n, int pos_f64, char *base);
+size_t nlist_layout(mhip_nlist *nl, int64_t nq, int k, bool masked, bool d2, char *base);
+
 // Stable LSD radix sort of (u64 key, u32 value) pairs on bits [lo_bit, bits)
 // of the key (lo_bit a multiple of 8).  Buffers: k0/v0 hold the input; the
 // sorted result is returned in *kout/*vout (one of the two ping-pong
@@ -49,6 +56,8 @@ size_t mlp_blob_bytes();
 int nlist_export(mhip_ctx *ctx, const mhip_nlist *nl, int32_t *ngb_out, float *dist_out);
 int nlist_export64(mhip_ctx *ctx, const mhip_nlist *nl, int32_t *ngb_out, double *dist_out);
 int nlist_hsml(mhip_ctx *ctx, const mhip_nlist *nl, double *h_out);
+int nlist_rows64(mhip_ctx *ctx, const mhip_nlist *nl, const double *m_rows, double *h, double *rho, double *vol,
+                 int32_t *status);
 int nlist_subset(mhip_ctx *ctx, const mhip_nlist *full, const int64_t *qidx, int64_t nq, const double *m_rows,
                  float *h_out, float *rho_out, float *vol_out, int32_t *status_out, mhip_nlist *nl);
 
@@ -72,7 +81,7 @@ int reconstruct(mhip_ctx *ctx, const double *targets, int64_t nt, int dim, doubl
                 const float *d1, const float *d2, int order, void *out);
 
 int apply_ops(mhip_ctx *ctx, const mhip_nlist *nl, const void *f, int f_f64, int64_t nf_rows,
-              int K, int order, int weighted, float *out1, float *out2, int32_t *status);
+              int K, int order, int weighted, float *out1, float *out2, int32_t *status, int32_t *any);
 
 int weights_rows(mhip_ctx *ctx, const void *pos, int pos_f64, int64_t n, int dim,
                  const int32_t *ngb, int64_t nq, int k, const double *h, const int64_t *indices,
@@ -100,6 +109,7 @@ struct ApplyArgs {
     float *out1, *out2;  // [row][K][DIM], [row][K][ND-DIM]
     int32_t *status;     // per row, may be null
     int or_status;       // 1: OR the bits into status instead of storing them
+    int32_t *any;        // OR of every row's bits (cleared by the field permutation), may be null
 };
 
 // every snapshot of a batch in one launch (table and block prefix on the
@@ -154,8 +164,10 @@ int integrate(mhip_ctx *ctx, const void *vol, int vol_f64, const void *f, int f_
 template <typename FT>
 __global__ __launch_bounds__(256) void k_permute_fields(const FT *__restrict__ f, int64_t nf_rows, int K,
                                                        const uint32_t *__restrict__ perm, int64_t n,
-                                                       int64_t npad, FT *__restrict__ fs) {
+                                                       int64_t npad, FT *__restrict__ fs,
+                                                       int32_t *__restrict__ any = nullptr) {
     const int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (p == 0 && any) *any = 0;  // the derivative kernel's status word
     if (p >= npad) return;
     const uint32_t o = p < n ? perm[p] : 0xffffffffu;
     for (int c = 0; c < K; c++) {

@@ -1014,13 +1014,6 @@ __global__ __launch_bounds__(256) void k_rows_split(const RowRec *__restrict__ r
     if (status_out) status_out[r] = v.status;
 }
 
-static int nl_grow(mhip_ctx *ctx, void **p, size_t bytes) {
-    if (*p) (void)hipFree(*p);
-    *p = nullptr;
-    if (!bytes) return 0;
-    return check_hip(ctx, hipMalloc(p, bytes), "hipMalloc (neighbour list)");
-}
-
 template <int KCAP>
 static void launch_main(const KnnArgs &a, bool p64, dim3 g, hipStream_t s) {
     if (p64)
@@ -1041,22 +1034,29 @@ static void launch_main_k(const KnnArgs &a, bool p64, dim3 g, hipStream_t s) {
     else launch_main<129>(a, p64, g, s);
 }
 
-static int nl_reserve(mhip_ctx *ctx, mhip_nlist *nl, int64_t nq, int k) {
-    int rc = 0;
-    if (nl->cap < nq || nl->k < k) {
-        void **arr[] = {(void **)&nl->qsorted, (void **)&nl->qrow, (void **)&nl->tau,
-                        (void **)&nl->h,       (void **)&nl->status};
-        for (auto p : arr)
-            if ((rc = nl_grow(ctx, p, nq * 4))) return rc;
-        if ((rc = nl_grow(ctx, (void **)&nl->rowrec, nq * 16))) return rc;
-        if ((rc = nl_grow(ctx, (void **)&nl->amb, (nq + 1) * 4))) return rc;
-        if ((rc = nl_grow(ctx, (void **)&nl->defer, (nq / WAVE + 2) * 4))) return rc;
-        if ((rc = nl_grow(ctx, (void **)&nl->h64, nq * 8))) return rc;
-        if ((rc = nl_grow(ctx, (void **)&nl->idx, (size_t)nq * k * 4))) return rc;
-        if ((rc = nl_grow(ctx, (void **)&nl->d2, (size_t)nq * k * 4))) return rc;
-        nl->cap = nq;
-        nl->k = k;
+size_t nlist_layout(mhip_nlist *nl, int64_t nq, int k, bool masked, bool d2, char *base) {
+    Carve c{base};
+    nl->idx = c.take<uint32_t>(nq * k);
+    nl->h64 = c.take<double>(nq);
+    nl->rowrec = c.take<RowRec>(nq);
+    nl->tau = c.take<float>(nq);
+    nl->h = c.take<float>(nq);
+    nl->status = c.take<int32_t>(nq);
+    nl->amb = c.take<uint32_t>(nq + 1);
+    nl->defer = c.take<uint32_t>(nq / WAVE + 2);
+    nl->qsorted = masked ? c.take<uint32_t>(nq) : nullptr;
+    nl->qrow = masked ? c.take<uint32_t>(nq) : nullptr;
+    nl->d2 = d2 ? c.take<float>(nq * k) : nullptr;
+    return c.off;
+}
+
+static int nl_reserve(mhip_ctx *ctx, mhip_nlist *nl, int64_t nq, int k, bool masked, bool d2) {
+    const int rc = block_reserve(ctx, nl->mem, nlist_layout(nl, nq, k, masked, d2, nullptr), "neighbour list");
+    if (rc) {
+        nl->nq = 0;
+        return rc;
     }
+    nlist_layout(nl, nq, k, masked, d2, nl->mem.p);
     return 0;
 }
 
@@ -1113,7 +1113,7 @@ int knn_run(mhip_ctx *ctx, const mhip_index *ix, const int64_t *qidx, int64_t nq
     if (!qidx) nq = ix->n;
     if (nq < 1) return fail(ctx, -1, "no query rows");
     int rc = 0;
-    if ((rc = nl_reserve(ctx, nl, nq, k))) return rc;
+    if ((rc = nl_reserve(ctx, nl, nq, k, qidx != nullptr, (flags & 1) != 0))) return rc;
     nl->nq = nq;
     nl->k = k;
     nl->index = ix;
@@ -1267,7 +1267,7 @@ int nlist_subset(mhip_ctx *ctx, const mhip_nlist *full, const int64_t *qidx, int
     if (nq < 1) return fail(ctx, -1, "no query rows");
     const int k = full->k;
     int rc = 0;
-    if ((rc = nl_reserve(ctx, nl, nq, k))) return rc;
+    if ((rc = nl_reserve(ctx, nl, nq, k, true, full->has_d2 != 0))) return rc;
     nl->nq = nq;
     nl->k = k;
     nl->index = ix;
@@ -1356,6 +1356,54 @@ int nlist_hsml(mhip_ctx *ctx, const mhip_nlist *nl, double *h_out) {
     hipLaunchKernelGGL(k_rows_h64, dim3((unsigned)((nl->nq + 255) / 256)), dim3(256), 0, ctx->stream, nl->h64,
                        nl->masked ? nl->qrow : nullptr, nl->index->perm, nl->nq, h_out);
     return check_hip(ctx, hipGetLastError(), "hsml copy launch");
+}
+
+// h, density and volume of the rows in float64 (Meshoid.py:165-170) and their
+// status: as k_rows_rec and k_rows_split, one scattered record per row (two
+// 16-byte writes to one 32-byte sector), then a coalesced split
+struct __align__(16) RowRec64 {
+    double h, rho, vol;
+    int32_t status, pad;
+};
+__global__ __launch_bounds__(256) void k_rows64_rec(const uint32_t *__restrict__ srow, int64_t nq, int k, int dim,
+                                                   const double *__restrict__ h64, const int32_t *__restrict__ st,
+                                                   const double *__restrict__ m_rows, RowRec64 *__restrict__ rec) {
+    const int64_t s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (s >= nq) return;
+    const uint32_t r = srow[s];
+    const double h = h64[s];
+    const double vn = dim == 3 ? 4.18879020478639098 : (dim == 2 ? 3.14159265358979324 : 2.0);
+    const double m = m_rows ? m_rows[r] : 1.0;
+    const double hp = dim == 3 ? h * h * h : (dim == 2 ? h * h : h);
+    const double rho = (double)k * m / (vn * hp);
+    rec[r] = RowRec64{h, rho, m / rho, st[s], 0};
+}
+
+__global__ __launch_bounds__(256) void k_rows64_split(const RowRec64 *__restrict__ rec, int64_t nq,
+                                                     double *__restrict__ h, double *__restrict__ rho,
+                                                     double *__restrict__ vol, int32_t *__restrict__ status) {
+    const int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (r >= nq) return;
+    const RowRec64 v = rec[r];
+    if (h) h[r] = v.h;
+    if (rho) rho[r] = v.rho;
+    if (vol) vol[r] = v.vol;
+    if (status) status[r] = v.status;
+}
+
+int nlist_rows64(mhip_ctx *ctx, const mhip_nlist *nl, const double *m_rows, double *h, double *rho, double *vol,
+                 int32_t *status) {
+    const mhip_index *ix = nl->index;
+    if (!ix || nl->nq < 1) return fail(ctx, -1, "neighbour list is empty");
+    int rc = 0;
+    RowRec64 *rec = (RowRec64 *)scratch(ctx, (size_t)nl->nq * sizeof(RowRec64), &rc);
+    if (!rec) return rc;
+    ProfRegion pr(ctx, "nlist_rows64");
+    const dim3 g((unsigned)((nl->nq + 255) / 256));
+    hipLaunchKernelGGL(k_rows64_rec, g, dim3(256), 0, ctx->stream, nl->masked ? nl->qrow : ix->perm, nl->nq, nl->k,
+                       ix->dim, nl->h64, nl->status, m_rows, rec);
+    hipLaunchKernelGGL(k_rows64_split, g, dim3(256), 0, ctx->stream, rec, nl->nq, h, rho, vol, status);
+    return check_hip(ctx, hipGetLastError(), "row output launch");
 }
 
 int nlist_export(mhip_ctx *ctx, const mhip_nlist *nl, int32_t *ngb_out, float *dist_out) {

@@ -23,8 +23,9 @@ def _dev_index(device) -> int:
     return d.index if d.index is not None else torch.cuda.current_device()
 
 
-def context(device=None) -> ctypes.c_void_p:
-    """Per-device context bound to torch's current stream of that device."""
+def context(device=None, *objs) -> ctypes.c_void_p:
+    """Per-device context bound to torch's current stream of that device.
+    objs: the indices and lists whose memory the call uses."""
     idx = _dev_index(device)
     ctx = _CTX.get(idx)
     if ctx is None:
@@ -34,8 +35,36 @@ def context(device=None) -> ctypes.c_void_p:
         rc = lib.mhip_ctx_create(idx, None, ctypes.byref(ctx))
         raise_for(rc, None, "mhip_ctx_create failed")
         _CTX[idx] = ctx
-    lib.mhip_ctx_set_stream(ctx, ctypes.c_void_p(torch.cuda.current_stream(idx).cuda_stream))
+    stream = torch.cuda.current_stream(idx)
+    lib.mhip_ctx_set_stream(ctx, ctypes.c_void_p(stream.cuda_stream))
+    for o in objs:
+        o._mem.used_on(stream)
     return ctx
+
+
+class _Memory:
+    """Device memory of an index or a list, from torch's caching allocator: a
+    program that makes and drops them (every Meshoid does) gets the same
+    blocks back without the driver allocating and, on release, waiting for the
+    device.  The block is freed on the stream it was allocated on; other
+    streams that use it are made known to the allocator."""
+
+    __slots__ = ("block", "stream")
+
+    def __init__(self):
+        self.block = self.stream = None
+
+    def reserve(self, need, device, give):
+        """At least need bytes on device; give(pointer, bytes) on a new block."""
+        if self.block is not None and self.block.numel() >= need and self.block.device == device:
+            return
+        self.block = torch.empty(max(int(need), 1), dtype=torch.uint8, device=device)
+        self.stream = torch.cuda.current_stream(device).cuda_stream
+        raise_for(give(ctypes.c_void_p(self.block.data_ptr()), self.block.numel()), None, "storage")
+
+    def used_on(self, stream):
+        if self.block is not None and stream.cuda_stream != self.stream:
+            self.block.record_stream(stream)
 
 
 def prof_enable(level=1, device=None):
@@ -78,6 +107,7 @@ class SpatialIndex:
     def __init__(self):
         self.h = ctypes.c_void_p()
         raise_for(lib.mhip_index_create(ctypes.byref(self.h)), None, "index create")
+        self._mem = _Memory()
         self.pos = None
         self.n = 0
         self.dim = 0
@@ -88,8 +118,11 @@ class SpatialIndex:
         if pos.dim() == 1:
             pos = pos[:, None]
         n, dim = pos.shape
-        ctx = context(pos.device)
-        rc = lib.mhip_index_build(ctx, self.h, ptr(pos), int(pos.dtype == torch.float64), n, dim,
+        f64 = int(pos.dtype == torch.float64)
+        self._mem.reserve(lib.mhip_index_bytes(n, f64), pos.device,
+                          lambda p, b: lib.mhip_index_storage(self.h, p, b))
+        ctx = context(pos.device, self)
+        rc = lib.mhip_index_build(ctx, self.h, ptr(pos), f64, n, dim,
                                   float(boxsize) if boxsize else -1.0)
         raise_for(rc, ctx)
         self.pos = pos  # the library reads it for float64 boundary resolution
@@ -99,7 +132,7 @@ class SpatialIndex:
     def order(self) -> torch.Tensor:
         """Original row of each sorted position (int64, Hilbert order)."""
         perm = torch.empty(self.n, dtype=torch.int32, device=self.pos.device)
-        ctx = context(self.pos.device)
+        ctx = context(self.pos.device, self)
         raise_for(lib.mhip_index_order(ctx, self.h, ptr(perm)), ctx)
         return perm.to(torch.int64)
 
@@ -110,7 +143,7 @@ class SpatialIndex:
         return [float(v) for v in bb]
 
     def __del__(self):
-        if getattr(self, "h", None):
+        if getattr(self, "h", None) and lib is not None:
             lib.mhip_index_destroy(self.h)
             self.h = None
 
@@ -121,10 +154,16 @@ class NeighborList:
     def __init__(self):
         self.h = ctypes.c_void_p()
         raise_for(lib.mhip_nlist_create(ctypes.byref(self.h)), None, "nlist create")
+        self._mem = _Memory()
         self.nq = 0
         self.k = 0
         self.index = None
         self.keep_dist = False
+
+    def _reserve(self, nq, k, masked, keep_dist, device):
+        flags = _lib.KNN_KEEP_DIST if keep_dist else 0
+        self._mem.reserve(lib.mhip_nlist_bytes(nq, k, int(masked), flags), device,
+                          lambda p, b: lib.mhip_nlist_storage(self.h, p, b))
 
     def export(self, want_ngb=True, want_dist=True, f64=False):
         """(ngb int32 (nq,k), dist (nq,k)) rows ascending, as cKDTree.query.
@@ -134,7 +173,7 @@ class NeighborList:
         ngb = torch.empty((self.nq, self.k), dtype=torch.int32, device=dev) if want_ngb else None
         dt = torch.float64 if f64 else torch.float32
         dist = torch.empty((self.nq, self.k), dtype=dt, device=dev) if want_dist else None
-        ctx = context(dev)
+        ctx = context(dev, self, self.index)
         fn = lib.mhip_nlist_export_f64 if f64 else lib.mhip_nlist_export
         raise_for(fn(ctx, self.h, ptr(ngb), ptr(dist)), ctx)
         return ngb, dist
@@ -143,12 +182,24 @@ class NeighborList:
         """float64 smoothing lengths of the rows (nq,), refined over the final
         neighbours; the derivative operators fit with these."""
         out = torch.empty(self.nq, dtype=torch.float64, device=self.index.pos.device)
-        ctx = context(out.device)
+        ctx = context(out.device, self, self.index)
         raise_for(lib.mhip_nlist_hsml(ctx, self.h, ptr(out)), ctx)
         return out
 
+    def rows64(self, m_rows=None):
+        """(h, density, volume, status) of the rows: float64 and int32 (nq,)."""
+        _need(m_rows, (torch.float64,), "m_rows")
+        if m_rows is not None and m_rows.numel() != self.nq:
+            raise ValueError("m_rows must have one entry per query row")
+        dev = self.index.pos.device
+        h, rho, vol = (torch.empty(self.nq, dtype=torch.float64, device=dev) for _ in range(3))
+        status = torch.empty(self.nq, dtype=torch.int32, device=dev)
+        ctx = context(dev, self, self.index)
+        raise_for(lib.mhip_nlist_rows64(ctx, self.h, ptr(m_rows), ptr(h), ptr(rho), ptr(vol), ptr(status)), ctx)
+        return h, rho, vol, status
+
     def __del__(self):
-        if getattr(self, "h", None):
+        if getattr(self, "h", None) and lib is not None:
             lib.mhip_nlist_destroy(self.h)
             self.h = None
 
@@ -177,7 +228,8 @@ def knn_hsml(index: SpatialIndex, k: int, qidx=None, m_rows=None, seed_h=None, k
         out = {name: torch.empty(nq, dtype=torch.float32, device=dev) for name in ("h", "rho", "vol")}
         out["status"] = torch.empty(nq, dtype=torch.int32, device=dev)
     nl = nlist if nlist is not None else NeighborList()
-    ctx = context(dev)
+    nl._reserve(nq, int(k), qidx is not None, keep_dist, dev)
+    ctx = context(dev, nl, index)
     rc = lib.mhip_knn_hsml(ctx, index.h, ptr(qidx), nq, int(k), ptr(m_rows), ptr(seed_h),
                            ptr(seed_r), ptr(out.get("h")), ptr(out.get("rho")), ptr(out.get("vol")),
                            ptr(out.get("status")),
@@ -190,7 +242,8 @@ def knn_hsml(index: SpatialIndex, k: int, qidx=None, m_rows=None, seed_h=None, k
     return out
 
 
-def nlist_subset(full: NeighborList, qidx: torch.Tensor, m_rows=None, nlist: NeighborList | None = None):
+def nlist_subset(full: NeighborList, qidx: torch.Tensor, m_rows=None, nlist: NeighborList | None = None,
+                 out=None):
     """The rows qidx of an unmasked list: what knn_hsml(index, k, qidx=qidx,
     m_rows=m_rows) returns, without a new search (a particle's neighbours and
     smoothing length do not depend on the mask)."""
@@ -203,23 +256,27 @@ def nlist_subset(full: NeighborList, qidx: torch.Tensor, m_rows=None, nlist: Nei
         raise IndexError("query index out of range")
     if m_rows is not None and m_rows.numel() != nq:
         raise ValueError("m_rows must have one entry per query row")
-    out = {name: torch.empty(nq, dtype=torch.float32, device=dev) for name in ("h", "rho", "vol")}
-    out["status"] = torch.empty(nq, dtype=torch.int32, device=dev)
+    if out is None:
+        out = {name: torch.empty(nq, dtype=torch.float32, device=dev) for name in ("h", "rho", "vol")}
+        out["status"] = torch.empty(nq, dtype=torch.int32, device=dev)
     nl = nlist if nlist is not None else NeighborList()
-    ctx = context(dev)
-    raise_for(lib.mhip_nlist_subset(ctx, full.h, ptr(qidx), nq, ptr(m_rows), ptr(out["h"]), ptr(out["rho"]),
-                                    ptr(out["vol"]), ptr(out["status"]), nl.h), ctx)
+    nl._reserve(nq, full.k, True, full.keep_dist, dev)
+    ctx = context(dev, nl, full, index)
+    raise_for(lib.mhip_nlist_subset(ctx, full.h, ptr(qidx), nq, ptr(m_rows), ptr(out.get("h")),
+                                    ptr(out.get("rho")), ptr(out.get("vol")), ptr(out.get("status")), nl.h), ctx)
     nl.nq, nl.k, nl.index, nl.keep_dist = nq, full.k, index, full.keep_dist
     out["nlist"] = nl
     return out
 
 
 def apply_D(nl: NeighborList, f: torch.Tensor, order=1, weighted=True, want_d1=True,
-            want_d2=False, out1=None, out2=None, status=None):
+            want_d2=False, out1=None, out2=None, status=None, any_status=None):
     """Least-squares derivatives of f over the list's rows.
 
     f: (nf_rows, K) contiguous float32/float64 device tensor.  Returns
-    (d1 (nq,K,dim) or None, d2 (nq,K,nd2) or None, status int32 (nq,))."""
+    (d1 (nq,K,dim) or None, d2 (nq,K,nd2) or None, status int32 (nq,)).
+    any_status: int32 (1,) device tensor that takes the OR of the rows' status
+    instead (status is then None unless given)."""
     _need(f, (torch.float32, torch.float64), "f")
     if f.dim() == 1:
         f = f[:, None]
@@ -231,12 +288,12 @@ def apply_D(nl: NeighborList, f: torch.Tensor, order=1, weighted=True, want_d1=T
         out1 = torch.empty((nl.nq, K, dim), dtype=torch.float32, device=dev)
     if want_d2 and out2 is None:
         out2 = torch.empty((nl.nq, K, nd2), dtype=torch.float32, device=dev)
-    if status is None:
+    if status is None and any_status is None:
         status = torch.empty(nl.nq, dtype=torch.int32, device=dev)
-    ctx = context(dev)
-    rc = lib.mhip_apply_D(ctx, nl.h, ptr(f), int(f.dtype == torch.float64), nf, K, int(order),
-                          int(bool(weighted)), ptr(out1 if want_d1 else None),
-                          ptr(out2 if want_d2 else None), ptr(status))
+    ctx = context(dev, nl, nl.index)
+    rc = lib.mhip_apply_D_any(ctx, nl.h, ptr(f), int(f.dtype == torch.float64), nf, K, int(order),
+                              int(bool(weighted)), ptr(out1 if want_d1 else None),
+                              ptr(out2 if want_d2 else None), ptr(status), ptr(any_status))
     raise_for(rc, ctx)
     return (out1 if want_d1 else None), (out2 if want_d2 else None), status
 
@@ -310,7 +367,7 @@ def kernel_average(nl: NeighborList, f: torch.Tensor) -> torch.Tensor:
     if f.dim() != 1:
         raise ValueError("KernelAverage takes a scalar field of shape (N,)")
     out = torch.empty(nl.nq, dtype=torch.float64, device=f.device)
-    ctx = context(f.device)
+    ctx = context(f.device, nl, nl.index)
     raise_for(lib.mhip_kernel_average(ctx, nl.h, ptr(f), int(f.dtype == torch.float64), f.shape[0],
                                       ptr(out)), ctx)
     return out
@@ -323,7 +380,7 @@ def kernel_variance(nl: NeighborList, f: torch.Tensor) -> torch.Tensor:
     f2 = f.reshape(f.shape[0], -1).contiguous() if f.dim() != 2 else f
     K = f2.shape[1]
     out = torch.empty((nl.nq, K), dtype=torch.float64, device=f.device)
-    ctx = context(f.device)
+    ctx = context(f.device, nl, nl.index)
     raise_for(lib.mhip_kernel_variance(ctx, nl.h, ptr(f2), int(f.dtype == torch.float64), f2.shape[0],
                                        K, ptr(out)), ctx)
     return out
@@ -373,7 +430,7 @@ def nearest(index: SpatialIndex, points: torch.Tensor) -> torch.Tensor:
     if dim != index.dim:
         raise ValueError(f"target_points have dimension {dim}, the particles {index.dim}")
     out = torch.empty(nt, dtype=torch.int64, device=points.device)
-    ctx = context(points.device)
+    ctx = context(points.device, index)
     raise_for(lib.mhip_nearest(ctx, index.h, ptr(points), nt, dim, ptr(out)), ctx)
     return out
 

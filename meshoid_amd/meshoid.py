@@ -46,15 +46,14 @@ class Meshoid:
             pos = pos[:, None]
         self.verbose = verbose
         self.N, self.dim = pos.shape
-        if particle_mask is None:
-            self.particle_mask = np.arange(self.N)
-        else:
+        self._mask = self._mask_d = None  # every particle (see particle_mask)
+        if particle_mask is not None:
             pm = particle_mask.cpu().numpy() if isinstance(particle_mask, torch.Tensor) else particle_mask
             if np.array(pm).dtype == np.dtype("bool"):
-                self.particle_mask = np.arange(len(pm))[pm]
+                self._mask = np.arange(len(pm))[pm]
             else:
-                self.particle_mask = np.asarray(pm)
-        self.Nmask = len(self.particle_mask)
+                self._mask = np.asarray(pm)
+        self.Nmask = self.N if self._mask is None else len(self._mask)
         if des_ngb is None:
             des_ngb = {1: 4, 2: 20, 3: 32}[self.dim]
         self.des_ngb = des_ngb
@@ -65,11 +64,13 @@ class Meshoid:
         self._pos_d = as_device(pos)
         self._center = self._L = None
         if m is None:
-            m = np.repeat(1.0, self.N)
-        m = m.cpu().numpy() if isinstance(m, torch.Tensor) else np.asarray(m)
-        self.m = m[self.particle_mask]
-        self._identity_mask = self.Nmask == self.N and np.array_equal(
-            self.particle_mask, np.arange(self.N))
+            self._m = None  # unit masses (see m)
+        else:
+            m = m.cpu().numpy() if isinstance(m, torch.Tensor) else np.asarray(m)
+            self._m = m.copy() if self._mask is None and len(m) == self.N else m[self.particle_mask]
+        self._m_len = self.Nmask
+        self._identity_mask = self._mask is None or (self.Nmask == self.N and np.array_equal(
+            self._mask, np.arange(self.N)))
         self._nl = None
         self._nl_full = None  # the unmasked list of the current tree, kept for masked updates
         self._dev = {}
@@ -86,6 +87,33 @@ class Meshoid:
             self._np["density"] = self.m / self._np["vol"]
 
     # ------------------------------------------------------------------ state
+    # The reference holds the mask and the masses as host arrays.  Here the
+    # defaults (every particle, unit masses) and a mask found on the device
+    # (Reconstruct) become host arrays when a caller asks for them: at 2^22
+    # particles the arrays, their indexed copies and the transfers took 16 ms
+    # of a 27 ms Meshoid(pos).D(f).  Once handed out they are the truth, since
+    # a caller may write to them.
+    @property
+    def particle_mask(self):
+        if self._mask is None:
+            self._mask = np.arange(self.N) if self._mask_d is None else self._mask_d.cpu().numpy()
+            self._mask_d = None
+        return self._mask
+
+    @particle_mask.setter
+    def particle_mask(self, v):
+        self._mask, self._mask_d = v, None
+
+    @property
+    def m(self):
+        if self._m is None:
+            self._m = np.repeat(1.0, self._m_len)
+        return self._m
+
+    @m.setter
+    def m(self, v):
+        self._m = v
+
     def _cached(self, name):
         if name in self._np:
             return self._np[name]
@@ -190,26 +218,29 @@ class Meshoid:
         if self.verbose:
             print("Finding neighbors...")
         dev = self._pos_d.device
-        m_rows = np.asarray(self.m[self.particle_mask], dtype=np.float64)  # Meshoid.py:169
-        m_d = torch.from_numpy(np.ascontiguousarray(m_rows)).to(dev)
-        qidx = None
-        if not self._identity_mask:
-            pm = np.asarray(self.particle_mask, dtype=np.int64)
+        m_d = None  # unit masses
+        if self._m is not None or self._m_len != self.N:
+            m_rows = np.asarray(self.m[self.particle_mask], dtype=np.float64)  # Meshoid.py:169
+            m_d = torch.from_numpy(np.ascontiguousarray(m_rows)).to(dev)
+        qidx = self._mask_d
+        if self._mask is not None and not self._identity_mask:
+            pm = np.asarray(self._mask, dtype=np.int64)
             if pm.size and (pm.min() < -self.N or pm.max() >= self.N):
                 raise IndexError("particle_mask index out of range")
             qidx = torch.from_numpy(np.where(pm < 0, pm + self.N, pm)).to(dev)
+        elif self._mask is not None and len(self._mask) != self.N:
+            raise ValueError("m_rows must have one entry per query row")  # replaced mask, as ever
         full = self._nl_full
         if qidx is not None and full is not None and full.k == self.des_ngb and full.index is self.tree:
             # the rows of the unmasked list are the masked search's result
             if self._nl is full:
                 self._nl = None
-            out = engine.nlist_subset(full, qidx, m_rows=m_d, nlist=self._nl)
+            out = engine.nlist_subset(full, qidx, nlist=self._nl, out={})
         else:
             if qidx is not None and self._nl is full:
                 self._nl = None  # keep the unmasked list intact
             # ngbdist is exported in float64 from the positions: the list keeps no distances
-            out = engine.knn_hsml(self.tree, self.des_ngb, qidx=qidx, m_rows=m_d, keep_dist=False,
-                                  nlist=self._nl)
+            out = engine.knn_hsml(self.tree, self.des_ngb, qidx=qidx, keep_dist=False, nlist=self._nl, out={})
             if qidx is None:
                 self._nl_full = out["nlist"]
         if self.verbose:
@@ -221,9 +252,8 @@ class Meshoid:
             self._np.pop(key, None)
         # float64 h of the final neighbours (HsmlIter's root to ~1e-13), and
         # density and volume from it in float64, as Meshoid.py:165-170
-        h = self._nl.h64()
-        rho = self.des_ngb * m_d / (self.volnorm * h**self.dim)
-        self._dev = {"kernel_radius": h, "density": rho, "vol": m_d / rho, "status": out["status"]}
+        h, rho, vol, status = self._nl.rows64(m_d)
+        self._dev = {"kernel_radius": h, "density": rho, "vol": vol, "status": status}
 
     def get_kernel_weights(self):
         """W(r_ij / h_i) normalised over each row's neighbours
@@ -287,7 +317,9 @@ class Meshoid:
         is_t = isinstance(f, torch.Tensor)
         tail = tuple(f.shape[1:])
         fd = as_device(f)
-        if not self._identity_mask:
+        if self._mask_d is not None:
+            fd = fd[self._mask_d]
+        elif not self._identity_mask:
             fd = fd[torch.as_tensor(self.particle_mask, device=dev)]
         out = engine.integrate(vol.contiguous(), fd.reshape(fd.shape[0], -1).contiguous()).reshape(tail)
         return out if is_t else out.cpu().numpy()
@@ -358,9 +390,10 @@ class Meshoid:
         w = self._weighted.setdefault(order, bool(weighted))
         if self.verbose and order not in self._dw:
             print(f"Computing weights for derivatives of order {order}...")
-        d1, d2, st = engine.apply_D(self._nl, fd, order=order, weighted=w, want_d1=not second,
-                                    want_d2=second)
-        if bool(((st & ST_SINGULAR) != 0).any()):
+        st = torch.empty(1, dtype=torch.int32, device=fd.device)
+        d1, d2, _ = engine.apply_D(self._nl, fd, order=order, weighted=w, want_d1=not second, want_d2=second,
+                                   any_status=st)
+        if int(st) & ST_SINGULAR:
             raise np.linalg.LinAlgError("Matrix is singular to machine precision.")
         return d2 if second else d1
 
@@ -384,10 +417,16 @@ class Meshoid:
         (Nmask, ..., nd2), 3D order [xx, yy, zz, xy, yz, zx]."""
         return self._apply(f, 2, weighted, second=True)
 
+    def _masked_rows(self, v):
+        """v[particle_mask]"""
+        if self._mask is None and self._mask_d is None and len(v) >= self.N:
+            return v[: self.N]
+        return v[self.particle_mask]
+
     def Curl(self, v, correct_sign=False):
         """Curl of a vector field (Meshoid.py:297-315).  The reference's
         component signs are kept unless correct_sign=True."""
-        dv = self.D(v[self.particle_mask])
+        dv = self.D(self._masked_rows(v))
         c = [dv[:, 1, 2] - dv[:, 2, 1], dv[:, 0, 2] - dv[:, 2, 0], dv[:, 0, 1] - dv[:, 1, 0]]
         if correct_sign:
             c = [-c[0], c[1], -c[2]]
@@ -397,14 +436,25 @@ class Meshoid:
 
     def Div(self, v):
         """Divergence of a vector field (Meshoid.py:317-331)."""
-        dv = self.D(v[self.particle_mask])
+        dv = self.D(self._masked_rows(v))
         return dv[:, 0, 0] + dv[:, 1, 1] + dv[:, 2, 2]
 
     # ---------------------------------------------------- reconstruction
     def _set_mask(self, idx):
-        self.particle_mask = idx
-        self.Nmask = len(idx)
-        self._identity_mask = self.Nmask == self.N and np.array_equal(idx, np.arange(self.N))
+        """particle_mask := idx, sorted distinct particles on the device;
+        False when it holds these already."""
+        n = idx.numel()
+        if self._mask is not None:
+            same = len(self._mask) == n and np.array_equal(self._mask, idx.cpu().numpy())
+        elif self._mask_d is not None:
+            same = self._mask_d.numel() == n and bool(torch.equal(self._mask_d, idx))
+        else:
+            same = n == self.N
+        if not same:
+            self._identity_mask = n == self.N
+            self._mask, self._mask_d = None, (None if self._identity_mask else idx)
+            self.Nmask = n
+        return not same
 
     def Reconstruct(self, f, target_points, order: int = 1):
         """Values of f at arbitrary points from each point's nearest particle
@@ -448,9 +498,7 @@ class Meshoid:
         if order not in (1, 2):
             raise ValueError("order must be 0, 1 or 2")
         uniq, inv = engine.unique_inverse(nbr, self.N)
-        u = uniq.cpu().numpy()
-        if not np.array_equal(self.particle_mask, u):
-            self._set_mask(u)
+        if self._set_mask(uniq):
             self.TreeUpdate()  # neighbour lists of just the target neighbours
             self.reset_dweights()
         if not floating:

@@ -69,7 +69,7 @@ class SeedModel:
     def predict(self, index: engine.SpatialIndex) -> torch.Tensor:
         """Predicted smoothing length per particle (original row order)."""
         h = torch.empty(index.n, dtype=torch.float32, device=self.device)
-        ctx = engine.context(self.device)
+        ctx = engine.context(self.device, index)
         raise_for(lib.mhip_seed_predict(ctx, index.h, engine.ptr(self.blob()), engine.ptr(h)), ctx)
         return h
 
@@ -97,7 +97,7 @@ def load_default(k=32, device=None):
 def features(index: engine.SpatialIndex) -> torch.Tensor:
     """Raw features (n, 28) in original row order."""
     F = torch.empty((index.n, NIN), dtype=torch.float32, device=index.pos.device)
-    ctx = engine.context(index.pos.device)
+    ctx = engine.context(index.pos.device, index)
     raise_for(lib.mhip_seed_features(ctx, index.h, engine.ptr(F)), ctx)
     return F
 
