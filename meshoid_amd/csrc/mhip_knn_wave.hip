@@ -560,7 +560,7 @@ __global__ __launch_bounds__(64 * KW_WAVES) void k_knn_wave(KnnArgs a, uint32_t 
 // anyway); k = 100 10^6 3.31 / 2.84, clustered 2^22 16.0 / 13.7.  Few queries
 // in a large set lie far apart and share no leaves.
 bool knn_wave_serves(int64_t n, int64_t nq, int k, int dim, bool per) {
-    if (n >= (int64_t)1 << 30) return false;  // 32-bit byte offsets
+    if (n >= (int64_t)1 << 28) return false;  // 16 threads a query; 32-bit byte offsets
     if (k > 64 || nq < n / 4) return true;
     int64_t most = dim == 3 ? 100000 : 45000;
     if (k > 32) most *= 3;

@@ -10,6 +10,7 @@
 // neighbour list (column-major sorted-space indices) and recompute each pair
 // distance in float64 from the hi + lo positions, which is exact for float32
 // inputs, instead of reading back float32 distances.
+#include <algorithm>
 #include <string>
 
 #include "../../include/meshoid_hip.h"
@@ -17,24 +18,28 @@
 
 namespace mhip {
 
-// W(r/h) / sum_j W(r_j/h) per row of a row-major (nq, k) distance array
+// W(r/h) / sum_j W(r_j/h) per row of a row-major (nq, k) distance array, KWT_LANES
+// lanes per row: a row's distances are read and its weights written in whole
+// lines (one thread per row strode over k lines).  The second pass reads the
+// distances again, from cache.
+constexpr int KWT_LANES = 16;
 template <typename DT, typename HT>
 __global__ __launch_bounds__(256) void k_kernel_weights(const DT *__restrict__ dist, const HT *__restrict__ h,
                                                         int64_t nq, int k, double *__restrict__ w) {
-    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (i >= nq) return;
-    const double ih = 1.0 / (double)h[i];
-    const DT *d = dist + i * k;
-    double *o = w + i * k;
-    double s = 0.0;
-    for (int j = 0; j < k; j++) {
-        const double v = kernel_w<double>((double)d[j] * ih);
-        o[j] = v;
-        s += v;
+    const int g = (int)threadIdx.x % KWT_LANES;
+    const int64_t step = (int64_t)gridDim.x * (256 / KWT_LANES);
+    for (int64_t i = blockIdx.x * (int64_t)(256 / KWT_LANES) + threadIdx.x / KWT_LANES; i < nq; i += step) {
+        const double ih = 1.0 / (double)h[i];
+        const DT *d = dist + i * k;
+        double *o = w + i * k;
+        double s = 0.0;
+        for (int j = g; j < k; j += KWT_LANES) s += kernel_w<double>((double)d[j] * ih);
+#pragma unroll
+        for (int x = KWT_LANES / 2; x > 0; x >>= 1) s += __shfl_xor(s, x);
+        // a row whose kernel sum is zero gives 0/0 = NaN, as the reference does
+        const double is = 1.0 / s;
+        for (int j = g; j < k; j += KWT_LANES) o[j] = kernel_w<double>((double)d[j] * ih) * is;
     }
-    // a row whose kernel sum is zero gives 0/0 = NaN, as the reference does
-    const double is = 1.0 / s;
-    for (int j = 0; j < k; j++) o[j] *= is;
 }
 
 struct KopsArgs {
@@ -149,7 +154,8 @@ int kernel_weights(mhip_ctx *ctx, const void *dist, int dist_f64, const void *h,
                    double *w) {
     if (nq < 0 || k < 1) return fail(ctx, -1, "bad kernel-weight shape");
     if (nq == 0) return 0;
-    const dim3 g((unsigned)((nq + 255) / 256)), b(256);
+    const int64_t rows = 256 / KWT_LANES;  // per block
+    const dim3 g((unsigned)std::min<int64_t>((nq + rows - 1) / rows, 1 << 20)), b(256);
 #define MHIP_KW(DT, HT) \
     hipLaunchKernelGGL((k_kernel_weights<DT, HT>), g, b, 0, ctx->stream, (const DT *)dist, (const HT *)h, nq, k, w)
     if (dist_f64) {
