@@ -580,24 +580,32 @@ static void launch_wave(const KnnArgs &a, bool per, bool p64, int64_t blocks, in
 
 template <int NR>
 static void launch_wave_k(const KnnArgs &a, bool per, bool p64, bool deferred, hipStream_t s) {
-    const int64_t nb = (a.nq + 4 * KW_WAVES - 1) / (4 * KW_WAVES);  // blocks of four slots a wavefront
     if (deferred) {
-        const int64_t nb = (a.nq + WAVE - 1) / WAVE * (WAVE / (4 * KW_WAVES));  // parts of whole wavefronts
         // most of the list on a grid that needs no loop: in an open set it is
-        // short, in a periodic one it holds the wavefronts near the faces
-        const int64_t n1 = std::min<int64_t>(nb, per ? KW_LIST_PER : KW_LIST_OPEN);
+        // short and a query a wavefront ends sooner than four (2^22 clustered
+        // points: 0.135 ms against 0.281), in a periodic one it holds the
+        // wavefronts near the faces
+        const int64_t waves = (a.nq + WAVE - 1) / WAVE;
+        constexpr int64_t P1 = WAVE / KW_WAVES, P4 = P1 / 4;  // blocks per wavefront of the list
         if (a.n >= (int64_t)1 << 30) {
-            launch_wave<NR, 4, KW_LOOP, uint64_t>(a, per, p64, std::min(nb, KW_LIST_OPEN), 0, s);
-            return;
+            launch_wave<NR, 4, KW_LOOP, uint64_t>(a, per, p64, std::min(waves * P4, KW_LIST_OPEN), 0, s);
+        } else if (per) {
+            const int64_t n1 = std::min(waves * P4, KW_LIST_PER);
+            launch_wave<NR, 4, KW_LIST, uint32_t>(a, per, p64, n1, 0, s);
+            if (waves * P4 > n1)
+                launch_wave<NR, 4, KW_LOOP, uint32_t>(a, per, p64, std::min(waves * P4 - n1, KW_LIST_OPEN), n1, s);
+        } else {
+            const int64_t n1 = std::min(waves * P1, 4 * KW_LIST_OPEN);
+            launch_wave<NR, 1, KW_LIST, uint32_t>(a, per, p64, n1, 0, s);
+            if (waves * P1 > n1)
+                launch_wave<NR, 1, KW_LOOP, uint32_t>(a, per, p64, std::min(waves * P1 - n1, KW_LIST_OPEN), n1, s);
         }
-        launch_wave<NR, 4, KW_LIST, uint32_t>(a, per, p64, n1, 0, s);
-        if (nb > n1) launch_wave<NR, 4, KW_LOOP, uint32_t>(a, per, p64, std::min(nb - n1, KW_LIST_OPEN), n1, s);
     } else if (a.nq <= 32768) {
         // one slot per wavefront while there are fewer wavefronts than the
         // chip holds, else four
         launch_wave<NR, 1, KW_ALL, uint32_t>(a, per, p64, (a.nq + KW_WAVES - 1) / KW_WAVES, 0, s);
     } else {
-        launch_wave<NR, 4, KW_ALL, uint32_t>(a, per, p64, nb, 0, s);
+        launch_wave<NR, 4, KW_ALL, uint32_t>(a, per, p64, (a.nq + 4 * KW_WAVES - 1) / (4 * KW_WAVES), 0, s);
     }
 }
 
