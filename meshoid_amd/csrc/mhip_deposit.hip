@@ -23,9 +23,16 @@
 // first cell of their footprint, and each block takes a run of the sorted
 // particles; a brick's run of at least BIN_DENSE particles accumulates in an
 // LDS window (the brick plus the footprint reach above it, 4096 cells) that
-// is added to the HBM map once, shorter runs take float64 atomics in HBM.
-// Particles whose footprint exceeds the window (or BIG_CELLS) go to a kernel
-// that spreads one particle over a whole block.
+// is added to the HBM map once, shorter runs take float64 atomics in HBM.  In
+// the window a footprint below WAVE_CELLS cells is one lane's work and a larger
+// one a wavefront's, a cell per lane.  Footprints wider than the window are
+// deposited tile by tile of the map, again a wavefront each.
+//
+// float64 arithmetic bounds all of it, about 45 vector instructions a cell, 21
+// of them float64.  2^22 clustered particles, radii of 32 neighbours: the
+// 1024^2 map 9.8 -> 2.6 ms (windows 2.25 -> 0.64, wide footprints 7.16 -> 1.77:
+// one block per particle ran at the rate of float64 atomics in L2), the 128^3
+// volume 4.3 -> 1.1 ms.
 #include "mhip_internal.hpp"
 
 namespace mhip {
@@ -36,22 +43,36 @@ constexpr int DEP_TILE = 128;                 // map side held whole in LDS (128
 constexpr double KERNEL2D_NORM = 1.8189136353359467;  // 40 / (7 pi)
 
 // binned deposition
-constexpr int BIN_CHUNK = 2048;   // sorted particles per block
-constexpr int BIN_DENSE = 32;     // a brick's run of this many particles in a block uses the window
+// sorted particles per block: a block of large footprints is the launch's tail
+// (2048 a block: 1.5 and 1.6 ms for map and volume, 512: 0.70 and 1.07, 256:
+// 0.64 and 0.90)
+constexpr int BIN_CHUNK = 256;
+// a brick's run of this many particles in a block uses the window (64, 32, 16:
+// 1.15, 1.13, 1.11 ms of the volume)
+constexpr int BIN_DENSE = 16;
 constexpr int WIN_CELLS = 4096;   // LDS window, float64 cells (32 KB)
 constexpr int BRICK2 = 32, WIN2 = 64;  // maps: brick side, window side (footprint span <= 33)
 constexpr int BRICK3 = 8, WIN3 = 16;   // volumes: brick side, window side (span <= 9)
 static_assert(WIN2 * WIN2 == WIN_CELLS && WIN3 * WIN3 * WIN3 == WIN_CELLS, "window size");
-static_assert(BIN_CHUNK <= 65535, "run offsets and lengths are packed in 16 bits");
-// sort keys: brick << SIZE_BITS | (SIZE_MAX_RANK - footprint cells), so a
-// brick's particles come largest footprint first and a wavefront's 64
-// footprints are alike (its lanes finish together)
-constexpr int SIZE_BITS = 11;
-// conservative footprints up to this many cells keep their weights in
-// registers between the total and the deposit (the window kernel is limited
-// to 3 waves per SIMD by its LDS, so the registers cost no occupancy)
-constexpr int WCACHE2 = 25, WCACHE3 = 27;
+// sort keys: brick << SIZE_BITS | (SIZE_MAX_RANK - min(footprint cells,
+// SIZE_MAX_RANK)), so a brick's particles come widest first and the small
+// ones in order: a wavefront's 64 lanes finish together (from WAVE_CELLS on
+// the order no longer matters)
+constexpr int SIZE_BITS = 6;
 constexpr uint32_t SIZE_MAX_RANK = (1u << SIZE_BITS) - 1;
+// conservative footprints up to this many cells (4^2, 2^3: the narrowest, h of
+// two spacings on a map and one in a volume) keep their weights in registers
+// between the total and the deposit; at 27 cells the registers halved the
+// wavefronts in flight (volume 1.24 ms against 1.16)
+constexpr int WCACHE2 = 16, WCACHE3 = 8;
+// in the window, footprints of at least this many cells are deposited by a
+// whole wavefront, a cell per lane (up to WAVE_CACHE turns of it keep their
+// weights in registers); smaller ones by one lane each.  By one lane all, a
+// background particle's ~340 cells kept a few lanes of one block busy at the end
+// (volume 3.5 ms against 1.9); 32 and 64 measure alike.
+constexpr int WAVE_CELLS = 64;
+constexpr int WAVE_CACHE = 8;
+static_assert(WAVE_CELLS <= SIZE_MAX_RANK + 1, "footprints one lane deposits are told apart by size");
 
 struct DepArgs {
     const void *f, *pos, *h;
@@ -62,19 +83,25 @@ struct DepArgs {
     double dx;            // size / (res - 1)
     int res, conservative;
     double *grid;           // (res, res), [gx][gy]
-    uint32_t *big, *nbig;   // particles left to the block-per-particle kernel
+    uint32_t *big, *nbig;   // wide particles and their number (whole-map path)
     int nb;                 // bricks per axis (binned path)
 };
 
-MHIP_DEV double kernel2d(double q) {
-    double k;
-    if (q <= 0.5) {
-        k = 1.0 - 6.0 * q * q * (1.0 - q);
-    } else {
-        const double a = 1.0 - q;
-        k = 2.0 * a * a * a;
-    }
-    return k * KERNEL2D_NORM;
+// The cubic spline of r^2 at 1/h: 2 (1-q)_+^3 - (1-2q)_+^3, q = r / h, the same
+// function as its two branches (and 0 beyond q = 1) without them; r from the
+// reciprocal square root and one Newton step (a correctly rounded root gives
+// the same errors of the maps).  18 float64 instructions, where sqrt's own
+// expansion and both branches took about 40; r^2 below 1e-300 counts as 1e-300
+// (q = 0 to rounding).  Offsets and r^2 are rounded as the reference rounds
+// them: where a footprint's few points all lie near r = h, 1 - q multiplies a
+// last-place difference by ten.
+MHIP_DEV double spline_r2(double r2, double hinv) {
+    r2 = fmax(r2, 1e-300);
+    const double y = __builtin_amdgcn_rsq(r2);
+    double r = r2 * y;
+    r = fma(0.5 * y, fma(-r, r, r2), r);
+    const double q = r * hinv, a = fmax(1.0 - q, 0.0), b = fmax(fma(-2.0, q, 1.0), 0.0);
+    return fma(a + a, a * a, -(b * b * b));
 }
 
 template <typename T>
@@ -83,7 +110,7 @@ MHIP_DEV double ld(const void *p, int64_t i) {
 }
 
 struct Foot {
-    double xs0, xs1, hs, hinv, w;  // projected position, h, 1/h, per-weight factor
+    double xs0, xs1, hinv, w;  // projected position, 1/h, factor of the spline's value
     int gx0, gx1, gy0, gy1;
 };
 
@@ -109,9 +136,9 @@ MHIP_DEV bool footprint(const DepArgs &a, int64_t i, Foot &fp) {
     double hs = fmin(fmax(a.smooth * hv, a.hmin), 1e100);
     if (a.conservative) hs = fmax(hs, a.dx);
     if (!(hs > 0.0) || !isfinite(fp.xs0) || !isfinite(fp.xs1) || !isfinite(fv)) return false;
-    fp.hs = hs;
     fp.hinv = 1.0 / hs;
-    fp.w = a.conservative ? fv : fv * fp.hinv * fp.hinv;
+    // conservative: shares of f, in which the kernel's constant cancels
+    fp.w = a.conservative ? fv : KERNEL2D_NORM * (fv * fp.hinv * fp.hinv);
     fp.gx0 = lo_index((fp.xs0 - hs) / a.dx + 1.0, a.res);
     fp.gx1 = hi_index((fp.xs0 + hs) / a.dx, a.res);
     fp.gy0 = lo_index((fp.xs1 - hs) / a.dx + 1.0, a.res);
@@ -119,15 +146,162 @@ MHIP_DEV bool footprint(const DepArgs &a, int64_t i, Foot &fp) {
     return fp.gx0 <= fp.gx1 && fp.gy0 <= fp.gy1;
 }
 
-// kernel weight at grid point (gx, gy), 0 when it lies beyond h
+// offset of grid line g from the particle, per axis
+MHIP_DEV double line_off(double xs, int g, double dx) { return xs - g * dx; }
+
+// kernel weight at grid point (gx, gy) without the kernel's constant, 0 when
+// it lies beyond h
 MHIP_DEV double cell_weight(const DepArgs &a, const Foot &fp, int gx, int gy) {
-    double ddx = fp.xs0 - gx * a.dx;
-    ddx *= ddx;
-    double ddy = fp.xs1 - gy * a.dx;
-    ddy *= ddy;
-    const double r = sqrt(ddx + ddy);
-    if (r > fp.hs) return 0.0;
-    return kernel2d(r * fp.hinv);
+    const double x = line_off(fp.xs0, gx, a.dx), y = line_off(fp.xs1, gy, a.dx);
+    return spline_r2(x * x + y * y, fp.hinv);
+}
+
+// visit(gx, gy, weight) over the cells [gx0, gx1] x [gy0, gy1]
+template <typename F>
+MHIP_DEV void each_cell(const DepArgs &a, const Foot &fp, int gx0, int gx1, int gy0, int gy1, F visit) {
+    for (int gx = gx0; gx <= gx1; gx++)
+        for (int gy = gy0; gy <= gy1; gy++) visit(gx, gy, cell_weight(a, fp, gx, gy));
+}
+
+// conservative variant: the particle's total weight over its (clipped)
+// footprint, by which each weight is divided; 1 for the plain variant
+MHIP_DEV double foot_total(const DepArgs &a, const Foot &fp) {
+    if (!a.conservative) return 1.0;
+    double tot = 0.0;
+    each_cell(a, fp, fp.gx0, fp.gx1, fp.gy0, fp.gy1, [&](int, int, double k) { tot += k; });
+    return tot;
+}
+
+// lane l's value of v in every lane (l uniform)
+MHIP_DEV int lane_value(int v, int l) { return __builtin_amdgcn_readlane(v, l); }
+MHIP_DEV double lane_value(double v, int l) {
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, l);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), l);
+    return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+MHIP_DEV Foot lane_foot(const Foot &f, int l) {
+    Foot r;
+    r.xs0 = lane_value(f.xs0, l);
+    r.xs1 = lane_value(f.xs1, l);
+    r.hinv = lane_value(f.hinv, l);
+    r.w = lane_value(f.w, l);
+    r.gx0 = lane_value(f.gx0, l);
+    r.gx1 = lane_value(f.gx1, l);
+    r.gy0 = lane_value(f.gy0, l);
+    r.gy1 = lane_value(f.gy1, l);
+    return r;
+}
+
+MHIP_DEV double wave_sum(double v) {
+    for (int o = WAVE / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, WAVE);
+    return v;
+}
+
+// The walk of `stride` lanes (a wavefront, a block) over a box of cells, a cell
+// per lane in row-major order: lane l starts at cell l and moves on by `stride`
+// cells at a time, rows and planes by carries (one division per box, where a
+// division per cell would cost more than the weight).
+struct Walk2 {
+    int x, y;  // the lane's cell
+    int sx, sy, wy, x1, y1;
+    MHIP_DEV void start(int lane, int stride, int x0, int y0, int x1_, int y1_) {
+        x1 = x1_;
+        y1 = y1_;
+        wy = y1 - y0 + 1;
+        const int row = lane / wy;
+        sx = stride / wy;
+        sy = stride - sx * wy;
+        x = x0 + row;
+        y = y0 + (lane - row * wy);
+    }
+    MHIP_DEV bool inside() const { return x <= x1; }
+    MHIP_DEV void next() {
+        x += sx;
+        y += sy;
+        if (y > y1) {
+            y -= wy;
+            x++;
+        }
+    }
+};
+
+struct Walk3 {
+    int x, y, z;
+    int sx, sy, sz, wy, wz, x1, y1, z1;
+    MHIP_DEV void start(int lane, int stride, const int *lo, const int *hi) {
+        x1 = hi[0];
+        y1 = hi[1];
+        z1 = hi[2];
+        wy = y1 - lo[1] + 1;
+        wz = z1 - lo[2] + 1;
+        const int row = lane / wz, srow = stride / wz, plane = row / wy;
+        sz = stride - srow * wz;
+        sx = srow / wy;
+        sy = srow - sx * wy;
+        x = lo[0] + plane;
+        y = lo[1] + (row - plane * wy);
+        z = lo[2] + (lane - row * wz);
+    }
+    MHIP_DEV bool inside() const { return x <= x1; }
+    MHIP_DEV void next() {
+        x += sx;
+        y += sy;
+        z += sz;
+        if (z > z1) {
+            z -= wz;
+            y++;
+        }
+        if (y > y1) {
+            y -= wy;
+            x++;
+        }
+    }
+};
+
+// The cells of one particle by a whole wavefront: weight(walk) is the weight
+// of the lane's present cell, add(walk, share) deposits its share.
+// Conservative shares are weight / (sum of the weights), plain ones the weight.
+template <typename Walk, typename W, typename A>
+MHIP_DEV void wave_spread(const Walk &w0, int ncell, bool conservative, W weight, A add) {
+    if (!conservative) {
+        for (Walk w = w0; w.inside(); w.next()) {
+            const double k = weight(w);
+            if (k != 0.0) add(w, k);
+        }
+    } else if (ncell <= WAVE * WAVE_CACHE) {
+        double wc[WAVE_CACHE], tot = 0.0;
+        Walk w = w0;
+#pragma unroll
+        for (int t = 0; t < WAVE_CACHE; t++) {
+            wc[t] = 0.0;
+            if (t * WAVE < ncell) {
+                if (w.inside()) wc[t] = weight(w);
+                tot += wc[t];
+                w.next();
+            }
+        }
+        tot = wave_sum(tot);
+        if (!(tot > 0.0)) return;
+        const double inv = 1.0 / tot;
+        w = w0;
+#pragma unroll
+        for (int t = 0; t < WAVE_CACHE; t++)
+            if (t * WAVE < ncell) {
+                if (wc[t] != 0.0) add(w, wc[t] * inv);
+                w.next();
+            }
+    } else {
+        double tot = 0.0;
+        for (Walk w = w0; w.inside(); w.next()) tot += weight(w);
+        tot = wave_sum(tot);
+        if (!(tot > 0.0)) return;
+        const double inv = 1.0 / tot;
+        for (Walk w = w0; w.inside(); w.next()) {
+            const double k = weight(w);
+            if (k != 0.0) add(w, k * inv);
+        }
+    }
 }
 
 // block b: map tile (b % ntile) (tw x tw cells held in LDS) and particle
@@ -174,12 +348,13 @@ __global__ __launch_bounds__(DEP_THREADS) void k_deposit_tiles(DepArgs a, int tw
                 }
             }
             if (tot == 0.0) continue;
+            const double inv = 1.0 / tot;
             gx = fp.gx0;
             gy = fp.gy0;
 #pragma unroll
             for (int c = 0; c < WCACHE2; c++) {
                 if (c < cells) {
-                    if (wc[c] != 0.0) atomicAdd(&sg[(gx - tx0) * tw + (gy - ty0)], wc[c] * fp.w / tot);
+                    if (wc[c] != 0.0) atomicAdd(&sg[(gx - tx0) * tw + (gy - ty0)], wc[c] * inv * fp.w);
                     if (++gy > fp.gy1) {
                         gy = fp.gy0;
                         gx++;
@@ -195,16 +370,13 @@ __global__ __launch_bounds__(DEP_THREADS) void k_deposit_tiles(DepArgs a, int tw
         // whole footprint, not only this tile's part)
         double tot = 1.0;
         if (a.conservative) {
-            tot = 0.0;
-            for (int gx = fp.gx0; gx <= fp.gx1; gx++)
-                for (int gy = fp.gy0; gy <= fp.gy1; gy++) tot += cell_weight(a, fp, gx, gy);
+            tot = foot_total(a, fp);
             if (tot == 0.0) continue;
         }
-        for (int gx = gx0; gx <= gx1; gx++)
-            for (int gy = gy0; gy <= gy1; gy++) {
-                const double k = cell_weight(a, fp, gx, gy);
-                if (k != 0.0) atomicAdd(&sg[(gx - tx0) * tw + (gy - ty0)], a.conservative ? k * fp.w / tot : k * fp.w);
-            }
+        const double inv = 1.0 / tot;
+        each_cell(a, fp, gx0, gx1, gy0, gy1, [&](int gx, int gy, double k) {
+            if (k != 0.0) atomicAdd(&sg[(gx - tx0) * tw + (gy - ty0)], k * inv * fp.w);
+        });
     }
     __syncthreads();
     for (int c = threadIdx.x; c < tw * tw; c += DEP_THREADS) {
@@ -213,24 +385,16 @@ __global__ __launch_bounds__(DEP_THREADS) void k_deposit_tiles(DepArgs a, int tw
     }
 }
 
-// conservative variant: the particle's total weight over its (clipped)
-// footprint, by which each weight is divided; 1 for the plain variant
-MHIP_DEV double foot_total(const DepArgs &a, const Foot &fp) {
-    if (!a.conservative) return 1.0;
-    double tot = 0.0;
-    for (int gx = fp.gx0; gx <= fp.gx1; gx++)
-        for (int gy = fp.gy0; gy <= fp.gy1; gy++) tot += cell_weight(a, fp, gx, gy);
-    return tot;
-}
-
 // ---------------------------------------------------------------------------
 // Binned deposition.  A policy P gives, for its kind of grid:
 //   key(a, i, cells)     the brick of particle i's first footprint cell (and
-//                        the footprint's cells), or skip(a) when it has
-//                        nothing to deposit here (no footprint, or listed for
-//                        the block-per-particle kernel)
+//                        the footprint's cells); skip(a) + that brick when the
+//                        footprint is too large for the window (it goes to the
+//                        tiles below), 2 skip(a) when there is none
 //   direct(a, i)         deposit particle i with float64 atomics in HBM
-//   window(a, i, k, w)   deposit particle i (brick k) into the LDS window w
+//   foot(a, i, fp), cells(fp)   particle i's footprint and its cells
+//   window(a, fp, k, w)  deposit a particle (brick k) into the LDS window w
+//   window_wave(a, fp, l, k, w)   the same for lane l's, by the wavefront
 //   flush(a, k, c, v)    add window cell c of brick k (value v) to the map
 // ---------------------------------------------------------------------------
 struct Map2 {
@@ -239,79 +403,140 @@ struct Map2 {
     static MHIP_DEV uint32_t key(const DepArgs &a, int64_t i, uint32_t &cells) {
         Foot fp;
         cells = 0;
-        if (!footprint(a, i, fp)) return skip(a);
+        if (!footprint(a, i, fp)) return 2 * skip(a);
+        const uint32_t brick = (uint32_t)(fp.gx0 / BRICK2) * (uint32_t)a.nb + (uint32_t)(fp.gy0 / BRICK2);
         const int sx = fp.gx1 - fp.gx0 + 1, sy = fp.gy1 - fp.gy0 + 1;
         if (sx > WIN2 - BRICK2 + 1 || sy > WIN2 - BRICK2 + 1 || (int64_t)sx * sy > BIG_CELLS) {
-            a.big[atomicAdd(a.nbig, 1u)] = (uint32_t)i;
-            return skip(a);
+            cells = SIZE_MAX_RANK;
+            return skip(a) + brick;
         }
         cells = (uint32_t)(sx * sy);
-        return (uint32_t)(fp.gx0 / BRICK2) * (uint32_t)a.nb + (uint32_t)(fp.gy0 / BRICK2);
+        return brick;
     }
     static MHIP_DEV void direct(const DepArgs &a, uint32_t i) {
         Foot fp;
         footprint(a, i, fp);  // keyed, so it has a footprint
         const double tot = foot_total(a, fp);
         if (tot == 0.0) return;
-        for (int gx = fp.gx0; gx <= fp.gx1; gx++)
-            for (int gy = fp.gy0; gy <= fp.gy1; gy++) {
-                const double k = cell_weight(a, fp, gx, gy);
-                if (k != 0.0) atomicAdd(&a.grid[(int64_t)gx * a.res + gy], a.conservative ? k * fp.w / tot : k * fp.w);
-            }
+        const double inv = 1.0 / tot;
+        each_cell(a, fp, fp.gx0, fp.gx1, fp.gy0, fp.gy1, [&](int gx, int gy, double k) {
+            if (k != 0.0) atomicAdd(&a.grid[(int64_t)gx * a.res + gy], k * inv * fp.w);
+        });
     }
     // the window holds cells [ox, ox + 64) x [oy, oy + 64) of the brick's
     // origin (ox, oy); a keyed footprint starts inside the brick and spans at
-    // most 33 cells per axis, so it stays inside
-    static MHIP_DEV void window(const DepArgs &a, uint32_t i, uint32_t key, double *win) {
-        Foot fp;
-        footprint(a, i, fp);
+    // most 33 cells per axis, so it stays inside.  A lane goes round its
+    // footprint from a cell of its own: the particles of a clump, stored
+    // together, cover the same few cells, and lanes in step would add to one
+    // address 64 at a time.
+    using F = Foot;
+    static MHIP_DEV bool foot(const DepArgs &a, uint32_t i, F &fp) { return footprint(a, i, fp); }
+    static MHIP_DEV int cells(const F &fp) { return (fp.gx1 - fp.gx0 + 1) * (fp.gy1 - fp.gy0 + 1); }
+    // lane l's particle, by the whole wavefront
+    static MHIP_DEV void window_wave(const DepArgs &a, const F &mine, int l, uint32_t key, double *win) {
+        const F fp = lane_foot(mine, l);
         const int ox = (int)(key / (uint32_t)a.nb) * BRICK2, oy = (int)(key % (uint32_t)a.nb) * BRICK2;
-        const int wy = fp.gy1 - fp.gy0 + 1, ncell = (fp.gx1 - fp.gx0 + 1) * wy;
+        const int origin = ox * WIN2 + oy;
+        Walk2 w;
+        w.start(threadIdx.x % WAVE, WAVE, fp.gx0, fp.gy0, fp.gx1, fp.gy1);
+        wave_spread(
+            w, cells(fp), a.conservative != 0, [&](const Walk2 &c) { return cell_weight(a, fp, c.x, c.y); },
+            [&](const Walk2 &c, double k) { atomicAdd(&win[c.x * WIN2 + c.y - origin], k * fp.w); });
+    }
+    static MHIP_DEV void window(const DepArgs &a, const F &fp, uint32_t key, double *win) {
+        const int ox = (int)(key / (uint32_t)a.nb) * BRICK2, oy = (int)(key % (uint32_t)a.nb) * BRICK2;
+        const int wx = fp.gx1 - fp.gx0 + 1, wy = fp.gy1 - fp.gy0 + 1, ncell = wx * wy;
+        const uint32_t lane = threadIdx.x % WAVE;
+        const int gxs = fp.gx0 + (int)(lane / (uint32_t)wy % (uint32_t)wx), gys = fp.gy0 + (int)(lane % (uint32_t)wy);
+        int gx = gxs, gy = gys;
+        auto next = [&]() {
+            if (++gy > fp.gy1) {
+                gy = fp.gy0;
+                if (++gx > fp.gx1) gx = fp.gx0;
+            }
+        };
         if (a.conservative && ncell <= WCACHE2) {
             // small footprints: the weights stay in registers between the
-            // total (summed in foot_total's order) and the deposit
+            // total and the deposit
             double wc[WCACHE2];
             double tot = 0.0;
-            int gx = fp.gx0, gy = fp.gy0;
 #pragma unroll
             for (int c = 0; c < WCACHE2; c++) {
                 wc[c] = 0.0;
                 if (c < ncell) {
                     wc[c] = cell_weight(a, fp, gx, gy);
                     tot += wc[c];
-                    if (++gy > fp.gy1) {
-                        gy = fp.gy0;
-                        gx++;
-                    }
+                    next();
                 }
             }
             if (tot == 0.0) return;
-            gx = fp.gx0;
-            gy = fp.gy0;
+            const double inv = 1.0 / tot;
+            gx = gxs;
+            gy = gys;
 #pragma unroll
             for (int c = 0; c < WCACHE2; c++) {
                 if (c < ncell) {
-                    if (wc[c] != 0.0) atomicAdd(&win[(gx - ox) * WIN2 + (gy - oy)], wc[c] * fp.w / tot);
-                    if (++gy > fp.gy1) {
-                        gy = fp.gy0;
-                        gx++;
-                    }
+                    if (wc[c] != 0.0) atomicAdd(&win[(gx - ox) * WIN2 + (gy - oy)], wc[c] * inv * fp.w);
+                    next();
                 }
             }
             return;
         }
         const double tot = foot_total(a, fp);
         if (tot == 0.0) return;
-        for (int gx = fp.gx0; gx <= fp.gx1; gx++)
-            for (int gy = fp.gy0; gy <= fp.gy1; gy++) {
-                const double k = cell_weight(a, fp, gx, gy);
-                if (k != 0.0) atomicAdd(&win[(gx - ox) * WIN2 + (gy - oy)], a.conservative ? k * fp.w / tot : k * fp.w);
-            }
+        const double inv = 1.0 / tot;
+        for (int c = 0; c < ncell; c++) {
+            const double k = cell_weight(a, fp, gx, gy);
+            if (k != 0.0) atomicAdd(&win[(gx - ox) * WIN2 + (gy - oy)], k * inv * fp.w);
+            next();
+        }
     }
     static MHIP_DEV void flush(const DepArgs &a, uint32_t key, int c, double v) {
         const int gx = (int)(key / (uint32_t)a.nb) * BRICK2 + c / WIN2;
         const int gy = (int)(key % (uint32_t)a.nb) * BRICK2 + c % WIN2;
         if (gx < a.res && gy < a.res) atomicAdd(&a.grid[(int64_t)gx * a.res + gy], v);
+    }
+
+    // ---- tiles of WIN2^2 cells
+    static constexpr int SIDE = WIN2;
+    static MHIP_DEV void box(const F &fp, int *lo, int *hi) {
+        lo[0] = fp.gx0;
+        hi[0] = fp.gx1;
+        lo[1] = fp.gy0;
+        hi[1] = fp.gy1;
+        lo[2] = hi[2] = 0;
+    }
+    static MHIP_DEV void corner(int64_t tile, int nt, int *t0) {
+        t0[0] = (int)(tile / nt) * SIDE;
+        t0[1] = (int)(tile % nt) * SIDE;
+        t0[2] = 0;
+    }
+    static MHIP_DEV bool meets(const DepArgs &, const int *lo, const int *hi, const int *t0) {
+        return lo[0] < t0[0] + SIDE && hi[0] >= t0[0] && lo[1] < t0[1] + SIDE && hi[1] >= t0[1];
+    }
+    // this thread's share (of `stride`) of the sum of the weights
+    static MHIP_DEV double total(const DepArgs &a, const F &fp, int thread, int stride) {
+        Walk2 w;
+        double tot = 0.0;
+        for (w.start(thread, stride, fp.gx0, fp.gy0, fp.gx1, fp.gy1); w.inside(); w.next())
+            tot += cell_weight(a, fp, w.x, w.y);
+        return tot;
+    }
+    static MHIP_DEV void tile_wave(const DepArgs &a, const F &mine, double inv, int l, const int *t0, double *win) {
+        const F fp = lane_foot(mine, l);
+        const double f = a.conservative ? fp.w * lane_value(inv, l) : fp.w;
+        const int origin = t0[0] * SIDE + t0[1];
+        Walk2 w;
+        w.start(threadIdx.x % WAVE, WAVE, max(fp.gx0, t0[0]), max(fp.gy0, t0[1]), min(fp.gx1, t0[0] + SIDE - 1),
+                min(fp.gy1, t0[1] + SIDE - 1));
+        for (; w.inside(); w.next()) {
+            const double k = cell_weight(a, fp, w.x, w.y);
+            if (k != 0.0) atomicAdd(&win[w.x * SIDE + w.y - origin], k * f);
+        }
+    }
+    static MHIP_DEV void tile_flush(const DepArgs &a, const int *t0, int c, double v) {
+        const int gx = t0[0] + c / SIDE, gy = t0[1] + c % SIDE;
+        atomicAdd(&a.grid[(int64_t)gx * a.res + gy], v);
     }
 };
 
@@ -371,7 +596,7 @@ __global__ __launch_bounds__(DEP_THREADS) void k_bin_deposit(typename P::Args a,
     __syncthreads();
     for (int e = threadIdx.x; e < m; e += DEP_THREADS) {
         const uint32_t k = skey[e];
-        if (k == skip) continue;
+        if (k >= skip) break;  // the rest is wider than a window, or nothing
         const int lo = first_not_below(skey, m, k), hi = first_above(skey, m, k);
         if (hi - lo >= BIN_DENSE) {
             // at most BIN_CHUNK / BIN_DENSE runs this long
@@ -385,7 +610,18 @@ __global__ __launch_bounds__(DEP_THREADS) void k_bin_deposit(typename P::Args a,
     for (uint32_t r = 0; r < nrun; r++) {
         const int lo = (int)(runs[r] & 0xffffu), len = (int)(runs[r] >> 16);
         const uint32_t k = skey[lo];
-        for (int e = threadIdx.x; e < len; e += DEP_THREADS) P::window(a, vals[cs + lo + e], k, win);
+        // lane l of wavefront w: particle 4 l + w of each 256 (a brick's
+        // particles come largest first, so the four share the large ones)
+        const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
+        for (int b = 0; b < len; b += DEP_THREADS) {
+            const int e = b + lane * (DEP_THREADS / WAVE) + wave;
+            typename P::F fp;
+            const bool has = e < len && P::foot(a, vals[cs + lo + e], fp);
+            const bool wide = has && P::cells(fp) >= WAVE_CELLS;
+            for (uint64_t todo = __ballot(wide); todo; todo &= todo - 1)
+                P::window_wave(a, fp, __builtin_ctzll(todo), k, win);
+            if (has && !wide) P::window(a, fp, k, win);
+        }
         __syncthreads();
         for (int c = threadIdx.x; c < WIN_CELLS; c += DEP_THREADS) {
             const double v = win[c];
@@ -398,63 +634,205 @@ __global__ __launch_bounds__(DEP_THREADS) void k_bin_deposit(typename P::Args a,
     }
 }
 
-// bits of a sort key in [0, skip]
-static int key_bits(uint32_t skip) { return 64 - __builtin_clzll((unsigned long long)skip | 1ull); }
+// ---------------------------------------------------------------------------
+// Footprints wider than a window.  The grid is cut into tiles of SIDE^dim =
+// 4096 cells held in LDS; a block goes over its share of the wide particles,
+// keeps those that meet its tile and deposits, a wavefront per particle and a
+// cell per lane, the cells inside.  Tile and particle meet by tests on boxes
+// of cells, 64 groups of 64 particles at once and then the particles of a
+// group, so no list of pairs is made; the particles are in brick order, so a
+// group's box is little larger than one footprint.
+// One block per particle adding each cell to HBM ran at the rate of float64
+// atomics in L2, 1.1e11 a second; here they stay in LDS and each tile is added
+// once per block.
+// ---------------------------------------------------------------------------
+struct Wide {
+    const uint32_t *list;  // the particles, count of them from list[range[0]]
+    uint32_t *range;       // first, count
+    int *boxes;            // (groups, 6): lowest and highest cell on each axis
+    double *inv;           // 1 / total weight by place in the list; null: plain shares
+};
 
-// the binned path: keys, sort, runs; the block-per-particle list in big/nbig
-// (cleared beforehand).  Scratch: keys 16 n, values 8 n, radix counts.
+// first of the sorted keys (brick << SIZE_BITS | size) with brick >= k, by a
+// wavefront: 64 splits of the range at a time
+MHIP_DEV int64_t wave_lower_bound(const uint64_t *__restrict__ keys, int64_t n, uint32_t k) {
+    const int lane = threadIdx.x % WAVE;
+    int64_t lo = 0, hi = n;  // the answer is in [lo, hi]
+    while (lo < hi) {
+        const int64_t step = (hi - lo + WAVE - 1) / WAVE;
+        const int64_t p = lo + lane * step;
+        const int below = __popcll(__ballot(p < hi && (uint32_t)(keys[p] >> SIZE_BITS) < k));
+        if (below == 0) return lo;
+        const int64_t last = lo + (below - 1) * step;  // below k
+        hi = min(hi, last + step);
+        lo = last + 1;
+    }
+    return lo;
+}
+
+__global__ __launch_bounds__(WAVE) void k_wide_range(const uint64_t *__restrict__ keys, int64_t n, uint32_t skip,
+                                                     uint32_t *__restrict__ range) {
+    const int64_t lo = wave_lower_bound(keys, n, skip), hi = wave_lower_bound(keys, n, 2 * skip);
+    if (threadIdx.x == 0) {
+        range[0] = (uint32_t)lo;
+        range[1] = (uint32_t)(hi - lo);
+    }
+}
+
+MHIP_DEV int wave_min_i(int v) {
+    for (int o = WAVE / 2; o > 0; o >>= 1) v = min(v, __shfl_xor(v, o, WAVE));
+    return v;
+}
+MHIP_DEV int wave_max_i(int v) {
+    for (int o = WAVE / 2; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o, WAVE));
+    return v;
+}
+
+// the groups' boxes, a wavefront per group
 template <class P>
-int bin_deposit(mhip_ctx *ctx, typename P::Args a, uint32_t skip, char *sc) {
+__global__ __launch_bounds__(DEP_THREADS) void k_wide_boxes(typename P::Args a, Wide wd) {
+    const uint32_t first = wd.range[0], count = wd.range[1];
+    const int lane = threadIdx.x % WAVE;
+    const uint32_t ng = (uint32_t)(((uint64_t)count + WAVE - 1) / WAVE);
+    const uint32_t stride = gridDim.x * (DEP_THREADS / WAVE);
+    for (uint32_t g = blockIdx.x * (DEP_THREADS / WAVE) + threadIdx.x / WAVE; g < ng; g += stride) {
+        const int64_t e = (int64_t)g * WAVE + lane;
+        typename P::F fp;
+        int lo[3] = {INT32_MAX, INT32_MAX, INT32_MAX}, hi[3] = {INT32_MIN, INT32_MIN, INT32_MIN};
+        if (e < count && P::foot(a, wd.list[first + e], fp)) P::box(fp, lo, hi);
+        for (int c = 0; c < 3; c++) {
+            const int l = wave_min_i(lo[c]), h = wave_max_i(hi[c]);
+            if (lane == 0) {
+                wd.boxes[(size_t)g * 6 + c] = l;
+                wd.boxes[(size_t)g * 6 + 3 + c] = h;
+            }
+        }
+    }
+}
+
+// conservative: 1 / (sum of the weights), a block per particle
+template <class P>
+__global__ __launch_bounds__(DEP_THREADS) void k_wide_totals(typename P::Args a, Wide wd) {
+    __shared__ double part[DEP_THREADS / WAVE];
+    const uint32_t first = wd.range[0], count = wd.range[1];
+    for (uint32_t e = blockIdx.x; e < count; e += gridDim.x) {
+        typename P::F fp;
+        P::foot(a, wd.list[first + e], fp);  // listed, so it has a footprint
+        const double p = wave_sum(P::total(a, fp, threadIdx.x, DEP_THREADS));
+        if (threadIdx.x % WAVE == 0) part[threadIdx.x / WAVE] = p;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            double tot = 0.0;
+            for (int w = 0; w < DEP_THREADS / WAVE; w++) tot += part[w];
+            wd.inv[e] = tot > 0.0 ? 1.0 / tot : 0.0;
+        }
+        __syncthreads();
+    }
+}
+
+// block b: tile b % ntile, groups b / ntile, + nslice, ... of the wide
+// particles (neighbouring groups meet the same tiles, so each of a tile's
+// blocks gets its share of them).  The block's four wavefronts go over the
+// same groups and take every fourth particle.
+template <class P>
+__global__ __launch_bounds__(DEP_THREADS) void k_wide_tiles(typename P::Args a, Wide wd, int nt, int64_t ntile,
+                                                            int nslice) {
+    __shared__ double win[WIN_CELLS];
+    const uint32_t first = wd.range[0], count = wd.range[1];
+    const int64_t ng = ((int64_t)count + WAVE - 1) / WAVE;
+    const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
+    for (int64_t b = blockIdx.x; b < ntile * nslice; b += gridDim.x) {
+        const int slice = (int)(b / ntile);
+        int t0[3];
+        P::corner(b % ntile, nt, t0);
+        bool any = false;
+        for (int64_t g = slice + (int64_t)nslice * threadIdx.x; g < ng && !any; g += (int64_t)nslice * DEP_THREADS)
+            any = P::meets(a, wd.boxes + g * 6, wd.boxes + g * 6 + 3, t0);
+        if (!__syncthreads_or(any)) continue;
+        for (int c = threadIdx.x; c < WIN_CELLS; c += DEP_THREADS) win[c] = 0.0;
+        __syncthreads();
+        for (int64_t g0 = slice; g0 < ng; g0 += (int64_t)nslice * WAVE) {
+            const int64_t g = g0 + (int64_t)nslice * lane;
+            const bool near = g < ng && P::meets(a, wd.boxes + g * 6, wd.boxes + g * 6 + 3, t0);
+            for (uint64_t gs = __ballot(near); gs; gs &= gs - 1) {
+                const int64_t e = (g0 + (int64_t)nslice * __builtin_ctzll(gs)) * WAVE + lane;
+                typename P::F fp;
+                double inv = 1.0;
+                bool take = e < count && lane % (DEP_THREADS / WAVE) == wave && P::foot(a, wd.list[first + e], fp);
+                if (take) {
+                    int lo[3], hi[3];
+                    P::box(fp, lo, hi);
+                    take = P::meets(a, lo, hi, t0);
+                    if (wd.inv) {
+                        inv = wd.inv[e];
+                        take = take && inv != 0.0;
+                    }
+                }
+                for (uint64_t ps = __ballot(take); ps; ps &= ps - 1)
+                    P::tile_wave(a, fp, inv, __builtin_ctzll(ps), t0, win);
+            }
+        }
+        __syncthreads();
+        for (int c = threadIdx.x; c < WIN_CELLS; c += DEP_THREADS) {
+            const double v = win[c];
+            if (v != 0.0) P::tile_flush(a, t0, c, v);
+        }
+        __syncthreads();
+    }
+}
+
+// the wide particles list[range[0] .. + range[1]) into the map.  At least
+// WIDE_BLOCKS blocks, so that a few tiles still fill the chip; a block whose
+// groups meet nothing ends after the box tests.
+// (Map of 1024^2: 2048, 4096, 8192 blocks 2.61, 2.50, 2.62 ms.)
+constexpr int64_t WIDE_BLOCKS = 4096;
+template <class P>
+void wide_deposit(mhip_ctx *ctx, typename P::Args a, const Wide &wd, int64_t ntile) {
+    hipStream_t s = ctx->stream;
+    const int64_t ng = (a.n + WAVE - 1) / WAVE;
+    const int nt = (a.res + P::SIDE - 1) / P::SIDE;
+    const int nslice = (int)std::min<int64_t>(ng, std::max<int64_t>(1, WIDE_BLOCKS / ntile));
+    hipLaunchKernelGGL(k_wide_boxes<P>, dim3((unsigned)std::min<int64_t>(1024, (ng + 3) / 4)), dim3(DEP_THREADS), 0, s,
+                       a, wd);
+    if (wd.inv)
+        hipLaunchKernelGGL(k_wide_totals<P>, dim3((unsigned)std::min<int64_t>(4096, a.n)), dim3(DEP_THREADS), 0, s, a,
+                           wd);
+    hipLaunchKernelGGL(k_wide_tiles<P>, dim3((unsigned)std::min<int64_t>(1 << 22, ntile * nslice)), dim3(DEP_THREADS),
+                       0, s, a, wd, nt, ntile, nslice);
+}
+
+// bits of a sort key in [0, top]
+static int key_bits(uint32_t top) { return 64 - __builtin_clzll((unsigned long long)top | 1ull); }
+
+// words the boxes of n particles take
+static size_t box_words(int64_t n) { return ((size_t)n / WAVE + 1) * 6; }
+// scratch for n particles: keys 16 n, values 8 n (room for the boxes), radix
+// counts, the wide particles' range.  The totals and boxes take the halves of
+// the keys and values that the sort leaves free.
+static size_t val_words(int64_t n) { return std::max((size_t)n, box_words(n)); }
+static size_t bin_scratch_bytes(int64_t n) {
+    return (size_t)n * 16 + val_words(n) * 8 + radix_counts_words(std::max<int64_t>(n, 1)) * 4 + 8 + 64;
+}
+
+// the binned path: keys, sort, runs, then the tiles of the wide particles
+template <class P>
+int bin_deposit(mhip_ctx *ctx, typename P::Args a, uint32_t skip, int64_t ntile, bool conservative, char *sc) {
     const int64_t n = a.n;
     if (n <= 0) return 0;
     uint64_t *k0 = (uint64_t *)sc, *k1 = k0 + n;
-    uint32_t *v0 = (uint32_t *)(k1 + n), *v1 = v0 + n, *counts = v1 + n;
+    uint32_t *v0 = (uint32_t *)(k1 + n), *v1 = v0 + val_words(n), *range = v1 + val_words(n), *counts = range + 2;
     hipStream_t s = ctx->stream;
     hipLaunchKernelGGL(k_bin_keys<P>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a, k0, v0);
     uint64_t *ks;
     uint32_t *vs;
-    int rc = radix_sort_pairs(ctx, k0, v0, k1, v1, counts, n, key_bits(skip) + SIZE_BITS, &ks, &vs);
+    int rc = radix_sort_pairs(ctx, k0, v0, k1, v1, counts, n, key_bits(2 * skip) + SIZE_BITS, &ks, &vs);
     if (rc) return rc;
     hipLaunchKernelGGL(k_bin_deposit<P>, dim3((unsigned)((n + BIN_CHUNK - 1) / BIN_CHUNK)), dim3(DEP_THREADS), 0, s,
                        a, ks, vs);
+    hipLaunchKernelGGL(k_wide_range, dim3(1), dim3(WAVE), 0, s, ks, n, skip, range);
+    const Wide wd{vs, range, (int *)(vs == v0 ? v1 : v0), conservative ? (double *)(ks == k0 ? k1 : k0) : nullptr};
+    wide_deposit<P>(ctx, a, wd, ntile);
     return 0;
-}
-
-// scratch bytes of bin_deposit plus the block-per-particle list (n + 1 words)
-static size_t bin_scratch_bytes(int64_t n) {
-    return (size_t)n * 24 + radix_counts_words(std::max<int64_t>(n, 1)) * 4 + ((size_t)n + 1) * 4 + 256;
-}
-
-// one block per listed particle (footprints above BIG_CELLS), HBM atomics
-__global__ __launch_bounds__(DEP_THREADS) void k_deposit_big(DepArgs a) {
-    __shared__ double red[DEP_THREADS];
-    const uint32_t nb = *a.nbig;
-    for (uint32_t e = blockIdx.x; e < nb; e += gridDim.x) {
-        Foot fp;
-        footprint(a, a.big[e], fp);  // listed, so it has a footprint
-        const int wy = fp.gy1 - fp.gy0 + 1;
-        const int64_t cells = (int64_t)(fp.gx1 - fp.gx0 + 1) * wy;
-        double tot = 1.0;
-        if (a.conservative) {
-            double part = 0.0;
-            for (int64_t c = threadIdx.x; c < cells; c += DEP_THREADS)
-                part += cell_weight(a, fp, fp.gx0 + (int)(c / wy), fp.gy0 + (int)(c % wy));
-            red[threadIdx.x] = part;
-            __syncthreads();
-            for (int o = DEP_THREADS / 2; o > 0; o >>= 1) {
-                if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-                __syncthreads();
-            }
-            tot = red[0];
-            __syncthreads();
-            if (tot == 0.0) continue;
-        }
-        for (int64_t c = threadIdx.x; c < cells; c += DEP_THREADS) {
-            const int gx = fp.gx0 + (int)(c / wy), gy = fp.gy0 + (int)(c % wy);
-            const double k = cell_weight(a, fp, gx, gy);
-            if (k != 0.0) atomicAdd(&a.grid[(int64_t)gx * a.res + gy], a.conservative ? k * fp.w / tot : k * fp.w);
-        }
-    }
 }
 
 __global__ __launch_bounds__(256) void k_grid_fill(double *__restrict__ g, int64_t n, double v) {
@@ -467,8 +845,8 @@ __global__ __launch_bounds__(256) void k_grid_scale(double *__restrict__ g, int6
         g[i] *= s;
 }
 
-__global__ void k_u32_zero(uint32_t *p) {
-    if (threadIdx.x == 0) *p = 0u;
+__global__ void k_range_zero(uint32_t *range) {
+    if (threadIdx.x < 2) range[threadIdx.x] = 0u;
 }
 
 // ---------------------------------------------------------------------------
@@ -479,7 +857,6 @@ __global__ void k_u32_zero(uint32_t *p) {
 // (g mod res) instead of clipping them.  kernel3d is the compact-support
 // spline: 0 beyond r = h (the reference leaves it unassigned there).
 // ---------------------------------------------------------------------------
-constexpr double KERNEL3D_NORM = 2.546479089470325;  // 8 / pi
 constexpr int64_t BIG_CELLS_3D = 512;
 
 struct Dep3Args {
@@ -491,26 +868,13 @@ struct Dep3Args {
     double dx;
     int res, periodic;
     double *grid;  // (res, res, res)
-    uint32_t *big, *nbig;
     int nb;  // bricks per axis
 };
 
 struct Foot3 {
-    double x[3], hs, hinv, f;
+    double x[3], hinv, f;
     int g0[3], g1[3];
 };
-
-MHIP_DEV double kernel3d(double q) {
-    if (q > 1.0) return 0.0;
-    double k;
-    if (q <= 0.5) {
-        k = 1.0 - 6.0 * q * q * (1.0 - q);
-    } else {
-        const double a = 1.0 - q;
-        k = 2.0 * a * a * a;
-    }
-    return k * KERNEL3D_NORM;
-}
 
 MHIP_DEV bool footprint3(const Dep3Args &a, int64_t i, Foot3 &fp) {
     const double o[3] = {a.ox, a.oy, a.oz};
@@ -521,7 +885,6 @@ MHIP_DEV bool footprint3(const Dep3Args &a, int64_t i, Foot3 &fp) {
     const double hs = fmin(fmax(hv, a.hmin), 1e100);
     if (!(hs > 0.0) || !isfinite(fp.x[0]) || !isfinite(fp.x[1]) || !isfinite(fp.x[2]) || !isfinite(fp.f))
         return false;
-    fp.hs = hs;
     fp.hinv = 1.0 / hs;
     for (int c = 0; c < 3; c++) {
         const double lo = (fp.x[c] - hs) / a.dx + 1.0, hi = (fp.x[c] + hs) / a.dx;
@@ -540,14 +903,30 @@ MHIP_DEV bool footprint3(const Dep3Args &a, int64_t i, Foot3 &fp) {
     return true;
 }
 
+MHIP_DEV Foot3 lane_foot(const Foot3 &f, int l) {
+    Foot3 r;
+    for (int c = 0; c < 3; c++) {
+        r.x[c] = lane_value(f.x[c], l);
+        r.g0[c] = lane_value(f.g0[c], l);
+        r.g1[c] = lane_value(f.g1[c], l);
+    }
+    r.hinv = lane_value(f.hinv, l);
+    r.f = lane_value(f.f, l);
+    return r;
+}
+
+// kernel weight without the kernel's constant, which cancels in the shares
 MHIP_DEV double weight3(const Dep3Args &a, const Foot3 &fp, int gx, int gy, int gz) {
-    double dx2 = fp.x[0] - gx * a.dx;
-    dx2 *= dx2;
-    double dy2 = fp.x[1] - gy * a.dx;
-    dy2 *= dy2;
-    double dz2 = fp.x[2] - gz * a.dx;
-    dz2 *= dz2;
-    return kernel3d(sqrt(dx2 + dy2 + dz2) * fp.hinv);
+    const double x = line_off(fp.x[0], gx, a.dx), y = line_off(fp.x[1], gy, a.dx), z = line_off(fp.x[2], gz, a.dx);
+    return spline_r2(x * x + y * y + z * z, fp.hinv);
+}
+
+// visit(gx, gy, gz, weight) over the footprint
+template <typename F>
+MHIP_DEV void each_cell3(const Dep3Args &a, const Foot3 &fp, F visit) {
+    for (int gx = fp.g0[0]; gx <= fp.g1[0]; gx++)
+        for (int gy = fp.g0[1]; gy <= fp.g1[1]; gy++)
+            for (int gz = fp.g0[2]; gz <= fp.g1[2]; gz++) visit(gx, gy, gz, weight3(a, fp, gx, gy, gz));
 }
 
 MHIP_DEV int64_t cell3(const Dep3Args &a, int gx, int gy, int gz) {
@@ -561,9 +940,7 @@ MHIP_DEV int64_t cell3(const Dep3Args &a, int gx, int gy, int gz) {
 
 MHIP_DEV double foot3_total(const Dep3Args &a, const Foot3 &fp) {
     double tot = 0.0;
-    for (int gx = fp.g0[0]; gx <= fp.g1[0]; gx++)
-        for (int gy = fp.g0[1]; gy <= fp.g1[1]; gy++)
-            for (int gz = fp.g0[2]; gz <= fp.g1[2]; gz++) tot += weight3(a, fp, gx, gy, gz);
+    each_cell3(a, fp, [&](int, int, int, double k) { tot += k; });
     return tot;
 }
 
@@ -582,7 +959,11 @@ struct Vol3 {
     static MHIP_DEV uint32_t key(const Dep3Args &a, int64_t i, uint32_t &ncell) {
         Foot3 fp;
         ncell = 0;
-        if (!footprint3(a, i, fp)) return skip(a);
+        if (!footprint3(a, i, fp)) return 2 * skip(a);
+        const uint32_t nb = (uint32_t)a.nb;
+        const uint32_t brick =
+            ((uint32_t)(wrapped_first(a, fp, 0) / BRICK3) * nb + (uint32_t)(wrapped_first(a, fp, 1) / BRICK3)) * nb +
+            (uint32_t)(wrapped_first(a, fp, 2) / BRICK3);
         int64_t cells = 1;
         bool fits = true;
         for (int c = 0; c < 3; c++) {
@@ -591,92 +972,107 @@ struct Vol3 {
             cells *= fits ? sp : 1;
         }
         if (!fits || cells > BIG_CELLS_3D) {
-            a.big[atomicAdd(a.nbig, 1u)] = (uint32_t)i;
-            return skip(a);
+            ncell = SIZE_MAX_RANK;
+            return skip(a) + brick;
         }
         ncell = (uint32_t)cells;
-        const uint32_t nb = (uint32_t)a.nb;
-        return ((uint32_t)(wrapped_first(a, fp, 0) / BRICK3) * nb + (uint32_t)(wrapped_first(a, fp, 1) / BRICK3)) * nb +
-               (uint32_t)(wrapped_first(a, fp, 2) / BRICK3);
+        return brick;
     }
     static MHIP_DEV void direct(const Dep3Args &a, uint32_t i) {
         Foot3 fp;
         footprint3(a, i, fp);  // keyed, so it has a footprint
         const double tot = foot3_total(a, fp);
         if (!(tot > 0.0)) return;
-        for (int gx = fp.g0[0]; gx <= fp.g1[0]; gx++)
-            for (int gy = fp.g0[1]; gy <= fp.g1[1]; gy++)
-                for (int gz = fp.g0[2]; gz <= fp.g1[2]; gz++) {
-                    const double k = weight3(a, fp, gx, gy, gz);
-                    if (k != 0.0) atomicAdd(&a.grid[cell3(a, gx, gy, gz)], fp.f * k / tot);
-                }
+        const double inv = 1.0 / tot;
+        each_cell3(a, fp, [&](int gx, int gy, int gz, double k) {
+            if (k != 0.0) atomicAdd(&a.grid[cell3(a, gx, gy, gz)], k * inv * fp.f);
+        });
     }
-    static MHIP_DEV void window(const Dep3Args &a, uint32_t i, uint32_t key, double *win) {
-        Foot3 fp;
-        footprint3(a, i, fp);
-        // window index of the footprint's first cell on each axis (0..7)
+    using F = Foot3;
+    static MHIP_DEV bool foot(const Dep3Args &a, uint32_t i, F &fp) { return footprint3(a, i, fp); }
+    static MHIP_DEV int cells(const F &fp) {
+        return (fp.g1[0] - fp.g0[0] + 1) * (fp.g1[1] - fp.g0[1] + 1) * (fp.g1[2] - fp.g0[2] + 1);
+    }
+    // a cell's place in a window or tile, up to that of its origin (modulo
+    // 2^32: unwrapped indices of a periodic box can be large)
+    static MHIP_DEV uint32_t slot(int x, int y, int z) {
+        return ((uint32_t)x * WIN3 + (uint32_t)y) * WIN3 + (uint32_t)z;
+    }
+    // window index of the footprint's first cell on each axis (0..7)
+    static MHIP_DEV void place(const Dep3Args &a, const F &fp, uint32_t key, int *s) {
         const uint32_t nb = (uint32_t)a.nb;
         const int b[3] = {(int)(key / (nb * nb)), (int)(key / nb % nb), (int)(key % nb)};
-        int s[3];
         for (int c = 0; c < 3; c++) s[c] = wrapped_first(a, fp, c) - b[c] * BRICK3;
-        const int wy = fp.g1[1] - fp.g0[1] + 1, wz = fp.g1[2] - fp.g0[2] + 1;
-        const int ncell = (fp.g1[0] - fp.g0[0] + 1) * wy * wz;
+    }
+    static MHIP_DEV void window_wave(const Dep3Args &a, const F &mine, int l, uint32_t key, double *win) {
+        const F fp = lane_foot(mine, l);
+        int s[3];
+        place(a, fp, key, s);
+        const uint32_t origin = slot(fp.g0[0] - s[0], fp.g0[1] - s[1], fp.g0[2] - s[2]);
+        Walk3 w;
+        w.start(threadIdx.x % WAVE, WAVE, fp.g0, fp.g1);
+        wave_spread(
+            w, cells(fp), true, [&](const Walk3 &c) { return weight3(a, fp, c.x, c.y, c.z); },
+            [&](const Walk3 &c, double k) { atomicAdd(&win[slot(c.x, c.y, c.z) - origin], k * fp.f); });
+    }
+    static MHIP_DEV void window(const Dep3Args &a, const F &fp, uint32_t key, double *win) {
+        int s[3];
+        place(a, fp, key, s);
+        const int wx = fp.g1[0] - fp.g0[0] + 1, wy = fp.g1[1] - fp.g0[1] + 1, wz = fp.g1[2] - fp.g0[2] + 1;
+        const int ncell = wx * wy * wz;
+        // a starting cell for each lane, as in Map2::window
+        const uint32_t lane = threadIdx.x % WAVE, row = lane / (uint32_t)wz;
+        const int g[3] = {fp.g0[0] + (int)(row / (uint32_t)wy % (uint32_t)wx), fp.g0[1] + (int)(row % (uint32_t)wy),
+                          fp.g0[2] + (int)(lane % (uint32_t)wz)};
+        int gx = g[0], gy = g[1], gz = g[2];
+        auto next = [&]() {
+            if (++gz > fp.g1[2]) {
+                gz = fp.g0[2];
+                if (++gy > fp.g1[1]) {
+                    gy = fp.g0[1];
+                    if (++gx > fp.g1[0]) gx = fp.g0[0];
+                }
+            }
+        };
+        auto at = [&]() {
+            return (gx - fp.g0[0] + s[0]) * (WIN3 * WIN3) + (gy - fp.g0[1] + s[1]) * WIN3 + (gz - fp.g0[2] + s[2]);
+        };
         if (ncell <= WCACHE3) {
             // small footprints: the weights stay in registers between the
-            // total (summed in foot3_total's order) and the deposit
+            // total and the deposit
             double wc[WCACHE3];
             double tot = 0.0;
-            int gx = fp.g0[0], gy = fp.g0[1], gz = fp.g0[2];
 #pragma unroll
             for (int c = 0; c < WCACHE3; c++) {
                 wc[c] = 0.0;
                 if (c < ncell) {
                     wc[c] = weight3(a, fp, gx, gy, gz);
                     tot += wc[c];
-                    if (++gz > fp.g1[2]) {
-                        gz = fp.g0[2];
-                        if (++gy > fp.g1[1]) {
-                            gy = fp.g0[1];
-                            gx++;
-                        }
-                    }
+                    next();
                 }
             }
             if (!(tot > 0.0)) return;
-            gx = fp.g0[0];
-            gy = fp.g0[1];
-            gz = fp.g0[2];
+            const double inv = 1.0 / tot;
+            gx = g[0];
+            gy = g[1];
+            gz = g[2];
 #pragma unroll
             for (int c = 0; c < WCACHE3; c++) {
                 if (c < ncell) {
-                    if (wc[c] != 0.0) {
-                        const int w = ((gx - fp.g0[0] + s[0]) * WIN3 + (gy - fp.g0[1] + s[1])) * WIN3 +
-                                      (gz - fp.g0[2] + s[2]);
-                        atomicAdd(&win[w], fp.f * wc[c] / tot);
-                    }
-                    if (++gz > fp.g1[2]) {
-                        gz = fp.g0[2];
-                        if (++gy > fp.g1[1]) {
-                            gy = fp.g0[1];
-                            gx++;
-                        }
-                    }
+                    if (wc[c] != 0.0) atomicAdd(&win[at()], wc[c] * inv * fp.f);
+                    next();
                 }
             }
             return;
         }
         const double tot = foot3_total(a, fp);
         if (!(tot > 0.0)) return;
-        for (int gx = fp.g0[0]; gx <= fp.g1[0]; gx++)
-            for (int gy = fp.g0[1]; gy <= fp.g1[1]; gy++)
-                for (int gz = fp.g0[2]; gz <= fp.g1[2]; gz++) {
-                    const double k = weight3(a, fp, gx, gy, gz);
-                    if (k != 0.0) {
-                        const int c = ((gx - fp.g0[0] + s[0]) * WIN3 + (gy - fp.g0[1] + s[1])) * WIN3 +
-                                      (gz - fp.g0[2] + s[2]);
-                        atomicAdd(&win[c], fp.f * k / tot);
-                    }
-                }
+        const double inv = 1.0 / tot;
+        for (int c = 0; c < ncell; c++) {
+            const double k = weight3(a, fp, gx, gy, gz);
+            if (k != 0.0) atomicAdd(&win[at()], k * inv * fp.f);
+            next();
+        }
     }
     static MHIP_DEV void flush(const Dep3Args &a, uint32_t key, int c, double v) {
         const uint32_t nb = (uint32_t)a.nb;
@@ -686,38 +1082,73 @@ struct Vol3 {
         if (!a.periodic && (gx >= a.res || gy >= a.res || gz >= a.res)) return;
         atomicAdd(&a.grid[cell3(a, gx, gy, gz)], v);
     }
-};
 
-// one block per listed particle (footprints above BIG_CELLS_3D)
-__global__ __launch_bounds__(DEP_THREADS) void k_density3d_big(Dep3Args a) {
-    __shared__ double red[DEP_THREADS];
-    const uint32_t nb = *a.nbig;
-    for (uint32_t e = blockIdx.x; e < nb; e += gridDim.x) {
-        Foot3 fp;
-        footprint3(a, a.big[e], fp);  // listed, so it has a footprint
-        const int wy = fp.g1[1] - fp.g0[1] + 1, wz = fp.g1[2] - fp.g0[2] + 1;
-        const int64_t cells = (int64_t)(fp.g1[0] - fp.g0[0] + 1) * wy * wz;
-        double part = 0.0;
-        for (int64_t c = threadIdx.x; c < cells; c += DEP_THREADS)
-            part += weight3(a, fp, fp.g0[0] + (int)(c / ((int64_t)wy * wz)), fp.g0[1] + (int)((c / wz) % wy),
-                            fp.g0[2] + (int)(c % wz));
-        red[threadIdx.x] = part;
-        __syncthreads();
-        for (int o = DEP_THREADS / 2; o > 0; o >>= 1) {
-            if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-            __syncthreads();
-        }
-        const double tot = red[0];
-        __syncthreads();
-        if (!(tot > 0.0)) continue;
-        for (int64_t c = threadIdx.x; c < cells; c += DEP_THREADS) {
-            const int gx = fp.g0[0] + (int)(c / ((int64_t)wy * wz)), gy = fp.g0[1] + (int)((c / wz) % wy),
-                      gz = fp.g0[2] + (int)(c % wz);
-            const double k = weight3(a, fp, gx, gy, gz);
-            if (k != 0.0) atomicAdd(&a.grid[cell3(a, gx, gy, gz)], fp.f * k / tot);
+    // ---- tiles of WIN3^3 cells; a periodic footprint meets a tile once for
+    // each m with cells of it shifted by m res inside
+    static constexpr int SIDE = WIN3;
+    static MHIP_DEV int floor_div(int x, int d) { return x >= 0 ? x / d : -1 - (-1 - x) / d; }
+    static MHIP_DEV void box(const F &fp, int *lo, int *hi) {
+        for (int c = 0; c < 3; c++) {
+            lo[c] = fp.g0[c];
+            hi[c] = fp.g1[c];
         }
     }
-}
+    static MHIP_DEV void corner(int64_t tile, int nt, int *t0) {
+        t0[0] = (int)(tile / ((int64_t)nt * nt)) * SIDE;
+        t0[1] = (int)(tile / nt % nt) * SIDE;
+        t0[2] = (int)(tile % nt) * SIDE;
+    }
+    // first and last shift m of the cells lo..hi that meets the tile's cells on
+    // one axis (the tile's cells past the grid are none: the grid's own images
+    // are there)
+    static MHIP_DEV void shifts(const Dep3Args &a, int lo, int hi, int t0, int &m0, int &m1) {
+        const int t1 = min(t0 + SIDE, a.res) - 1;
+        m0 = a.periodic ? -floor_div(t1 - lo, a.res) : (lo <= t1 ? 0 : 1);
+        m1 = a.periodic ? floor_div(hi - t0, a.res) : (hi >= t0 ? 0 : -1);
+    }
+    static MHIP_DEV bool meets(const Dep3Args &a, const int *lo, const int *hi, const int *t0) {
+        bool all = true;
+        for (int c = 0; c < 3; c++) {
+            int m0, m1;
+            shifts(a, lo[c], hi[c], t0[c], m0, m1);
+            all = all && m0 <= m1;
+        }
+        return all;
+    }
+    static MHIP_DEV double total(const Dep3Args &a, const F &fp, int thread, int stride) {
+        Walk3 w;
+        double tot = 0.0;
+        for (w.start(thread, stride, fp.g0, fp.g1); w.inside(); w.next()) tot += weight3(a, fp, w.x, w.y, w.z);
+        return tot;
+    }
+    static MHIP_DEV void tile_wave(const Dep3Args &a, const F &mine, double inv, int l, const int *t0, double *win) {
+        const F fp = lane_foot(mine, l);
+        const double f = fp.f * lane_value(inv, l);
+        int m0[3], m1[3];
+        for (int c = 0; c < 3; c++) shifts(a, fp.g0[c], fp.g1[c], t0[c], m0[c], m1[c]);
+        for (int mx = m0[0]; mx <= m1[0]; mx++)
+            for (int my = m0[1]; my <= m1[1]; my++)
+                for (int mz = m0[2]; mz <= m1[2]; mz++) {
+                    // the tile's cells in the footprint's own indices
+                    const int o[3] = {t0[0] + mx * a.res, t0[1] + my * a.res, t0[2] + mz * a.res};
+                    int lo[3], hi[3];
+                    for (int c = 0; c < 3; c++) {
+                        lo[c] = max(fp.g0[c], o[c]);
+                        hi[c] = min(fp.g1[c], o[c] + min(SIDE, a.res - t0[c]) - 1);
+                    }
+                    const uint32_t origin = slot(o[0], o[1], o[2]);
+                    Walk3 w;
+                    for (w.start(threadIdx.x % WAVE, WAVE, lo, hi); w.inside(); w.next()) {
+                        const double k = weight3(a, fp, w.x, w.y, w.z);
+                        if (k != 0.0) atomicAdd(&win[slot(w.x, w.y, w.z) - origin], k * f);
+                    }
+                }
+    }
+    static MHIP_DEV void tile_flush(const Dep3Args &a, const int *t0, int c, double v) {
+        const int gx = t0[0] + c / (SIDE * SIDE), gy = t0[1] + c / SIDE % SIDE, gz = t0[2] + c % SIDE;
+        atomicAdd(&a.grid[((int64_t)gx * a.res + gy) * a.res + gz], v);
+    }
+};
 
 int grid_density(mhip_ctx *ctx, const void *f, int f_f64, const void *pos, int pos_f64, int64_t n, const void *h,
                  int h_f64, double hmin, double cx, double cy, double cz, double size, int res, int periodic,
@@ -747,19 +1178,12 @@ int grid_density(mhip_ctx *ctx, const void *f, int f_f64, const void *pos, int p
     int rc = 0;
     char *sc = (char *)scratch(ctx, bin_scratch_bytes(n), &rc);
     if (!sc) return rc;
-    // the sort buffers first (8-byte keys), the block-per-particle list last
-    a.nbig = (uint32_t *)(sc + (size_t)n * 24 + radix_counts_words(std::max<int64_t>(n, 1)) * 4);
-    a.big = a.nbig + 1;
     hipStream_t s = ctx->stream;
-    const int64_t ncell = (int64_t)res * res * res;
+    const int64_t ncell = (int64_t)res * res * res, nt = (res + WIN3 - 1) / WIN3;
     ProfRegion pr(ctx, "grid_density");
     hipLaunchKernelGGL(k_grid_fill, dim3((unsigned)std::min<int64_t>(4096, (ncell + 255) / 256)), dim3(256), 0, s,
                        grid, ncell, 0.0);
-    hipLaunchKernelGGL(k_u32_zero, dim3(1), dim3(64), 0, s, a.nbig);
-    if (n > 0) {
-        if ((rc = bin_deposit<Vol3>(ctx, a, (uint32_t)(a.nb * a.nb * a.nb), sc))) return rc;
-        hipLaunchKernelGGL(k_density3d_big, dim3(2048), dim3(DEP_THREADS), 0, s, a);
-    }
+    if ((rc = bin_deposit<Vol3>(ctx, a, (uint32_t)(a.nb * a.nb * a.nb), nt * nt * nt, true, sc))) return rc;
     const double inv = 1.0 / (a.dx * a.dx * a.dx);
     hipLaunchKernelGGL(k_grid_scale, dim3((unsigned)std::min<int64_t>(4096, (ncell + 255) / 256)), dim3(256), 0, s,
                        grid, ncell, inv);
@@ -794,14 +1218,15 @@ int surface_density(mhip_ctx *ctx, const void *f, int f_f64, const void *pos, in
     int rc = 0;
     char *sc = (char *)scratch(ctx, bin_scratch_bytes(n), &rc);
     if (!sc) return rc;
-    a.nbig = (uint32_t *)(sc + (size_t)n * 24 + radix_counts_words(std::max<int64_t>(n, 1)) * 4);
-    a.big = a.nbig + 1;
+    // whole-map path: totals, range, list, boxes
+    uint32_t *range = (uint32_t *)(sc + (size_t)n * 8);
+    a.nbig = range + 1;
+    a.big = range + 2;
     hipStream_t s = ctx->stream;
-    const int64_t ncell = (int64_t)res * res;
+    const int64_t ncell = (int64_t)res * res, nt = (res + WIN2 - 1) / WIN2;
     ProfRegion pr(ctx, "surface_density");
     hipLaunchKernelGGL(k_grid_fill, dim3((unsigned)std::min<int64_t>(1024, (ncell + 255) / 256)), dim3(256), 0, s,
                        grid, ncell, 0.0);
-    hipLaunchKernelGGL(k_u32_zero, dim3(1), dim3(64), 0, s, a.nbig);
     if (n > 0) {
         int ncu = 0;
         if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, ctx->device) != hipSuccess || ncu < 1)
@@ -814,14 +1239,16 @@ int surface_density(mhip_ctx *ctx, const void *f, int f_f64, const void *pos, in
                                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
                 return check_hip(ctx, hipGetLastError(), "deposit LDS size");
             const int64_t nchunk = std::max<int64_t>(1, std::min<int64_t>(ncu, (n + 255) / 256));
+            hipLaunchKernelGGL(k_range_zero, dim3(1), dim3(WAVE), 0, s, range);
             hipLaunchKernelGGL(k_deposit_tiles, dim3((unsigned)nchunk), dim3(DEP_THREADS), lds, s, a, res, 1,
                                (int)nchunk);
+            const Wide wd{a.big, range, (int *)(a.big + n), conservative ? (double *)sc : nullptr};
+            wide_deposit<Map2>(ctx, a, wd, nt * nt);
         } else {
             // binned by 32^2 bricks (per-tile LDS copies of the map would
             // re-read every particle per tile)
-            if ((rc = bin_deposit<Map2>(ctx, a, (uint32_t)a.nb * (uint32_t)a.nb, sc))) return rc;
+            if ((rc = bin_deposit<Map2>(ctx, a, (uint32_t)a.nb * (uint32_t)a.nb, nt * nt, conservative != 0, sc))) return rc;
         }
-        hipLaunchKernelGGL(k_deposit_big, dim3(2048), dim3(DEP_THREADS), 0, s, a);
     }
     if (conservative) {
         const double dx2inv = 1.0 / (a.dx * a.dx);

@@ -197,3 +197,51 @@ def test_surface_density_map_beyond_int32_cells(oracle, cons):
     del g
     torch.cuda.empty_cache()
     np.testing.assert_allclose(win, total, rtol=1e-12)
+
+
+@pytest.mark.parametrize("cells", [8, 32, 34, 64, 66, 200, 700])
+def test_surface_density_footprint_widths(oracle, cells):
+    """Footprints about `cells` map cells wide, each side of the lane /
+    wavefront / window / tile limits (64 cells, 33 and 64 on a side), maps of
+    whole and partial tiles, a list shorter and longer than a group of 64.
+    Offsets of up to 400 cells carry 400 float64 roundings, a weight's slope is
+    at most 3 per h >= 1 cell, and the sums are of one sign: 3e-13 of the
+    largest value; 1e-11 allows for the order of 500 terms."""
+    torch = _torch()
+    from meshoid_amd import engine
+
+    rng = np.random.default_rng(cells)
+    for res, n in ((65, 40), (128, 500), (130, 500), (385, 70)):
+        dx = 10.0 / (res - 1)
+        pos = rng.random((n, 2)) * 12 - 1
+        h = 0.5 * cells * dx * (1 + 0.02 * rng.standard_normal(n))
+        f = rng.random(n) + 0.1
+        for cons in (False, True):
+            say("width", cells, "res", res, "conservative", cons)
+            td = lambda a: torch.from_numpy(a).cuda()
+            g = engine.surface_density(td(f), td(pos), td(h), np.array([5.0, 5.0]), 10.0, res, 1.0, cons)
+            go = oracle.grid_surface_density(f, pos, np.clip(h, 2 * 10.0 / res, 1e100), np.array([5.0, 5.0]), 10.0,
+                                             res, cons)
+            _close(g.cpu().numpy(), go, f"width {cells} res {res} cons {cons}")
+
+
+@pytest.mark.parametrize("cells", [2, 4, 9, 11, 17, 45])
+def test_grid_density_footprint_widths(oracle, cells):
+    """The same for volumes (64 cells, 9 and 16 on a side), periodic boxes
+    whose footprints reach round them more than once included."""
+    torch = _torch()
+    from meshoid_amd import engine
+
+    rng = np.random.default_rng(cells)
+    for res, n in ((17, 300), (33, 70), (40, 200)):
+        dx = 10.0 / (res - 1)
+        pos = rng.random((n, 3)) * 10
+        h = 0.5 * cells * dx * (1 + 0.02 * rng.standard_normal(n))
+        f = rng.random(n) + 0.1
+        for periodic in (False, True):
+            say("width", cells, "res", res, "periodic", periodic)
+            td = lambda a: torch.from_numpy(a).cuda()
+            g = engine.grid_density(td(f), td(pos), td(h), np.array([5.0] * 3), 10.0, res, periodic, dx)
+            go = oracle.grid_density(f, pos, np.maximum(h, dx), np.array([5.0] * 3), 10.0, res,
+                                     10.0 if periodic else -1.0)
+            _close(g.cpu().numpy(), go, f"width {cells} res {res} periodic {periodic}")
