@@ -18,11 +18,15 @@
 // stably sorted by tile (so each tile's records keep the far-first order),
 // and the sorted records are cut into chunks of equal length, one wavefront
 // per chunk.  A wavefront holds one tile in LDS at a time and applies the
-// chunk's records of that tile in order (one lane per pixel of a footprint,
-// so its LDS updates stay in program order), writing one segment per (chunk,
-// tile).  A tile's particles thus spread over as many wavefronts as their
+// chunk's records of that tile in order (its LDS updates stay in program
+// order), writing one segment per (chunk, tile).  A tile's particles thus spread over as many wavefronts as their
 // number asks for, however clustered they are.  A last kernel composes each
 // pixel's segments farthest first from the background i0.
+//
+// 2^20 clustered particles, 128^2 pixels, one band: 1.55 -> 0.78 ms.  The
+// chunks took 1.06 ms, at one record at a time and 1.4 wavefronts a SIMD, and
+// take 0.31 (bound by their float64 arithmetic and the serial updates); the
+// sort by z, eight passes, and the gather are now as much.
 //
 // The reference's multi-threaded driver composes its chunks with the largest
 // z nearest the observer while each chunk is swept with the largest z
@@ -33,7 +37,9 @@
 namespace mhip {
 
 constexpr double FOUR_PI = 12.566370614359172;
-constexpr int64_t RT_CHUNK = 1024;  // records per wavefront, at least
+// chunks: about RT_CHUNKS of them (8 wavefronts a SIMD: a chunk is a serial
+// chain), of at least RT_CHUNK records
+constexpr int64_t RT_CHUNKS = 8192, RT_CHUNK = 64;
 constexpr double RT_KERNEL2D_NORM = 1.8189136353359467;  // 40 / (7 pi)
 
 MHIP_DEV double rt_kernel2d(double q) {
@@ -187,11 +193,19 @@ struct RtChunkArgs {
 // one wavefront per chunk of sorted records.  The chunk's records of tile t
 // form the segment stored in slot (chunk + t): the records are sorted by tile,
 // so a later chunk never holds a smaller tile and the slots are distinct.
+//
+// 64 records at a time: each lane loads one particle and clips its footprint
+// to the tile.  They are applied in ascending order, as many side by side as
+// their cells allow: a run of records of at most 4 cells 16 at once on 4 lanes
+// each, of at most 16 cells 4 at once, any other on the whole wavefront.  Each
+// lane computes what its cell does (tau, the exponentials: ~300 float64
+// instructions), then the records' lanes update the LDS one record after the
+// other.  Most particles of a snapshot are narrower than two pixels, so one
+// record at a time left 60 of 64 lanes idle in those instructions.
 __global__ __launch_bounds__(64) void k_rt_chunk(RtChunkArgs c) {
-    extern __shared__ double lds[];
+    extern __shared__ double2 lds2[];  // (I, tau) per pixel and band
     const RtArgs &a = c.p;
     const int tcells = a.tw * a.tw * a.nf;
-    double *I = lds, *T = lds + tcells;
     const int lane = threadIdx.x;
     const int64_t r0 = (int64_t)blockIdx.x * c.per, r1 = min(c.nrec, r0 + c.per);
     const int t0 = (int)c.keys[r0], t1 = (int)c.keys[r1 - 1];
@@ -200,33 +214,28 @@ __global__ __launch_bounds__(64) void k_rt_chunk(RtChunkArgs c) {
         if (s0 >= s1) continue;
         const int tx0 = (t / a.ntx) * a.tw, ty0 = (t % a.ntx) * a.tw;
         const int tx1 = min(tx0 + a.tw, a.res) - 1, ty1 = min(ty0 + a.tw, a.res) - 1;
-        for (int e = lane; e < tcells; e += 64) {
-            I[e] = 0.0;
-            T[e] = 0.0;
-        }
+        for (int e = lane; e < tcells; e += 64) lds2[e] = make_double2(0.0, 0.0);
         __syncthreads();
-        // 64 records at a time: each lane loads one particle and clips its
-        // footprint to the tile; they are then applied one after another in
-        // ascending order, their data broadcast from the loading lane
         for (int64_t base = s0; base < s1; base += 64) {
             const int64_t r = base + lane;
-            bool hit = false;
-            int64_t kk = 0;
-            double mh2 = 0.0, hinv = 0.0, kap1 = 0.0, src1 = 0.0;
+            uint32_t kk = 0;
+            double mh2 = 0.0, hinv = 0.0, kap1 = 0.0, src1 = 0.0, hs2 = 0.0;
+            int box = 0, cells = 0;  // first cell in the tile and row length; cells inside
             RtFoot f;
-            f.xs0 = f.xs1 = f.hs = 0.0;
-            f.gx0 = f.gy0 = 0;
-            f.gx1 = f.gy1 = -1;
+            f.xs0 = f.xs1 = 0.0;
             if (r < s1) {
                 kk = c.vals[r];
                 const double m = a.sm[kk];
                 if (rt_footprint(a.sx[kk], a.sy[kk], a.sh[kk], m, a.dx, a.res, f)) {
-                    f.gx0 = max(f.gx0, tx0);
-                    f.gx1 = min(f.gx1, tx1);
-                    f.gy0 = max(f.gy0, ty0);
-                    f.gy1 = min(f.gy1, ty1);
-                    hit = f.gx0 <= f.gx1 && f.gy0 <= f.gy1;
-                    mh2 = m / (f.hs * f.hs);
+                    const int gx0 = max(f.gx0, tx0), gx1 = min(f.gx1, tx1);
+                    const int gy0 = max(f.gy0, ty0), gy1 = min(f.gy1, ty1);
+                    if (gx0 <= gx1 && gy0 <= gy1) {
+                        const int wy = gy1 - gy0 + 1;
+                        cells = (gx1 - gx0 + 1) * wy;
+                        box = (gx0 - tx0) | (gy0 - ty0) << 8 | wy << 16;
+                    }
+                    hs2 = f.hs * f.hs;
+                    mh2 = m / hs2;
                     hinv = 1.0 / f.hs;
                     if (a.nf == 1) {
                         // one band: kappa and the source term travel with
@@ -236,75 +245,121 @@ __global__ __launch_bounds__(64) void k_rt_chunk(RtChunkArgs c) {
                     }
                 }
             }
-            uint64_t todo = __ballot(hit);
-            while (todo) {
-                const int src = __ffsll((long long)todo) - 1;
-                todo &= todo - 1;
-                const int64_t kp = __shfl(kk, src);
-                const double pxs0 = __shfl(f.xs0, src), pxs1 = __shfl(f.xs1, src), phs = __shfl(f.hs, src);
+            // a record without cells is as good as a small one
+            const uint64_t le4 = __ballot(cells <= 4), le16 = __ballot(cells <= 16);
+            const int nrec = (int)min<int64_t>(64, s1 - base);
+            for (int p0 = 0; p0 < nrec;) {
+                // the run of small records from p0 on
+                const uint64_t big4 = ~(le4 >> p0), big16 = ~(le16 >> p0);
+                const int run4 = min(big4 ? __builtin_ctzll(big4) : 64, min(16, nrec - p0));
+                const int run16 = min(big16 ? __builtin_ctzll(big16) : 64, min(4, nrec - p0));
+                const int cnt = run4 >= run16 && run4 > 0 ? run4 : max(run16, 1);
+                const int sh = run4 >= run16 && run4 > 0 ? 2 : run16 > 0 ? 4 : 6;
+                const int g = lane >> sh, src = min(p0 + g, 63);
+                const uint32_t kp = __shfl(kk, src);
+                const double pxs0 = __shfl(f.xs0, src), pxs1 = __shfl(f.xs1, src), phs2 = __shfl(hs2, src);
                 const double pmh2 = __shfl(mh2, src), phinv = __shfl(hinv, src);
                 const double pkap1 = __shfl(kap1, src), psrc1 = __shfl(src1, src);
-                const int pgx0 = __shfl(f.gx0, src), pgx1 = __shfl(f.gx1, src), pgy0 = __shfl(f.gy0, src),
-                          pgy1 = __shfl(f.gy1, src);
-                const double hs2 = phs * phs;
-                const int wy = pgy1 - pgy0 + 1, cells = (pgx1 - pgx0 + 1) * wy;
-                for (int q = lane; q < cells; q += 64) {
-                    const int gx = pgx0 + q / wy, gy = pgy0 + q % wy;
-                    double ddx = pxs0 - gx * a.dx;
+                const int pbox = __shfl(box, src);
+                const int scells = __shfl(cells, src);  // (every lane takes part)
+                const int pcells = g < cnt ? scells : 0;
+                const int wy = max(pbox >> 16, 1);
+                const float rw = 1.0f / (float)wy;  // q < 256, wy <= 16: (q + 1/2) rw truncates to q / wy
+                const int first = lane & ((1 << sh) - 1);
+                // cells beyond 64 take further turns; only a record by itself has them
+                for (int q = first; __any(q < pcells); q += 64) {
+                    const int qx = (int)(((float)q + 0.5f) * rw);
+                    const int lx = (pbox & 255) + qx, ly = (pbox >> 8 & 255) + (q - qx * wy);
+                    double ddx = pxs0 - (tx0 + lx) * a.dx;
                     ddx *= ddx;
-                    double ddy = pxs1 - gy * a.dx;
+                    double ddy = pxs1 - (ty0 + ly) * a.dx;
                     ddy *= ddy;
                     const double rr = ddx + ddy;
-                    if (rr > hs2) continue;
-                    const double kern = rt_kernel2d(sqrt(rr) * phinv);
-                    const int p = ((gx - tx0) * a.tw + (gy - ty0)) * a.nf;
+                    const bool in = q < pcells && rr <= phs2;
+                    const double kern = in ? rt_kernel2d(sqrt(rr) * phinv) : 0.0;
+                    const int p = (lx * a.tw + ly) * a.nf;
                     for (int b = 0; b < a.nf; b++) {
-                        const double kap = a.nf == 1 ? pkap1 : a.skap[kp * a.nf + b];
-                        const double sv = a.nf == 1 ? psrc1 : a.ssrc[kp * a.nf + b];
-                        const double tau = kap * kern * pmh2;
-                        // 1 - exp(-tau) = -expm1(-tau) stays accurate for small tau;
-                        // exp(-tau) itself comes from 1 + expm1(-tau) only while that
-                        // sum does not cancel (tau <= 1/2), from exp beyond
-                        const double em1 = expm1(-tau), fac2 = -em1;
-                        const double fac1 = tau <= 0.5 ? 1.0 + em1 : exp(-tau);
-                        T[p + b] += tau;
-                        I[p + b] = fac1 * I[p + b] + fac2 * sv;
+                        double tau = 0.0, fac1 = 1.0, add = 0.0;
+                        if (in) {
+                            const double kap = a.nf == 1 ? pkap1 : a.skap[(int64_t)kp * a.nf + b];
+                            const double sv = a.nf == 1 ? psrc1 : a.ssrc[(int64_t)kp * a.nf + b];
+                            tau = kap * kern * pmh2;
+                            // 1 - exp(-tau) = -expm1(-tau) stays accurate for small tau;
+                            // exp(-tau) itself comes from 1 + expm1(-tau) only while that
+                            // sum does not cancel (tau <= 1/2), from exp beyond
+                            const double em1 = expm1(-tau);
+                            add = -em1 * sv;
+                            fac1 = tau <= 0.5 ? 1.0 + em1 : exp(-tau);
+                        }
+                        for (int o = 0; o < cnt; o++)
+                            if (g == o && in) {
+                                double2 v = lds2[p + b];
+                                v.y += tau;
+                                v.x = fac1 * v.x + add;
+                                lds2[p + b] = v;
+                            }
                     }
                 }
+                p0 += cnt;
             }
         }
         __syncthreads();
         const int64_t o = ((int64_t)blockIdx.x + t) * tcells;
         for (int e = lane; e < tcells; e += 64) {
-            c.B[o + e] = I[e];
-            c.A[o + e] = exp(-T[e]);
+            const double2 v = lds2[e];
+            c.B[o + e] = v.x;
+            c.A[o + e] = exp(-v.y);
         }
         __syncthreads();
     }
 }
 
 // I = i0, then the pixel's tile segments, chunk by chunk (farthest first):
-// I <- A_s I + B_s, A_s = exp(-tau_s)
+// I <- A_s I + B_s, A_s = exp(-tau_s).  A clump's tile has hundreds of
+// segments, and one thread per pixel waited for them one by one: RT_PARTS
+// threads compose a part of them each, I -> A I + B, then one the parts.
+constexpr int RT_PARTS = 16;
 __global__ __launch_bounds__(256) void k_rt_compose(const double *__restrict__ B, const double *__restrict__ A,
                                                     const double *__restrict__ i0,
                                                     const uint32_t *__restrict__ tstart, int64_t per, int res,
                                                     int tw, int ntx, int nf, double *__restrict__ out) {
-    const int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (p >= (int64_t)res * res * nf) return;
-    const int b = (int)(p % nf);
-    const int64_t pix = p / nf;
-    const int gx = (int)(pix / res), gy = (int)(pix % res);
-    const int t = (gx / tw) * ntx + gy / tw;
-    const int64_t e = (int64_t)((gx % tw) * tw + gy % tw) * nf + b;
-    const int64_t tcells = (int64_t)tw * tw * nf;
-    double I = i0 ? i0[p] : 0.0;
-    const int64_t s0 = tstart[t], s1 = tstart[t + 1];
-    if (s0 < s1)
-        for (int64_t ch = s0 / per; ch <= (s1 - 1) / per; ch++) {
-            const int64_t o = (ch + t) * tcells + e;
-            I = A[o] * I + B[o];
+    constexpr int PIX = 256 / RT_PARTS;
+    __shared__ double pa[RT_PARTS][PIX], pb[RT_PARTS][PIX];
+    const int me = threadIdx.x % PIX, part = threadIdx.x / PIX;
+    const int64_t npix = (int64_t)res * res * nf;
+    for (int64_t p0 = blockIdx.x * (int64_t)PIX; p0 < npix; p0 += (int64_t)gridDim.x * PIX) {
+        const int64_t p = p0 + me;
+        double At = 1.0, Bt = 0.0;
+        if (p < npix) {
+            const int b = (int)(p % nf);
+            const int64_t pix = p / nf;
+            const int gx = (int)(pix / res), gy = (int)(pix % res);
+            const int t = (gx / tw) * ntx + gy / tw;
+            const int64_t e = (int64_t)((gx % tw) * tw + gy % tw) * nf + b;
+            const int64_t tcells = (int64_t)tw * tw * nf;
+            const int64_t s0 = tstart[t], s1 = tstart[t + 1];
+            if (s0 < s1) {
+                const int64_t c0 = s0 / per, nc = (s1 - 1) / per - c0 + 1;
+                const int64_t ce = c0 + nc * (part + 1) / RT_PARTS;
+#pragma unroll 4
+                for (int64_t ch = c0 + nc * part / RT_PARTS; ch < ce; ch++) {
+                    const int64_t o = (ch + t) * tcells + e;
+                    At *= A[o];
+                    Bt = A[o] * Bt + B[o];
+                }
+            }
         }
-    out[p] = I;
+        pa[part][me] = At;
+        pb[part][me] = Bt;
+        __syncthreads();
+        if (part == 0 && p < npix) {
+            double I = i0 ? i0[p] : 0.0;
+#pragma unroll
+            for (int k = 0; k < RT_PARTS; k++) I = pa[k][me] * I + pb[k][me];
+            out[p] = I;
+        }
+        __syncthreads();
+    }
 }
 
 __global__ __launch_bounds__(256) void k_rt_zero(uint32_t *__restrict__ p, int64_t n) {
@@ -345,12 +400,13 @@ int radtransfer(mhip_ctx *ctx, const double *j, const double *m, const double *k
         if ((rc = check_hip(ctx, hipStreamSynchronize(s), "radtransfer count"))) return rc;
         if (nrec > 0xffffffffull) return fail(ctx, -4, "more than 2^32 (particle, tile) pairs");
     }
-    // records per chunk: at least RT_CHUNK, and the segment maps within 1 GB
-    // (or twice one per tile)
+    // records per chunk: for RT_CHUNKS chunks, at least RT_CHUNK, and the
+    // segment maps within 1 GB (or twice one per tile)
     const int64_t tcells = (int64_t)tw * tw * nf;
     const int64_t slot_bytes = tcells * 16;
     const int64_t avail = std::max<int64_t>(2 * (int64_t)ntile, (int64_t)(1ll << 30) / slot_bytes);
-    const int64_t per = std::max<int64_t>(RT_CHUNK, ((int64_t)nrec + (avail - ntile) - 1) / (avail - ntile));
+    const int64_t most = std::min<int64_t>(RT_CHUNKS, avail - ntile);
+    const int64_t per = std::max<int64_t>(RT_CHUNK, ((int64_t)nrec + most - 1) / most);
     const int64_t nchunk = ((int64_t)nrec + per - 1) / per;
     const int64_t nslot = nchunk + ntile;
     const int64_t nr = (int64_t)nrec;
@@ -391,8 +447,9 @@ int radtransfer(mhip_ctx *ctx, const double *j, const double *m, const double *k
         hipLaunchKernelGGL(k_rt_zero, dim3((unsigned)((ntile + 256) / 256)), dim3(256), 0, s, tstart,
                            (int64_t)ntile + 1);
     }
-    hipLaunchKernelGGL(k_rt_compose, dim3((unsigned)((npix * nf + 255) / 256)), dim3(256), 0, s, B, A, i0, tstart, per,
-                       res, tw, ntx, nf, out);
+    hipLaunchKernelGGL(k_rt_compose,
+                       dim3((unsigned)std::min<int64_t>(1 << 22, (npix * nf * RT_PARTS + 255) / 256)), dim3(256), 0, s,
+                       B, A, i0, tstart, per, res, tw, ntx, nf, out);
     return check_hip(ctx, hipGetLastError(), "radtransfer launch");
 }
 

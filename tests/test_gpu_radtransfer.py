@@ -111,3 +111,30 @@ def test_radtransfer_thick_particles_before_bright_background(oracle):
     say("per-pixel max rel", err.max(), "darkest pixel", want.min())
     assert want.min() < 1e-10 * i0  # the sightlines are optically thick
     assert err.max() <= 1e-11
+
+
+@pytest.mark.parametrize("width,n", [(1, 1), (1, 64), (2, 65), (3, 500), (5, 500), (9, 500), (16, 500), (40, 130),
+                                     (0, 2000)])
+def test_radtransfer_footprint_widths(oracle, width, n):
+    """Records of at most 4, at most 16, at most and more than 64 cells, alone
+    and in the order of a mixed set (width 0), around 64 records and several
+    chunks.  2000 ordered steps of three roundings and tau of as many terms:
+    2e-12 of the largest value at most."""
+    _torch()
+    import meshoid_amd
+
+    rng = np.random.default_rng(100 * width + n)
+    res, size = 37, 12.0
+    dx = size / (res - 1)
+    x = rng.random((n, 3)) * 13 - 6.5
+    w = np.full(n, width) if width else rng.choice([1, 1, 1, 1, 2, 3, 5, 9, 16], n)
+    h = 0.5 * w * dx * (1 + 0.01 * rng.standard_normal(n))
+    m = (rng.random(n) + 0.1) * h**2
+    for nf in (1, 2):
+        j, kap = rng.random((n, nf)) * 10, np.exp(rng.normal(-1.0, 1.5, (n, nf)))
+        say("radtransfer width", width, "n", n, "bands", nf)
+        img = meshoid_amd.radtransfer(j, m, kap, x, h, res, size, center=[0.0, 0.0, 0.0], i0=1.0)
+        want = oracle.radtransfer(j, m, kap, x, h, res, size, center=[0.0, 0.0, 0.0], i0=1.0)
+        err = np.abs(img - want).max() / np.abs(want).max()
+        say("  max rel to image max", err)
+        assert err <= 2e-12
