@@ -174,14 +174,23 @@ __global__ __launch_bounds__(256) void k_sfc_keys(const PT *__restrict__ pos, in
 // ranks its 64 keys by digit with ballot-based matching.
 // ---------------------------------------------------------------------------
 constexpr int RS_THREADS = 256;
-constexpr int RS_ITEMS = 16;
-constexpr int RS_TILE = RS_THREADS * RS_ITEMS;
+// keys per thread: 16, or 4 up to RS_SMALL keys, where tiles of 4096 keys are too
+// few for the chip and each is a serial chain of 16 rankings.  At 4, whole calls:
+// 4096 points 306 -> 233 us, 65536 464 -> 391, 200000 437 -> 385, two planes of
+// 512^2 sightlines 1114 -> 978, 2^20 particles sorted by 64 bits 794 -> 768; at
+// 10^6 points the two are alike (4.95 ms), from there 16 scatters longer runs
+constexpr int RS_ITEMS = 16, RS_ITEMS_SMALL = 4;
+constexpr int64_t RS_SMALL = 1 << 20;
+constexpr int RS_TILE = RS_THREADS * RS_ITEMS, RS_TILE_SMALL = RS_THREADS * RS_ITEMS_SMALL;
 
+// enough for any number of keys up to n
 size_t radix_counts_words(int64_t n) {
-    int64_t nb = (n + RS_TILE - 1) / RS_TILE;
+    const int64_t small = std::min(n, RS_SMALL);
+    const int64_t nb = std::max((n + RS_TILE - 1) / RS_TILE, (small + RS_TILE_SMALL - 1) / RS_TILE_SMALL);
     return (size_t)(256 * std::max<int64_t>(nb, 1) + 256);
 }
 
+template <int ITEMS>
 __global__ __launch_bounds__(RS_THREADS) void k_rs_hist(const uint64_t *__restrict__ keys, int64_t n,
                                                         int shift, uint32_t *__restrict__ counts,
                                                         int nblocks) {
@@ -189,9 +198,9 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_hist(const uint64_t *__restri
     const int tid = threadIdx.x, w = tid >> 6;
     for (int i = tid; i < 1024; i += RS_THREADS) (&h[0][0])[i] = 0;
     __syncthreads();
-    const int64_t base = (int64_t)blockIdx.x * RS_TILE;
+    const int64_t base = (int64_t)blockIdx.x * (RS_THREADS * ITEMS);
 #pragma unroll 4
-    for (int r = 0; r < RS_ITEMS; r++) {
+    for (int r = 0; r < ITEMS; r++) {
         int64_t idx = base + r * RS_THREADS + tid;
         if (idx < n) atomicAdd(&h[w][(uint32_t)(keys[idx] >> shift) & 255u], 1u);
     }
@@ -238,39 +247,40 @@ __global__ __launch_bounds__(256) void k_rs_scan(uint32_t *__restrict__ counts, 
 // digit in the earlier quarters + its rank within its quarter, which keeps
 // the order of equal digits (the sort is stable).
 constexpr int RS_WAVES = RS_THREADS / WAVE;
-constexpr int RS_QUARTER = RS_TILE / RS_WAVES;  // keys per wavefront
+template <int ITEMS>
 __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(const uint64_t *__restrict__ kin,
                                                            const uint32_t *__restrict__ vin, int64_t n,
                                                            int shift, const uint32_t *__restrict__ counts,
                                                            const uint32_t *__restrict__ totals,
                                                            int nblocks, uint64_t *__restrict__ kout,
                                                            uint32_t *__restrict__ vout) {
-    __shared__ uint64_t s_key[RS_TILE];
-    __shared__ uint32_t s_val[RS_TILE];
+    constexpr int TILE = RS_THREADS * ITEMS, QUARTER = TILE / RS_WAVES;  // keys per block, wavefront
+    __shared__ uint64_t s_key[TILE];
+    __shared__ uint32_t s_val[TILE];
     __shared__ uint32_t s_wc[RS_WAVES][256];  // per-wave digit counts (running, then offsets)
     __shared__ uint32_t s_gb[256];            // global position of the tile's first key of each digit
     __shared__ uint32_t s_lb[256];            // tile-local position of the first key of each digit
     __shared__ uint32_t s_tmp[256];
     const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
-    const int64_t base = (int64_t)blockIdx.x * RS_TILE;
-    const int tn = (int)min<int64_t>(RS_TILE, n - base);
+    const int64_t base = (int64_t)blockIdx.x * TILE;
+    const int tn = (int)min<int64_t>(TILE, n - base);
 #pragma unroll
     for (int ww = 0; ww < RS_WAVES; ww++) s_wc[ww][tid] = 0;
     __syncthreads();
     // this wavefront's quarter: input indices w*QUARTER + r*64 + lane
-    uint64_t key[RS_ITEMS];
-    uint32_t val[RS_ITEMS], rk[RS_ITEMS];
+    uint64_t key[ITEMS];
+    uint32_t val[ITEMS], rk[ITEMS];
     const uint64_t lt_mask = (1ull << lane) - 1ull;
 #pragma unroll
-    for (int r = 0; r < RS_ITEMS; r++) {
-        const int i = w * RS_QUARTER + r * WAVE + lane;
+    for (int r = 0; r < ITEMS; r++) {
+        const int i = w * QUARTER + r * WAVE + lane;
         const bool valid = i < tn;
         key[r] = valid ? kin[base + i] : 0ull;
         val[r] = valid ? vin[base + i] : 0u;
     }
 #pragma unroll
-    for (int r = 0; r < RS_ITEMS; r++) {
-        const int i = w * RS_QUARTER + r * WAVE + lane;
+    for (int r = 0; r < ITEMS; r++) {
+        const int i = w * QUARTER + r * WAVE + lane;
         const bool valid = i < tn;
         const uint32_t d = (uint32_t)(key[r] >> shift) & 255u;
         uint64_t peers = __ballot(valid);
@@ -320,8 +330,8 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(const uint64_t *__res
     s_gb[tid] = s_tmp[tid] - totals[tid] + counts[(int64_t)tid * nblocks + blockIdx.x];
     __syncthreads();
 #pragma unroll
-    for (int r = 0; r < RS_ITEMS; r++) {
-        const int i = w * RS_QUARTER + r * WAVE + lane;
+    for (int r = 0; r < ITEMS; r++) {
+        const int i = w * QUARTER + r * WAVE + lane;
         if (i < tn) {
             const uint32_t d = (uint32_t)(key[r] >> shift) & 255u;
             const uint32_t pos = s_lb[d] + s_wc[w][d] + rk[r];
@@ -345,15 +355,18 @@ int radix_sort_pairs(mhip_ctx *ctx, uint64_t *k0, uint32_t *v0, uint64_t *k1, ui
     uint64_t *ka = k0, *kb = k1;
     uint32_t *va = v0, *vb = v1;
     if (n > 1) {
-        const int nblocks = (int)((n + RS_TILE - 1) / RS_TILE);
+        const bool small = n <= RS_SMALL;
+        const int tile = small ? RS_TILE_SMALL : RS_TILE;
+        const int nblocks = (int)((n + tile - 1) / tile);
         uint32_t *totals = counts + (size_t)256 * nblocks;
+        auto hist = small ? k_rs_hist<RS_ITEMS_SMALL> : k_rs_hist<RS_ITEMS>;
+        auto scatter = small ? k_rs_scatter<RS_ITEMS_SMALL> : k_rs_scatter<RS_ITEMS>;
         for (int shift = lo_bit; shift < bits; shift += 8) {
-            hipLaunchKernelGGL(k_rs_hist, dim3(nblocks), dim3(RS_THREADS), 0, ctx->stream, ka, n,
-                               shift, counts, nblocks);
+            hipLaunchKernelGGL(hist, dim3(nblocks), dim3(RS_THREADS), 0, ctx->stream, ka, n, shift, counts, nblocks);
             hipLaunchKernelGGL(k_rs_scan, dim3(256), dim3(256), 0, ctx->stream, counts, nblocks,
                                totals);
-            hipLaunchKernelGGL(k_rs_scatter, dim3(nblocks), dim3(RS_THREADS), 0, ctx->stream, ka,
-                               va, n, shift, counts, totals, nblocks, kb, vb);
+            hipLaunchKernelGGL(scatter, dim3(nblocks), dim3(RS_THREADS), 0, ctx->stream, ka, va, n, shift, counts,
+                               totals, nblocks, kb, vb);
             std::swap(ka, kb);
             std::swap(va, vb);
         }

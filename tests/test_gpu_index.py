@@ -81,3 +81,10 @@ def test_nan_position_rejected_large(where):
         pos[n - 1, 2] = np.nan
     with pytest.raises(ValueError):
         engine.SpatialIndex().build(torch.from_numpy(pos).cuda())
+
+
+@pytest.mark.parametrize("n", [256, 1023, 1024, 1025, 4097, (1 << 20) - 1, 1 << 20, (1 << 20) + 1])
+def test_sort_tiles(n):
+    """Whole and partial tiles of 1024 keys, and both sides of the size from
+    which tiles of 4096 keys are taken."""
+    test_sort_is_stable_hilbert_order(n)
