@@ -270,7 +270,7 @@ MHIP_DEV float hsml_step(float h, float n, float p, float kf) {
 }
 
 // smoothing length of one query slot (float32 copy and float64); the
-// row-order h, density and volume are formed from it by k_rows_out
+// row-order h, density and volume are formed from it by k_rows_rec
 MHIP_DEV void write_h(const KnnArgs &a, int64_t slot, double h) {
     a.h_slot[slot] = (float)h;
     a.h64_slot[slot] = h;
