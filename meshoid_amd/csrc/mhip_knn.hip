@@ -298,8 +298,7 @@ __global__ __launch_bounds__(KNN_BLOCK) void k_knn_main(KnnArgs a) {
     const uint32_t row = a.qrow ? a.qrow[qs_slot] : a.perm[qs_slot];
     // a radius seed starts the k+1 slots at (seed radius)^2 instead of +inf: a
     // lane whose (k+1)-th slot still holds that bound at the end missed
-    const float sr = (a.seed_r && !a.redo) ? a.seed_r[row] : 0.f;
-    const float tau0 = sr > 0.f && sr < 3e18f ? sr * sr : INFINITY;
+    const float tau0 = a.redo ? INFINITY : radius_bound(a, row);
     const TreeView &t = a.t;
     const float *__restrict__ sx = t.sx;
     const float *__restrict__ sy = t.sy;
@@ -609,7 +608,7 @@ __global__ __launch_bounds__(KNN_BLOCK) void k_knn_main(KnnArgs a) {
                 atomicAdd(a.stats + STAT_WAVES, 1ull);
             }
         }
-        if (live) a.st_slot[slot] = 0;
+        if (live) a.st_slot[slot] = row_deferred(a.redo, missed, a.st_slot[slot]);
         return;
     }
     __builtin_amdgcn_wave_barrier();
@@ -751,7 +750,7 @@ __global__ __launch_bounds__(KNN_BLOCK) void k_knn_main(KnnArgs a) {
     // ambiguous queries for the resolver, one vector atomic per wavefront by
     // its lowest active lane (lanes that missed a radius seed left earlier;
     // in the redo launch only the recomputed lanes are new)
-    const bool amb = live && (st & ST_AMBIGUOUS) && (!a.redo || missed);
+    const bool amb = live && (st & ST_AMBIGUOUS) && row_is_new(a.redo, missed);
     const uint64_t am = __ballot(amb);
     if (am) {
         const int leader = __ffsll((long long)__ballot(1)) - 1;

@@ -125,11 +125,11 @@ MHIP_DEV float threshold(const float (&v)[NR], float top, int n, int nr, int lo_
 
 // Search for one query.  s_c: the wavefront's candidate buffer (64 NR entries
 // of squared distance and sorted index); s_lq: its leaf queue; s_stk: its walk stack.  Members go to
-// s_out[j * ncol + col], j < k; returns the row's status bits, tau = the k-th
-// squared distance.
+// s_out[j * ncol + col], j < k; returns the row's status bits, tau and tau1 =
+// the k-th and (k+1)-th squared distance.
 template <int NR, bool PER, bool P64, typename OFF>
 MHIP_DEV int32_t wave_search(const KnnArgs &a, int64_t slot, uint32_t qp, uint2 *s_c, uint32_t *s_lq,
-                             uint32_t (*s_stk)[4], uint32_t *s_out, int col, int ncol, float &tau_out) {
+                             uint32_t (*s_stk)[4], uint32_t *s_out, int col, int ncol, float &tau_out, float &tau1_out) {
     constexpr int CAP = 64 * NR;
     const int lane = threadIdx.x & (WAVE - 1);
     const TreeView &t = a.t;
@@ -387,6 +387,7 @@ MHIP_DEV int32_t wave_search(const KnnArgs &a, int64_t slot, uint32_t qp, uint2 
     lds_order();
     if (lane == 0) a.tau[slot] = tau;
     tau_out = tau;
+    tau1_out = tau1;
     return st;
 }
 
@@ -499,6 +500,7 @@ __global__ __launch_bounds__(64 * KW_WAVES) void k_knn_wave(KnnArgs a, uint32_t 
     __shared__ uint32_t s_lq[KW_WAVES][KW_LEAFQ];
     __shared__ uint32_t s_stk[KW_WAVES][MAX_DEPTH / 2 + 1][4];
     __shared__ uint32_t s_out[KMAX * NCOL];
+    __shared__ uint32_t s_mine[LIST ? NCOL : 1];  // the rows this launch finishes
     const int w = threadIdx.x >> 6, row = (threadIdx.x & 63) >> 4;
     auto serve = [&](int64_t slot0) {
         // the slot of this lane's row in the smoothing-length stage
@@ -510,10 +512,19 @@ __global__ __launch_bounds__(64 * KW_WAVES) void k_knn_wave(KnnArgs a, uint32_t 
             const int col = w * PW + i;
             const int64_t slot = slot0 + col;
             if (slot >= a.nq) break;
+            if (LIST) {
+                const bool mine = row_was_deferred((int32_t)uniform((uint32_t)a.st_slot[slot]));
+                if ((threadIdx.x & 63) == 0) s_mine[col] = mine;
+                if (!mine) continue;
+            }
             const uint32_t qp = uniform(a.qsorted ? a.qsorted[slot] : (uint32_t)slot);
-            float tq;
-            const int32_t sq = wave_search<NR, PER, P64, OFF>(a, slot, qp, s_c[w], s_lq[w], s_stk[w], s_out, col,
-                                                              NCOL, tq);
+            float tq, tq1;
+            int32_t sq = wave_search<NR, PER, P64, OFF>(a, slot, qp, s_c[w], s_lq[w], s_stk[w], s_out, col, NCOL, tq,
+                                                        tq1);
+            if (LIST && a.seed_r) {
+                const float bound = radius_bound(a, a.qrow ? a.qrow[slot] : a.perm[slot]);
+                if (bound < INFINITY && tq1 >= bound) sq |= ST_RADIUS_MISS;
+            }
             if (row == i) {
                 tau = tq;
                 st = sq;
@@ -524,16 +535,19 @@ __global__ __launch_bounds__(64 * KW_WAVES) void k_knn_wave(KnnArgs a, uint32_t 
         const int col = w * PW + min(row, PW - 1);
         const int64_t slot = slot0 + col;
         if (__any(on)) {
-            // rows without a query repeat the wavefront's first
-            if (!on) qr = (uint32_t)__shfl((int)qr, 0);
-            const int c = on ? col : w * PW;
+            // rows without a query repeat the wavefront's first that has one
+            const int some = (int)__builtin_ctzll(__ballot(on));
+            const uint32_t q0 = (uint32_t)__shfl((int)qr, some);
+            const int c0 = __shfl(col, some);
+            if (!on) qr = q0;
+            const int c = on ? col : c0;
             if (a.k <= 32) row_hsml<2, PER, P64, LIST>(a, on, slot, qr, tau, st, s_out, c, NCOL);
             else row_hsml<(NR > 4 ? 8 : 4), PER, P64, LIST>(a, on, slot, qr, tau, st, s_out, c, NCOL);
         }
         __syncthreads();
         for (int e = threadIdx.x; e < a.k * NCOL; e += 64 * KW_WAVES) {
             const int64_t s = slot0 + e % NCOL;
-            if (s < a.nq) a.nl_idx[(int64_t)(e / NCOL) * a.nq + s] = s_out[e];
+            if (s < a.nq && (!LIST || s_mine[e % NCOL])) a.nl_idx[(int64_t)(e / NCOL) * a.nq + s] = s_out[e];
         }
     };
     constexpr uint32_t PARTS = WAVE / NCOL;
