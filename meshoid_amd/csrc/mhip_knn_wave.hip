@@ -21,6 +21,8 @@
 //           per lane and wave-wide sums.
 // The same float32 distances, box tests and ambiguity rule as the main
 // kernel, so the member sets are the same; ambiguous rows go to the resolver.
+#include <float.h>
+
 #include <algorithm>
 #include <type_traits>
 
@@ -139,7 +141,10 @@ MHIP_DEV int32_t wave_search(const KnnArgs &a, int64_t slot, uint32_t qp, uint2 
     const uint32_t lc = qp / LEAF;
     int m = 0;               // candidates in the buffer
     int next = 0;            // buffer fill at which the bound is tightened
-    float bound = INFINITY;  // at least the (k+1)-th smallest d2 found so far
+    // at least the (k+1)-th smallest d2 found so far.  Squared distances that
+    // overflow float32 are no candidates (as in the main kernel): a row with
+    // fewer than k others goes to the resolver
+    float bound = FLT_MAX;
 
     auto load = [&](float (&v)[NR], uint32_t (&ix)[NR], int nr) {
         lds_order();
@@ -182,7 +187,7 @@ MHIP_DEV int32_t wave_search(const KnnArgs &a, int64_t slot, uint32_t qp, uint2 
         load(v, ix, nr);
         float top = bound;
         int n = m;
-        if (top < INFINITY) {
+        if (top < FLT_MAX) {
             n = count_le<NR>(v, top, nr);
         } else {
             top = 0.f;
@@ -208,7 +213,7 @@ MHIP_DEV int32_t wave_search(const KnnArgs &a, int64_t slot, uint32_t qp, uint2 
     };
     // 64 particles, one per lane
     auto append = [&](float d2, uint32_t p, bool in) {
-        const bool pass = in && d2 <= bound;  // padding is NaN: never appended
+        const bool pass = in && d2 <= bound;  // never the NaN of padding
         const uint64_t b = __ballot(pass);
         const int pos = m + lane_rank(b);
         if (pass) s_c[pos] = make_uint2(__float_as_uint(d2), p);
@@ -374,9 +379,11 @@ MHIP_DEV int32_t wave_search(const KnnArgs &a, int64_t slot, uint32_t qp, uint2 
     int cnt;
     if (tau1 > tau) {
         cnt = min(compact(v, ix, nr, 0, [&](float x) { return x <= tau; }, CAP), k);
-    } else {  // float32 ties at the k-th: every closer one, then ties up to k
+    } else {
+        // float32 ties at the k-th: every closer one, then ties up to k (with
+        // fewer than k candidates tau is +inf, which fills the empty places)
         const int c = compact(v, ix, nr, 0, [&](float x) { return x < tau; }, k);
-        cnt = min(compact(v, ix, nr, min(c, k), [&](float x) { return x == tau; }, k), k);
+        cnt = min(compact(v, ix, nr, min(c, k), [&](float x) { return x == tau && x < INFINITY; }, k), k);
     }
     if (cnt != k) st |= ST_COUNT;
     for (int j = lane; j < k; j += 64) {
@@ -428,7 +435,8 @@ MHIP_DEV void row_hsml(const KnnArgs &a, bool on, int64_t slot, uint32_t qp, flo
     const float norm = (float)hsml_norm(a.dim), kf = (float)k;
     float hi = (float)hsml_bound_coeff(a.dim) * rmax;
     bool run = on && !(st & ST_COUNT) && hi > 0.f;
-    float h = run ? fmaxf(HSML_START * rmax, lo) : 0.f;
+    // (no k-th distance: as the main kernel)
+    float h = run ? fmaxf(HSML_START * rmax, lo) : (rmax < INFINITY ? 0.f : INFINITY);
     if (SEED && run && a.seed_h) {
         const float seed = a.seed_h[a.qrow ? a.qrow[slot] : a.perm[slot]];
         if (seed > lo && seed < hi) h = seed;
