@@ -85,10 +85,11 @@ int mhip_index_build(mhip_ctx *ctx, mhip_index *ix, const void *pos, int pos_f64
                      int dim, double boxsize);
 int mhip_index_destroy(mhip_index *ix);
 /* Device memory of the index from the caller (e.g. a caching allocator's):
- * bytes that n particles need, and the memory, which the caller keeps until
- * the index is destroyed or given other memory (ptr NULL: the library
- * allocates again); the index has to be built anew, and a build that needs
- * more fails with MHIP_ERR_VALUE.  The caller orders its reuse after the
+ * bytes that n particles need, and the memory, aligned to 16 bytes (else
+ * MHIP_ERR_VALUE), which the caller keeps until the index is destroyed or given
+ * other memory (ptr NULL: the library allocates again); the index has to be
+ * built anew, and a build that needs more fails with MHIP_ERR_VALUE and leaves
+ * the index empty, its lists unusable.  The caller orders its reuse after the
  * work queued on every stream that used the index. */
 int64_t mhip_index_bytes(int64_t n, int pos_f64);
 int mhip_index_storage(mhip_index *ix, void *ptr, int64_t bytes);

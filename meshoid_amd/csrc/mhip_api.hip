@@ -53,6 +53,9 @@ int block_reserve(mhip_ctx *ctx, Block &b, size_t need, const char *what) {
     return rc;
 }
 
+// whether the caller's memory can hold the arrays: they are read 16 bytes at a time
+static bool storage_fits(const void *p, int64_t bytes) { return bytes >= 0 && ((uintptr_t)p & 15) == 0; }
+
 // the caller's memory instead of the library's own (null: the library's again)
 static void block_storage(Block &b, void *p, int64_t bytes) {
     if (b.p && !b.ext) (void)hipFree(b.p);
@@ -216,7 +219,7 @@ int64_t mhip_index_bytes(int64_t n, int pos_f64) {
 }
 
 int mhip_index_storage(mhip_index *ix, void *ptr, int64_t bytes) {
-    if (!ix || bytes < 0) return MHIP_ERR_VALUE;
+    if (!ix || !storage_fits(ptr, bytes)) return MHIP_ERR_VALUE;
     ix->n = 0;  // what was built is gone
     block_storage(ix->mem, ptr, bytes);
     return MHIP_OK;
@@ -229,7 +232,7 @@ int64_t mhip_nlist_bytes(int64_t nq, int k, int masked, int flags) {
 }
 
 int mhip_nlist_storage(mhip_nlist *nl, void *ptr, int64_t bytes) {
-    if (!nl || bytes < 0) return MHIP_ERR_VALUE;
+    if (!nl || !storage_fits(ptr, bytes)) return MHIP_ERR_VALUE;
     nl->nq = 0;
     nl->index = nullptr;
     block_storage(nl->mem, ptr, bytes);

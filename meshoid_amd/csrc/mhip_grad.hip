@@ -737,7 +737,7 @@ static void dispatch_apply(const ApplyArgs &a, int dim, int order, dim3 g, hipSt
 int apply_ops(mhip_ctx *ctx, const mhip_nlist *nl, const void *f, int f_f64, int64_t nf_rows, int K,
               int order, int weighted, float *out1, float *out2, int32_t *status, int32_t *any) {
     const mhip_index *ix = nl->index;
-    if (!ix || nl->nq < 1) return fail(ctx, -1, "neighbour list is empty");
+    if (!ix || ix->n < 1 || nl->nq < 1) return fail(ctx, -1, "neighbour list is empty");
     if (order != 1 && order != 2) return fail(ctx, -1, "order must be 1 or 2");
     if (K < 1) return fail(ctx, -1, "no field components");
     int rc = 0;

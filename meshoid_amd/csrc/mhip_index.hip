@@ -520,7 +520,11 @@ int index_build(mhip_ctx *ctx, const void *pos, int pos_f64, int64_t n, int dim,
     const int depth = ts.depth;
     int rc = 0;
     if (depth > MAX_DEPTH) return fail(ctx, -4, "tree too deep");
-    if ((rc = block_reserve(ctx, ix->mem, index_layout(ix, n, pos_f64, nullptr), "index"))) return rc;
+    mhip_index sized;  // (the arrays of ix stay as they are until there is memory)
+    if ((rc = block_reserve(ctx, ix->mem, index_layout(&sized, n, pos_f64, nullptr), "index"))) {
+        ix->n = 0;  // what was built may be gone
+        return rc;
+    }
     index_layout(ix, n, pos_f64, ix->mem.p);
     ix->iperm_ok = 0;
     ix->n = n;

@@ -1305,7 +1305,7 @@ __global__ __launch_bounds__(256) void k_nl_subset(
 int nlist_subset(mhip_ctx *ctx, const mhip_nlist *full, const int64_t *qidx, int64_t nq, const double *m_rows,
                  float *h_out, float *rho_out, float *vol_out, int32_t *status_out, mhip_nlist *nl) {
     const mhip_index *ix = full->index;
-    if (!ix || full->nq < 1) return fail(ctx, -1, "neighbour list is empty");
+    if (!ix || ix->n < 1 || full->nq < 1) return fail(ctx, -1, "neighbour list is empty");
     if (full->masked || full->nq != ix->n) return fail(ctx, -1, "the source list must cover every particle");
     if (nl == full) return fail(ctx, -1, "the subset needs a list of its own");
     if (nq < 1) return fail(ctx, -1, "no query rows");
@@ -1344,7 +1344,7 @@ __global__ __launch_bounds__(256) void k_export64(const uint32_t *__restrict__ i
 
 int nlist_export64(mhip_ctx *ctx, const mhip_nlist *nl, int32_t *ngb_out, double *dist_out) {
     const mhip_index *ix = nl->index;
-    if (!ix || nl->nq < 1) return fail(ctx, -1, "neighbour list is empty");
+    if (!ix || ix->n < 1 || nl->nq < 1) return fail(ctx, -1, "neighbour list is empty");
     if (!ix->pos_in) return fail(ctx, -1, "the index holds no positions");
     ProfRegion pr(ctx, "nlist_export64");
     const dim3 g(export_blocks(nl->nq)), b(256);
@@ -1375,7 +1375,7 @@ __global__ __launch_bounds__(256) void k_rows_h64(const double *__restrict__ h64
 }
 
 int nlist_hsml(mhip_ctx *ctx, const mhip_nlist *nl, double *h_out) {
-    if (!nl->index || nl->nq < 1) return fail(ctx, -1, "neighbour list is empty");
+    if (!nl->index || nl->index->n < 1 || nl->nq < 1) return fail(ctx, -1, "neighbour list is empty");
     hipLaunchKernelGGL(k_rows_h64, dim3((unsigned)((nl->nq + 255) / 256)), dim3(256), 0, ctx->stream, nl->h64,
                        nl->masked ? nl->qrow : nullptr, nl->index->perm, nl->nq, h_out);
     return check_hip(ctx, hipGetLastError(), "hsml copy launch");
@@ -1417,7 +1417,7 @@ __global__ __launch_bounds__(256) void k_rows64_split(const RowRec64 *__restrict
 int nlist_rows64(mhip_ctx *ctx, const mhip_nlist *nl, const double *m_rows, double *h, double *rho, double *vol,
                  int32_t *status) {
     const mhip_index *ix = nl->index;
-    if (!ix || nl->nq < 1) return fail(ctx, -1, "neighbour list is empty");
+    if (!ix || ix->n < 1 || nl->nq < 1) return fail(ctx, -1, "neighbour list is empty");
     int rc = 0;
     RowRec64 *rec = (RowRec64 *)scratch(ctx, (size_t)nl->nq * sizeof(RowRec64), &rc);
     if (!rec) return rc;
@@ -1431,7 +1431,7 @@ int nlist_rows64(mhip_ctx *ctx, const mhip_nlist *nl, const double *m_rows, doub
 
 int nlist_export(mhip_ctx *ctx, const mhip_nlist *nl, int32_t *ngb_out, float *dist_out) {
     const mhip_index *ix = nl->index;
-    if (!ix || nl->nq < 1) return fail(ctx, -1, "neighbour list is empty");
+    if (!ix || ix->n < 1 || nl->nq < 1) return fail(ctx, -1, "neighbour list is empty");
     if (!nl->has_d2) return fail(ctx, -1, "neighbour list was built without distances");
     ProfRegion pr(ctx, "nlist_export");
     hipLaunchKernelGGL(k_export, dim3(export_blocks(nl->nq)), dim3(256),

@@ -205,7 +205,7 @@ int kernel_weights(mhip_ctx *ctx, const void *dist, int dist_f64, const void *h,
 int kernel_stat(mhip_ctx *ctx, const mhip_nlist *nl, const void *f, int f_f64, int64_t nf_rows, int K,
                 int which, double *out) {
     const mhip_index *ix = nl->index;
-    if (!ix || nl->nq < 1) return fail(ctx, -1, "neighbour list is empty");
+    if (!ix || ix->n < 1 || nl->nq < 1) return fail(ctx, -1, "neighbour list is empty");
     if (K < 1) return fail(ctx, -1, "no field components");
     if (which == 0 && K != 1) return fail(ctx, -1, "KernelAverage takes a scalar field");
     int rc = 0;
