@@ -291,13 +291,18 @@ __global__ __launch_bounds__(64) void k_rt_chunk(RtChunkArgs c) {
                             add = -em1 * sv;
                             fac1 = tau <= 0.5 ? 1.0 + em1 : exp(-tau);
                         }
-                        for (int o = 0; o < cnt; o++)
+                        // the fence keeps the turns apart: each lane takes one, so
+                        // without it they could be merged, and of two records at
+                        // one cell the first would be lost
+                        for (int o = 0; o < cnt; o++) {
                             if (g == o && in) {
                                 double2 v = lds2[p + b];
                                 v.y += tau;
                                 v.x = fac1 * v.x + add;
                                 lds2[p + b] = v;
                             }
+                            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                        }
                     }
                 }
                 p0 += cnt;
