@@ -298,7 +298,7 @@ __global__ __launch_bounds__(KNN_BLOCK) void k_knn_main(KnnArgs a) {
     const uint32_t row = a.qrow ? a.qrow[qs_slot] : a.perm[qs_slot];
     // a radius seed starts the k+1 slots at (seed radius)^2 instead of +inf: a
     // lane whose (k+1)-th slot still holds that bound at the end missed
-    const float tau0 = a.redo ? INFINITY : radius_bound(a, row);
+    const float tau0 = radius_bound((a.seed_r && !a.redo) ? a.seed_r[row] : 0.f);
     const TreeView &t = a.t;
     const float *__restrict__ sx = t.sx;
     const float *__restrict__ sy = t.sy;
@@ -608,7 +608,7 @@ __global__ __launch_bounds__(KNN_BLOCK) void k_knn_main(KnnArgs a) {
                 atomicAdd(a.stats + STAT_WAVES, 1ull);
             }
         }
-        if (live) a.st_slot[slot] = row_deferred(a.redo, missed, a.st_slot[slot]);
+        if (live && row_is_new(a.redo, missed)) a.st_slot[slot] = ROW_DEFERRED;
         return;
     }
     __builtin_amdgcn_wave_barrier();

@@ -182,12 +182,9 @@ struct KnnArgs {
     uint32_t wlcap;             // leaf-record capacity used (<= WLCAP; smaller only as a test hook)
 };
 
-// squared radius seed of an output row, +inf without one: a row whose (k+1)-th
-// squared distance is not below it missed (ST_RADIUS_MISS)
-MHIP_DEV float radius_bound(const KnnArgs &a, uint32_t row) {
-    const float sr = a.seed_r ? a.seed_r[row] : 0.f;
-    return sr > 0.f && sr < 3e18f ? sr * sr : INFINITY;
-}
+// square of a radius seed, +inf for none (0): a row whose (k+1)-th squared
+// distance is not below it missed (ST_RADIUS_MISS)
+MHIP_DEV float radius_bound(float sr) { return sr > 0.f && sr < 3e18f ? sr * sr : INFINITY; }
 
 MHIP_DEV void pad_list(const KnnArgs &a, int cnt, uint32_t qp, int64_t slot) {
     // never leave undefined indices behind: pad with the query itself

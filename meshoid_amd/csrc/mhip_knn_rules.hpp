@@ -19,16 +19,14 @@
 namespace mhip {
 
 // in a row's status between the launches: a deferring wavefront left the row
-// to the one-wavefront-per-query kernel (no bit of the public status)
+// to the one-wavefront-per-query kernel (no bit of the public status).  Rows
+// that an earlier launch finished keep their status.
 constexpr int32_t ROW_DEFERRED = 1 << 30;
 
 // whether the one-lane kernel is to finish this row, in the first launch or in
-// the redo launch (missed: the row's radius seed was too small in the first)
+// the redo launch (missed: the row's radius seed was too small in the first): a
+// wavefront lists such rows if it finishes them, and marks them if it defers
 MHIP_HD bool row_is_new(bool redo, bool missed) { return !redo || missed; }
-
-// the status that a deferring wavefront leaves: rows that the first launch
-// finished keep theirs
-MHIP_HD int32_t row_deferred(bool redo, bool missed, int32_t st) { return row_is_new(redo, missed) ? ROW_DEFERRED : st; }
 
 // whether the one-wavefront kernel is to finish this row of a deferred wavefront
 MHIP_HD bool row_was_deferred(int32_t st) { return (st & ROW_DEFERRED) != 0; }

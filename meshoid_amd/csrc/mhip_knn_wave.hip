@@ -530,7 +530,7 @@ __global__ __launch_bounds__(64 * KW_WAVES) void k_knn_wave(KnnArgs a, uint32_t 
             int32_t sq = wave_search<NR, PER, P64, OFF>(a, slot, qp, s_c[w], s_lq[w], s_stk[w], s_out, col, NCOL, tq,
                                                         tq1);
             if (LIST && a.seed_r) {
-                const float bound = radius_bound(a, a.qrow ? a.qrow[slot] : a.perm[slot]);
+                const float bound = radius_bound(a.seed_r[a.qrow ? a.qrow[slot] : a.perm[slot]]);
                 if (bound < INFINITY && tq1 >= bound) sq |= ST_RADIUS_MISS;
             }
             if (row == i) {

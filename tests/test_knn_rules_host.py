@@ -11,7 +11,7 @@ import pytest
 SRC = """
 #include "%s"
 extern "C" int is_new(int redo, int missed) { return mhip::row_is_new(redo, missed); }
-extern "C" int deferred(int redo, int missed, int st) { return mhip::row_deferred(redo, missed, st); }
+extern "C" int mark() { return mhip::ROW_DEFERRED; }
 extern "C" int was_deferred(int st) { return mhip::row_was_deferred(st); }
 """
 
@@ -45,7 +45,7 @@ def test_each_row_is_finished_and_listed_once(rules):
                 # first launch
                 if defer1:
                     on_list += 1
-                    st = [rules.deferred(0, 0, s) for s in st]
+                    st = [rules.mark() if rules.is_new(0, 0) else s for s in st]
                 else:
                     for r in range(3):
                         if miss[r]:
@@ -57,7 +57,7 @@ def test_each_row_is_finished_and_listed_once(rules):
                 if any(missed):
                     if defer2:
                         on_list += 1
-                        st = [rules.deferred(1, m, s) for m, s in zip(missed, st)]
+                        st = [rules.mark() if rules.is_new(1, m) else s for m, s in zip(missed, st)]
                     else:
                         for r in range(3):
                             if rules.is_new(1, missed[r]):
@@ -71,4 +71,4 @@ def test_each_row_is_finished_and_listed_once(rules):
                 assert finished == [1, 1, 1]
                 assert listed == [int(a) for a in amb] and sum(listed) <= 3
                 assert [bool(s & MISS) for s in st] == [bool(m) for m in miss]
-                assert all(s < 1 << 30 for s in st)
+                assert all(s < rules.mark() for s in st)
