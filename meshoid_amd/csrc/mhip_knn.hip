@@ -379,7 +379,9 @@ __global__ __launch_bounds__(KNN_BLOCK) void k_knn_main(KnnArgs a) {
     float g = NAN;                    // this lane's leaf's distance (NaN: none, or visited)
     int cls = 3, lpos = 0;            // next class; the curve's position in the block
     // the walk above the leaves is needed once per block of leaves: it lives
-    // in LDS, the scalar registers being short (48 hold a leaf's candidates)
+    // in LDS, the scalar registers being short (48 hold a leaf's candidates).
+    // Lane 0 writes it, and what is read is lane 0's own value (uniform), so no
+    // fence is needed
     struct Walk {
         uint32_t own;        // ancestor of the middle leaf whose subtree is done,
         int lev;             // its level
@@ -611,7 +613,7 @@ __global__ __launch_bounds__(KNN_BLOCK) void k_knn_main(KnnArgs a) {
         if (live && row_is_new(a.redo, missed)) a.st_slot[slot] = ROW_DEFERRED;
         return;
     }
-    __builtin_amdgcn_wave_barrier();
+    lds_order();  // lane 0 wrote the leaf record that every lane reads
     if (a.stats && lane == 0) {
         atomicAdd(a.stats + STAT_P1_LEAVES, (unsigned long long)n_leaf);
         atomicAdd(a.stats + STAT_P1_NODES, (unsigned long long)n_nodes);

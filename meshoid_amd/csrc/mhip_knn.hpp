@@ -128,6 +128,10 @@ MHIP_DEV void load_leaf(const TreeView &t, int64_t leaf, float (&cx)[LEAF], floa
     }
 }
 
+// orders this wavefront's LDS accesses (they execute in program order; this
+// keeps the compiler from moving them across)
+MHIP_DEV void lds_order() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
+
 // wavefront minimum / maximum on the DPP network: rows of 16, then the row
 // broadcasts; the result is in lane 63
 template <int CTRL, int ROWS>

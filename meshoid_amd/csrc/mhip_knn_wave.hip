@@ -70,10 +70,6 @@ MHIP_DEV int lane_rank(uint64_t m) {  // set bits of m below this lane
     return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
 }
 
-// orders this wavefront's LDS accesses (they execute in program order; this
-// keeps the compiler from moving them across)
-MHIP_DEV void lds_order() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
-
 // element p of a float array: with fewer than 2^30 of them (OFF = uint32_t)
 // through a 32-bit byte offset from a scalar base
 template <typename OFF>
