@@ -15,6 +15,8 @@
 #include <string>
 #include <vector>
 
+#include "mhip_hsml.hpp"
+
 #define MHIP_DEV __device__ __forceinline__
 
 namespace mhip {
@@ -66,12 +68,6 @@ MHIP_DEV void kernel_w_dw(T q, T &w, T &dw) {
         w = T(0);
         dw = T(0);
     }
-}
-
-// norm_d of kernel_density.py:26-31 and the bracket factor of :35
-MHIP_DEV double hsml_norm(int dim) { return dim == 3 ? 32.0 / 3 : (dim == 2 ? 40.0 / 7 : 8.0 / 3); }
-MHIP_DEV double hsml_bound_coeff(int dim) {
-    return dim == 3 ? 1.5638742363463305 : (dim == 2 ? 1.7984058958344455 : 2.33839974837265);
 }
 
 // nearest_image of src/meshoid/derivatives.py:8-14 (box > 0)

@@ -28,6 +28,8 @@
 //       rows.  Queries whose k-th and (k+1)-th distances float32 cannot order
 //       are re-ranked with float64 distances from the caller's positions, so
 //       neighbour sets equal the float64 kNN except for float64 ties.
+//       The same kernel finishes smoothing lengths that one float64 step does
+//       not give (rows where n(h) is flat at the root, see hsml_last).
 //   Wavefronts whose queries spread over a large region, and in periodic sets
 //   those whose balls reach a face of the box, are left to the other kernel.
 // It is bound by vector instructions: 27.9k a wavefront at 2^24 clustered
@@ -648,6 +650,7 @@ __global__ __launch_bounds__(KNN_BLOCK) void k_knn_main(KnnArgs a) {
         a.tau[slot] = tau;
     }
     double h64 = (double)h;
+    bool flat = false;  // h is left to the resolver
     // members: a candidate at or below tau passed its lane's queue filter
     // when its leaf was scanned, so it lies in a recorded leaf; leaves no
     // final ball reaches are skipped
@@ -740,19 +743,19 @@ __global__ __launch_bounds__(KNN_BLOCK) void k_knn_main(KnnArgs a) {
         // the resolver once it has rebuilt them
         if (live && cnt == a.k && h > 0.f && !(st & (ST_HSML_NOCONV | ST_AMBIGUOUS))) {
             if (STAGE)
-                h64 = refine_h64<false, P64>(a, q, h64, [&](int j) { return s_buf[w][j][lane]; });
+                h64 = refine_h64<false, P64>(a, q, h64, flat, [&](int j) { return s_buf[w][j][lane]; });
             else
-                h64 = refine_h64<false, P64>(a, q, h64, [&](int j) { return a.nl_idx[(int64_t)j * a.nq + slot]; });
+                h64 = refine_h64<false, P64>(a, q, h64, flat, [&](int j) { return a.nl_idx[(int64_t)j * a.nq + slot]; });
         }
     }
     if (live) {
         write_h(a, slot, h64);
         a.st_slot[slot] = st;
     }
-    // ambiguous queries for the resolver, one vector atomic per wavefront by
+    // ambiguous and flat queries for the resolver, one vector atomic per wavefront by
     // its lowest active lane (lanes that missed a radius seed left earlier;
     // in the redo launch only the recomputed lanes are new)
-    const bool amb = live && (st & ST_AMBIGUOUS) && row_is_new(a.redo, missed);
+    const bool amb = live && ((st & ST_AMBIGUOUS) || flat) && row_is_new(a.redo, missed);
     const uint64_t am = __ballot(amb);
     if (am) {
         const int leader = __ffsll((long long)__ballot(1)) - 1;
@@ -761,6 +764,44 @@ __global__ __launch_bounds__(KNN_BLOCK) void k_knn_main(KnnArgs a) {
         base = __shfl(base, leader);
         if (amb) a.amb[1 + base + __popcll(am & ((1ull << lane) - 1ull))] = (uint32_t)slot;
     }
+}
+
+// the float64 smoothing length of a slot by one wavefront, from its present one;
+// the list's members are in memory, up to two of them a lane (k <= 128)
+template <bool PER, bool P64>
+MHIP_DEV void refine_slot(const KnnArgs &a, const QPos &q, int64_t slot) {
+    const int lane = threadIdx.x;
+    double r[2] = {1e300, 1e300};  // (no member: no weight)
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+        if (u * WAVE + lane < a.k)
+            r[u] = member_dist<PER, P64>(a.t, q, a.nl_idx[(int64_t)(u * WAVE + lane) * a.nq + slot]);
+    const double h = hsml_refine(
+        a.h64_slot[slot], a.k, a.dim,
+        [&](double x) {
+            const double ix = 1.0 / x;
+            HsmlSums s;
+            s.add(r[0] * ix);
+            s.add(r[1] * ix);
+#pragma unroll
+            for (int o = WAVE / 2; o > 0; o >>= 1) {
+                s.w += __shfl_xor(s.w, o);
+                s.d1 += __shfl_xor(s.d1, o);
+                s.d2 += __shfl_xor(s.d2, o);
+            }
+            return s;
+        },
+        [&] {
+            HsmlRange g;
+#pragma unroll
+            for (int u = 0; u < 2; u++)
+                if (u * WAVE + lane < a.k) g.add(r[u]);
+#pragma unroll
+            for (int o = WAVE / 2; o > 0; o >>= 1)
+                g.join(HsmlRange{__shfl_xor(g.r0, o), __shfl_xor(g.r1, o), __shfl_xor(g.rk, o)});
+            return g;
+        });
+    if (lane == 0) write_h(a, slot, h);
 }
 
 // float64 squared distance between original particles i and j
@@ -896,36 +937,38 @@ MHIP_DEV void resolve_slot(const KnnArgs &a, const PT *__restrict__ pos_in, int6
         }
     }
     __syncthreads();
-    if (lane != 0) return;
-    // order the band by (exact d^2, original index) and take what is missing
-    for (int i = 1; i < nb; i++) {
-        const double v = s_bd[i];
-        const uint32_t vi = s_bi[i];
-        int j = i - 1;
-        while (j >= 0 && (s_bd[j] > v || (s_bd[j] == v && a.perm[s_bi[j]] > a.perm[vi]))) {
-            s_bd[j + 1] = s_bd[j];
-            s_bi[j + 1] = s_bi[j];
-            j--;
-        }
-        s_bd[j + 1] = v;
-        s_bi[j + 1] = vi;
-    }
-    for (int i = 0; i < nb && cnt < a.k; i++, cnt++) {
-        a.nl_idx[(int64_t)cnt * nq + slot] = s_bi[i];
-        if (a.nl_d2) a.nl_d2[(int64_t)cnt * nq + slot] = (float)s_bd[i];
-    }
-    if (cnt != a.k) {
+    // where float32 distances overflowed there was no solve yet
+    const float h0 = a.h_slot[slot];
+    if (!(h0 < INFINITY)) st &= ~ST_HSML_NOCONV;
+    // (cnt, nb and st are the same in every lane)
+    const int have = cnt, total = cnt < a.k ? min(cnt + nb, a.k) : cnt;
+    if (total != a.k)
         st |= ST_COUNT;
-        pad_list(a, min(cnt, a.k), qp, slot);
-    } else {
+    else
         st &= ~ST_COUNT;
-        if (a.h_slot[slot] > 0.f && !(st & ST_HSML_NOCONV)) {
-            const double h64 = refine_h64<PER, P64>(a, q, (double)a.h_slot[slot],
-                                                    [&](int j) { return a.nl_idx[(int64_t)j * nq + slot]; });
-            write_h(a, slot, h64);
+    if (lane == 0) {
+        // order the band by (exact d^2, original index) and take what is missing
+        for (int i = 1; i < nb; i++) {
+            const double v = s_bd[i];
+            const uint32_t vi = s_bi[i];
+            int j = i - 1;
+            while (j >= 0 && (s_bd[j] > v || (s_bd[j] == v && a.perm[s_bi[j]] > a.perm[vi]))) {
+                s_bd[j + 1] = s_bd[j];
+                s_bi[j + 1] = s_bi[j];
+                j--;
+            }
+            s_bd[j + 1] = v;
+            s_bi[j + 1] = vi;
         }
+        for (int i = 0; have + i < total; i++) {
+            a.nl_idx[(int64_t)(have + i) * nq + slot] = s_bi[i];
+            if (a.nl_d2) a.nl_d2[(int64_t)(have + i) * nq + slot] = (float)s_bd[i];
+        }
+        if (total != a.k) pad_list(a, min(total, a.k), qp, slot);
+        a.st_slot[slot] = st;
     }
-    a.st_slot[slot] = st;
+    __syncthreads();
+    if (total == a.k && h0 > 0.f && !(st & ST_HSML_NOCONV)) refine_slot<PER, P64>(a, q, slot);
 }
 
 // empties the lists of ambiguous slots and of deferred wavefronts (a kernel,
@@ -934,8 +977,9 @@ __global__ void k_lists_reset(uint32_t *__restrict__ amb, uint32_t *__restrict__
     if (threadIdx.x == 0) amb[0] = defer[0] = 0u;
 }
 
-// the list of ambiguous slots, one wavefront per slot (a grid-stride loop
-// over the list, whose length only the device knows)
+// the list of ambiguous slots and of those whose smoothing length one step does
+// not give, one wavefront per slot (a grid-stride loop over the list, whose
+// length only the device knows)
 template <bool PER, bool P64, typename PT>
 __global__ __launch_bounds__(64) void k_knn_resolve(KnnArgs a, const PT *__restrict__ pos_in) {
     __shared__ double s_bd[BAND_CAP];
@@ -943,8 +987,11 @@ __global__ __launch_bounds__(64) void k_knn_resolve(KnnArgs a, const PT *__restr
     const uint32_t count = a.amb[0];
     for (int64_t i = blockIdx.x; i < count; i += gridDim.x) {
         const int64_t slot = a.amb[1 + i];
-        if (slot >= a.nq || !(a.st_slot[slot] & ST_AMBIGUOUS)) continue;
-        resolve_slot<PER, P64, PT>(a, pos_in, slot, s_bd, s_bi);
+        if (slot >= a.nq) continue;
+        if (a.st_slot[slot] & ST_AMBIGUOUS)
+            resolve_slot<PER, P64, PT>(a, pos_in, slot, s_bd, s_bi);
+        else
+            refine_slot<PER, P64>(a, load_q<P64>(a.t, a.qsorted ? a.qsorted[slot] : (uint32_t)slot), slot);
         __syncthreads();  // the next slot reuses the band arrays
     }
 }

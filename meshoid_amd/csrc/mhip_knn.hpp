@@ -181,7 +181,7 @@ struct KnnArgs {
     uint32_t *nl_idx;
     float *nl_d2;
     unsigned long long *stats;  // work counters, may be null
-    uint32_t *amb;              // [0] count, [1..] ambiguous slots
+    uint32_t *amb;              // [0] count, [1..] slots for the resolver: ambiguous, or h not refined
     uint32_t *defer;            // [0] count, [1..] wavefronts (64 slots) left to the one-wavefront-per-query kernel
     uint32_t wlcap;             // leaf-record capacity used (<= WLCAP; smaller only as a test hook)
 };
@@ -231,45 +231,23 @@ MHIP_DEV double member_dist(const TreeView &t, const QPos &q, uint32_t p) {
     return pair_dist(d[0] * d[0] + d[1] * d[1] + d[2] * d[2]);
 }
 
-// One float64 step on the smoothing length over the final member list.  The
-// float32 solve before it leaves a relative error of ~1e-6 to 1e-5; the
-// derivative fits are sensitive to h through the weights of the outermost neighbours (d ln W / d ln h =
-// 3q / (1 - q) as q -> 1), so a 2.4e-7 error of h moves second-order
-// derivatives by up to ~6e-5.  The spline as truncated powers, W = 2 a^3 - b^3
-// with a = (1 - q)_+ and b = (1 - 2q)_+, gives W' = -6 (a^2 - b^2) and
-// W'' = 12 a - 24 b without branches, so Halley's step (cubic: third
-// derivatives of W are bounded) costs two more operations per neighbour than
-// Newton's and leaves h at the rounding level of the float64 sums.
-struct HsmlSums {
-    double w = 0.0, d1 = 0.0, d2 = 0.0;  // sums of W / 2, -W' q / 6, W'' q^2 / 12
-    MHIP_DEV void add(double q) {
-        const double a = fmax(1.0 - q, 0.0), b = fmax(fma(-2.0, q, 1.0), 0.0);
-        const double aa = a * a, bb = b * b, qc = fmin(q, 1.0);
-        w += fma(-0.5 * b, bb, a * aa);
-        const double t = (aa - bb) * qc;
-        d1 += t;
-        d2 = fma(fma(-2.0, b, a) * qc, qc, d2);
-    }
-};
-
-// the step from hd; a step beyond 1e-4 h means the float32 solve did not
-// converge: h is then kept
-MHIP_DEV double hsml_step64(const HsmlSums &s, double hd, int k, int dim) {
-    const double norm = hsml_norm(dim);
-    // n(h) = norm sum W(r_j / h) grows with h; p = h n'(h), c = h^2 n''(h)
-    const double f = norm * (2.0 * s.w) - (double)k;
-    const double p = norm * 6.0 * s.d1, c = norm * 12.0 * (s.d2 - s.d1);
-    const double rel = 2.0 * f * p / (2.0 * p * p - f * c);
-    return (p > 0.0 && fabs(rel) <= 1e-4) ? hd - hd * rel : hd;
-}
-
-// the whole step by one lane, member(j) giving the sorted index of member j < k
+// The float64 smoothing length by one lane, member(j) giving the sorted index of
+// member j < k: one step from the float32 solve.  flat: a step is not enough
+// (hsml_last); the row then goes to the resolver kernel, by the same list as the
+// ambiguous ones, which has a wavefront for it.
 template <bool PER, bool P64, typename F>
-MHIP_DEV double refine_h64(const KnnArgs &a, const QPos &q, double hd, F member) {
+MHIP_DEV double refine_h64(const KnnArgs &a, const QPos &q, double hd, bool &flat, F member) {
+    if (hsml_rootless(a.k, a.dim)) {
+        HsmlRange r;
+        for (int j = 0; j < a.k; j++) r.add(member_dist<PER, P64>(a.t, q, member(j)));
+        return r.r1;
+    }
     const double ih = 1.0 / hd;
     HsmlSums s;
     for (int j = 0; j < a.k; j++) s.add(member_dist<PER, P64>(a.t, q, member(j)) * ih);
-    return hsml_step64(s, hd, a.k, a.dim);
+    const HsmlStep st = hsml_halley(s, a.k, a.dim);
+    flat = !hsml_last(st, a.k, a.dim);
+    return flat ? hd : hd - hd * st.rel;
 }
 
 // Newton's step in the logarithms, ln n against ln h (n(h) is close to a power

@@ -66,6 +66,13 @@ MHIP_DEV float row_min(float x) {
     return fminf(x, ror_f<1>(x));
 }
 
+MHIP_DEV void row_join(HsmlRange &r) {
+    r.join(HsmlRange{ror_d<8>(r.r0), ror_d<8>(r.r1), ror_d<8>(r.rk)});
+    r.join(HsmlRange{ror_d<4>(r.r0), ror_d<4>(r.r1), ror_d<4>(r.rk)});
+    r.join(HsmlRange{ror_d<2>(r.r0), ror_d<2>(r.r1), ror_d<2>(r.rk)});
+    r.join(HsmlRange{ror_d<1>(r.r0), ror_d<1>(r.r1), ror_d<1>(r.rk)});
+}
+
 MHIP_DEV int lane_rank(uint64_t m) {  // set bits of m below this lane
     return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
 }
@@ -396,7 +403,7 @@ MHIP_DEV int32_t wave_search(const KnnArgs &a, int64_t slot, uint32_t qp, uint2 
 
 // Smoothing lengths of the wavefront's up to four queries, one per row of 16
 // lanes, MPL members per lane (16 MPL >= k): float64 distances of the members,
-// safeguarded float32 Newton, one float64 step (hsml_step64).  The same
+// safeguarded float32 Newton, one float64 step.  The same
 // control flow as the main kernel's solve.
 // SEED: a Newton seed per row (a.seed_h) may be given.
 template <int MPL, bool PER, bool P64, bool SEED>
@@ -472,18 +479,30 @@ MHIP_DEV void row_hsml(const KnnArgs &a, bool on, int64_t slot, uint32_t qp, flo
     if (run) st |= ST_HSML_NOCONV;
     double h64 = (double)h;
     const bool fine = on && h > 0.f && !(st & (ST_HSML_NOCONV | ST_AMBIGUOUS | ST_COUNT));
-    const double ih = fine ? 1.0 / h64 : 0.0;
-    HsmlSums s;
+    bool flat = false;  // (refine_h64)
+    if (hsml_rootless(k, a.dim)) {
+        HsmlRange r;
 #pragma unroll
-    for (int u = 0; u < MPL; u++) s.add(r64[u] * ih);
-    s.w = row_sum(s.w);
-    s.d1 = row_sum(s.d1);
-    s.d2 = row_sum(s.d2);
-    if (fine) h64 = hsml_step64(s, h64, k, a.dim);
+        for (int u = 0; u < MPL; u++)
+            if (u * 16 + rl < k) r.add(r64[u]);
+        row_join(r);
+        if (fine) h64 = r.r1;
+    } else {
+        const double ih = fine ? 1.0 / h64 : 0.0;
+        HsmlSums s;
+#pragma unroll
+        for (int u = 0; u < MPL; u++) s.add(r64[u] * ih);
+        s.w = row_sum(s.w);
+        s.d1 = row_sum(s.d1);
+        s.d2 = row_sum(s.d2);
+        const HsmlStep step = hsml_halley(s, k, a.dim);
+        flat = fine && !hsml_last(step, k, a.dim);
+        if (fine && !flat) h64 = h64 - h64 * step.rel;
+    }
     if (on && rl == 0) {
         write_h(a, slot, h64);
         a.st_slot[slot] = st;
-        if (st & ST_AMBIGUOUS) a.amb[1 + atomicAdd(a.amb, 1u)] = (uint32_t)slot;
+        if ((st & ST_AMBIGUOUS) || flat) a.amb[1 + atomicAdd(a.amb, 1u)] = (uint32_t)slot;
     }
 }
 
