@@ -21,6 +21,7 @@ ST_RADIUS_MISS = 128
 KNN_KEEP_DIST = 1
 KNN_SMALL_RECORD = 2  # test hook: every wavefront's leaf record overflows
 KNN_LANE = 4  # test hook: one lane per query whatever the sizes
+MAX_K = 128  # neighbours per particle
 NOALLOC_INTEGRATE_MAX_K = 64
 
 EXPORTED = [

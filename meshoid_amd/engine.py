@@ -119,8 +119,9 @@ class SpatialIndex:
             pos = pos[:, None]
         n, dim = pos.shape
         f64 = int(pos.dtype == torch.float64)
-        self._mem.reserve(lib.mhip_index_bytes(n, f64), pos.device,
-                          lambda p, b: lib.mhip_index_storage(self.h, p, b))
+        if 1 <= n < 2**32 - 1 and 1 <= dim <= 3:  # (else the library refuses, and what was built stays)
+            self._mem.reserve(lib.mhip_index_bytes(n, f64), pos.device,
+                              lambda p, b: lib.mhip_index_storage(self.h, p, b))
         ctx = context(pos.device, self)
         rc = lib.mhip_index_build(ctx, self.h, ptr(pos), f64, n, dim,
                                   float(boxsize) if boxsize else -1.0)
@@ -159,6 +160,7 @@ class NeighborList:
         self.k = 0
         self.index = None
         self.keep_dist = False
+        self.masked = False
 
     def _reserve(self, nq, k, masked, keep_dist, device):
         flags = _lib.KNN_KEEP_DIST if keep_dist else 0
@@ -217,7 +219,9 @@ def knn_hsml(index: SpatialIndex, k: int, qidx=None, m_rows=None, seed_h=None, k
     _need(seed_h, (torch.float32,), "seed_h")
     _need(seed_r, (torch.float32,), "seed_r")
     nq = index.n if qidx is None else qidx.numel()
-    if qidx is not None and nq and (int(qidx.min()) < 0 or int(qidx.max()) >= index.n):
+    if qidx is not None and nq == 0:
+        raise ValueError("no query rows")  # (an empty tensor's address is null, which means every particle)
+    if qidx is not None and (int(qidx.min()) < 0 or int(qidx.max()) >= index.n):
         raise IndexError("query index out of range")
     if m_rows is not None and m_rows.numel() != nq:
         raise ValueError("m_rows must have one entry per query row")
@@ -228,7 +232,8 @@ def knn_hsml(index: SpatialIndex, k: int, qidx=None, m_rows=None, seed_h=None, k
         out = {name: torch.empty(nq, dtype=torch.float32, device=dev) for name in ("h", "rho", "vol")}
         out["status"] = torch.empty(nq, dtype=torch.int32, device=dev)
     nl = nlist if nlist is not None else NeighborList()
-    nl._reserve(nq, int(k), qidx is not None, keep_dist, dev)
+    if 2 <= int(k) <= min(_lib.MAX_K, index.n):  # (else the library refuses, and a given list stays)
+        nl._reserve(nq, int(k), qidx is not None, keep_dist, dev)
     ctx = context(dev, nl, index)
     rc = lib.mhip_knn_hsml(ctx, index.h, ptr(qidx), nq, int(k), ptr(m_rows), ptr(seed_h),
                            ptr(seed_r), ptr(out.get("h")), ptr(out.get("rho")), ptr(out.get("vol")),
@@ -237,7 +242,7 @@ def knn_hsml(index: SpatialIndex, k: int, qidx=None, m_rows=None, seed_h=None, k
                            (_lib.KNN_LANE if lane else 0),
                            nl.h)
     raise_for(rc, ctx)
-    nl.nq, nl.k, nl.index, nl.keep_dist = nq, int(k), index, keep_dist
+    nl.nq, nl.k, nl.index, nl.keep_dist, nl.masked = nq, int(k), index, keep_dist, qidx is not None
     out["nlist"] = nl
     return out
 
@@ -260,11 +265,12 @@ def nlist_subset(full: NeighborList, qidx: torch.Tensor, m_rows=None, nlist: Nei
         out = {name: torch.empty(nq, dtype=torch.float32, device=dev) for name in ("h", "rho", "vol")}
         out["status"] = torch.empty(nq, dtype=torch.int32, device=dev)
     nl = nlist if nlist is not None else NeighborList()
-    nl._reserve(nq, full.k, True, full.keep_dist, dev)
+    if nq > 0 and nl is not full and not full.masked and full.nq == index.n:  # (else refused, as in knn_hsml)
+        nl._reserve(nq, full.k, True, full.keep_dist, dev)
     ctx = context(dev, nl, full, index)
     raise_for(lib.mhip_nlist_subset(ctx, full.h, ptr(qidx), nq, ptr(m_rows), ptr(out.get("h")),
                                     ptr(out.get("rho")), ptr(out.get("vol")), ptr(out.get("status")), nl.h), ctx)
-    nl.nq, nl.k, nl.index, nl.keep_dist = nq, full.k, index, full.keep_dist
+    nl.nq, nl.k, nl.index, nl.keep_dist, nl.masked = nq, full.k, index, full.keep_dist, True
     out["nlist"] = nl
     return out
 
