@@ -58,6 +58,10 @@ class _Memory:
         """At least need bytes on device; give(pointer, bytes) on a new block."""
         if self.block is not None and self.block.numel() >= need and self.block.device == device:
             return
+        if self.block is not None:
+            # the old block first: the two need not fit the card together
+            raise_for(give(None, 0), None, "storage")
+            self.block = None
         self.block = torch.empty(max(int(need), 1), dtype=torch.uint8, device=device)
         self.stream = torch.cuda.current_stream(device).cuda_stream
         raise_for(give(ctypes.c_void_p(self.block.data_ptr()), self.block.numel()), None, "storage")
