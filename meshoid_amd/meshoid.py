@@ -418,9 +418,10 @@ class Meshoid:
         return self._apply(f, 2, weighted, second=True)
 
     def _masked_rows(self, v):
-        """v[particle_mask]"""
-        if self._mask is None and self._mask_d is None and len(v) >= self.N:
-            return v[: self.N]
+        """v[particle_mask]; an array's rows as a view where that is all of them"""
+        if self._mask is None and self._mask_d is None and isinstance(v, (np.ndarray, torch.Tensor)):
+            if v.ndim and len(v) >= self.N:
+                return v[: self.N]
         return v[self.particle_mask]
 
     def Curl(self, v, correct_sign=False):
