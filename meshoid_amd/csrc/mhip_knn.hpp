@@ -264,10 +264,8 @@ MHIP_DEV void write_h(const KnnArgs &a, int64_t slot, double h) {
     a.h64_slot[slot] = h;
 }
 
-// one wavefront per query (mhip_knn_wave.hip): whether it is the faster kernel
-// for the whole set; its launch over every slot, or (deferred) over the
-// wavefronts in a.defer
-bool knn_wave_serves(int64_t n, int64_t nq, int k, int dim, bool per);
+// one wavefront per query (mhip_knn_wave.hip): its launch over every slot, or
+// (deferred) over the wavefronts in a.defer
 int knn_wave_launch(mhip_ctx *ctx, const KnnArgs &a, bool per, bool p64, bool deferred);
 
 }  // namespace mhip

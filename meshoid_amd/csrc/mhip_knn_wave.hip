@@ -1,6 +1,6 @@
 // Exact k-nearest-neighbour search with one wavefront per query, the smoothing
 // length and the member list (the results of k_knn_main in mhip_knn.hip, for
-// the sizes given at knn_wave_serves).
+// the sizes given at knn_wave_serves in mhip_knn_rules.hpp).
 //
 // The main kernel gives each lane a query and keeps its k + 1 smallest
 // distances in registers: a list insertion costs k + 1 instructions, and few
@@ -587,22 +587,6 @@ __global__ __launch_bounds__(64 * KW_WAVES) void k_knn_wave(KnnArgs a, uint32_t 
             __syncthreads();  // the next slots reuse s_out
         }
     }
-}
-
-// Where the lines lie (ms of the whole search, one lane / one wavefront per
-// query): k = 32 open 3D float32, 65536 particles 0.200 / 0.135, 10^5 0.212 /
-// 0.212, 3 10^5 0.369 / 0.560; 2D 32768 0.078 / 0.069, 65536 0.076 / 0.104;
-// k = 64 3D 3 10^5 0.69 / 0.68, 10^6 1.85 / 2.31; periodic float64 k = 32
-// 3 10^5 0.77 / 0.68, 10^6 1.90 / 2.28 (wavefronts near the faces come here
-// anyway); k = 100 10^6 3.31 / 2.84, clustered 2^22 16.0 / 13.7.  Few queries
-// in a large set lie far apart and share no leaves.
-bool knn_wave_serves(int64_t n, int64_t nq, int k, int dim, bool per) {
-    if (n >= (int64_t)1 << 28) return false;  // 16 threads a query; 32-bit byte offsets
-    if (k > 64 || nq < n / 4) return true;
-    int64_t most = dim == 3 ? 100000 : 45000;
-    if (k > 32) most *= 3;
-    if (per) most *= 3;
-    return n <= most;
 }
 
 template <int NR, int PW, int MODE, typename OFF>
