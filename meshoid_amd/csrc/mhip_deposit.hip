@@ -499,6 +499,18 @@ struct Map2 {
 
     // ---- tiles of WIN2^2 cells
     static constexpr int SIDE = WIN2;
+    // (ms by cells a tile, direct / tiles: 32768^2 630 3.3 / 5.9, 5000 14.0 / 9.5;
+    // 16384^2 800 2.1 / 2.6, 2500 2.3 / 2.1)
+    static constexpr int TILE_CELLS = 2000;
+    // this thread's share (of `stride`) of the cells, straight into the grid
+    static MHIP_DEV void spread(const DepArgs &a, const F &fp, double inv, int thread, int stride) {
+        const double f = fp.w * inv;
+        Walk2 w;
+        for (w.start(thread, stride, fp.gx0, fp.gy0, fp.gx1, fp.gy1); w.inside(); w.next()) {
+            const double k = cell_weight(a, fp, w.x, w.y);
+            if (k != 0.0) atomicAdd(&a.grid[(int64_t)w.x * a.res + w.y], k * f);
+        }
+    }
     static MHIP_DEV void box(const F &fp, int *lo, int *hi) {
         lo[0] = fp.gx0;
         hi[0] = fp.gx1;
@@ -641,17 +653,35 @@ __global__ __launch_bounds__(DEP_THREADS) void k_bin_deposit(typename P::Args a,
 // cell per lane, the cells inside.  Tile and particle meet by tests on boxes
 // of cells, 64 groups of 64 particles at once and then the particles of a
 // group, so no list of pairs is made; the particles are in brick order, so a
-// group's box is little larger than one footprint.
-// One block per particle adding each cell to HBM ran at the rate of float64
+// group's box is little larger than one footprint.  On large grids a tile would
+// meet a vanishing part of the groups, and the tests, tiles times groups, would
+// cost more than the deposit: there runs of 64 groups have boxes too, and only
+// the groups of those that meet the tile are tested (at least
+// WIDE_BLOCKS tiles; 2^22 particles 40 cells wide on a map of 32768^2 114 -> 17
+// ms, 12 cells wide in a volume of 1024^3 295 -> 64 ms).
+// One block per particle adding each cell to HBM runs at the rate of float64
 // atomics in L2, 1.1e11 a second; here they stay in LDS and each tile is added
-// once per block.
+// once per block.  That rate is the better one only where the tiles of a large
+// grid get few cells each (P::TILE_CELLS on average): a tile's tests, clearing and
+// reading cost as much as those atomics.  k_wide_boxes sums the footprints,
+// k_wide_direct or k_wide_tiles does the work.
 // ---------------------------------------------------------------------------
 struct Wide {
     const uint32_t *list;  // the particles, count of them from list[range[0]]
-    uint32_t *range;       // first, count
+    uint32_t *range;       // first, count; then room for cells (binned grids)
     int *boxes;            // (groups, 6): lowest and highest cell on each axis
+    int *runs;             // the same of each 64 groups; null: not tested
     double *inv;           // 1 / total weight by place in the list; null: plain shares
+    // sum of the footprints' cells (of a particle at most 2^31 counted); null:
+    // the tiles in any case
+    unsigned long long *cells;
 };
+
+// whether the wide particles are few enough to add their cells to HBM
+template <class P>
+MHIP_DEV bool wide_few(const Wide &wd, int64_t ntile) {
+    return wd.cells && *wd.cells < (unsigned long long)ntile * P::TILE_CELLS;
+}
 
 // first of the sorted keys (brick << SIZE_BITS | size) with brick >= k, by a
 // wavefront: 64 splits of the range at a time
@@ -676,6 +706,7 @@ __global__ __launch_bounds__(WAVE) void k_wide_range(const uint64_t *__restrict_
     if (threadIdx.x == 0) {
         range[0] = (uint32_t)lo;
         range[1] = (uint32_t)(hi - lo);
+        range[2] = range[3] = 0u;  // Wide::cells
     }
 }
 
@@ -699,12 +730,38 @@ __global__ __launch_bounds__(DEP_THREADS) void k_wide_boxes(typename P::Args a, 
         const int64_t e = (int64_t)g * WAVE + lane;
         typename P::F fp;
         int lo[3] = {INT32_MAX, INT32_MAX, INT32_MAX}, hi[3] = {INT32_MIN, INT32_MIN, INT32_MIN};
-        if (e < count && P::foot(a, wd.list[first + e], fp)) P::box(fp, lo, hi);
+        double cells = 0.0;
+        if (e < count && P::foot(a, wd.list[first + e], fp)) {
+            P::box(fp, lo, hi);
+            cells = 1.0;
+            for (int c = 0; c < 3; c++) cells *= (double)hi[c] - (double)lo[c] + 1.0;
+        }
+        if (wd.cells) {
+            cells = wave_sum(fmin(cells, 2147483648.0));
+            if (lane == 0) atomicAdd(wd.cells, (unsigned long long)cells);
+        }
         for (int c = 0; c < 3; c++) {
             const int l = wave_min_i(lo[c]), h = wave_max_i(hi[c]);
             if (lane == 0) {
                 wd.boxes[(size_t)g * 6 + c] = l;
                 wd.boxes[(size_t)g * 6 + 3 + c] = h;
+            }
+        }
+    }
+}
+
+// the boxes of each 64 groups, a wavefront per run
+__global__ __launch_bounds__(DEP_THREADS) void k_wide_runs(Wide wd) {
+    const int lane = threadIdx.x % WAVE;
+    const int64_t ng = ((int64_t)wd.range[1] + WAVE - 1) / WAVE, nrun = (ng + WAVE - 1) / WAVE;
+    const int64_t stride = (int64_t)gridDim.x * (DEP_THREADS / WAVE);
+    for (int64_t r = blockIdx.x * (int64_t)(DEP_THREADS / WAVE) + threadIdx.x / WAVE; r < nrun; r += stride) {
+        const int64_t g = min(r * WAVE + lane, ng - 1);
+        for (int c = 0; c < 3; c++) {
+            const int l = wave_min_i(wd.boxes[g * 6 + c]), h = wave_max_i(wd.boxes[g * 6 + 3 + c]);
+            if (lane == 0) {
+                wd.runs[r * 6 + c] = l;
+                wd.runs[r * 6 + 3 + c] = h;
             }
         }
     }
@@ -730,6 +787,18 @@ __global__ __launch_bounds__(DEP_THREADS) void k_wide_totals(typename P::Args a,
     }
 }
 
+// a block per particle, every cell added to the grid
+template <class P>
+__global__ __launch_bounds__(DEP_THREADS) void k_wide_direct(typename P::Args a, Wide wd, int64_t ntile) {
+    if (!wide_few<P>(wd, ntile)) return;
+    const uint32_t first = wd.range[0], count = wd.range[1];
+    for (uint32_t e = blockIdx.x; e < count; e += gridDim.x) {
+        typename P::F fp;
+        P::foot(a, wd.list[first + e], fp);  // listed, so it has a footprint
+        P::spread(a, fp, wd.inv ? wd.inv[e] : 1.0, threadIdx.x, DEP_THREADS);
+    }
+}
+
 // block b: tile b % ntile, groups b / ntile, + nslice, ... of the wide
 // particles (neighbouring groups meet the same tiles, so each of a tile's
 // blocks gets its share of them).  The block's four wavefronts go over the
@@ -738,38 +807,51 @@ template <class P>
 __global__ __launch_bounds__(DEP_THREADS) void k_wide_tiles(typename P::Args a, Wide wd, int nt, int64_t ntile,
                                                             int nslice) {
     __shared__ double win[WIN_CELLS];
+    if (wide_few<P>(wd, ntile)) return;
     const uint32_t first = wd.range[0], count = wd.range[1];
     const int64_t ng = ((int64_t)count + WAVE - 1) / WAVE;
+    // runs of 64 groups of this slice
+    const int64_t nrun = (ng + (int64_t)WAVE * nslice - 1) / ((int64_t)WAVE * nslice);
     const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
     for (int64_t b = blockIdx.x; b < ntile * nslice; b += gridDim.x) {
         const int slice = (int)(b / ntile);
         int t0[3];
         P::corner(b % ntile, nt, t0);
+        // whether 64 groups, and this lane's of them, meet the tile
+        auto run_meets = [&](int64_t r) {
+            return r < nrun && (!wd.runs || P::meets(a, wd.runs + r * 6, wd.runs + r * 6 + 3, t0));
+        };
+        auto group_meets = [&](int64_t g) {
+            return g < ng && P::meets(a, wd.boxes + g * 6, wd.boxes + g * 6 + 3, t0);
+        };
         bool any = false;
-        for (int64_t g = slice + (int64_t)nslice * threadIdx.x; g < ng && !any; g += (int64_t)nslice * DEP_THREADS)
-            any = P::meets(a, wd.boxes + g * 6, wd.boxes + g * 6 + 3, t0);
+        for (int64_t r0 = wave * WAVE; r0 < nrun && !any; r0 += DEP_THREADS)
+            for (uint64_t rs = __ballot(run_meets(r0 + lane)); rs && !any; rs &= rs - 1)
+                any = __any(group_meets(((r0 + __builtin_ctzll(rs)) * WAVE + lane) * nslice + slice));
         if (!__syncthreads_or(any)) continue;
         for (int c = threadIdx.x; c < WIN_CELLS; c += DEP_THREADS) win[c] = 0.0;
         __syncthreads();
-        for (int64_t g0 = slice; g0 < ng; g0 += (int64_t)nslice * WAVE) {
-            const int64_t g = g0 + (int64_t)nslice * lane;
-            const bool near = g < ng && P::meets(a, wd.boxes + g * 6, wd.boxes + g * 6 + 3, t0);
-            for (uint64_t gs = __ballot(near); gs; gs &= gs - 1) {
-                const int64_t e = (g0 + (int64_t)nslice * __builtin_ctzll(gs)) * WAVE + lane;
-                typename P::F fp;
-                double inv = 1.0;
-                bool take = e < count && lane % (DEP_THREADS / WAVE) == wave && P::foot(a, wd.list[first + e], fp);
-                if (take) {
-                    int lo[3], hi[3];
-                    P::box(fp, lo, hi);
-                    take = P::meets(a, lo, hi, t0);
-                    if (wd.inv) {
-                        inv = wd.inv[e];
-                        take = take && inv != 0.0;
+        for (int64_t r0 = 0; r0 < nrun; r0 += WAVE) {
+            for (uint64_t rs = __ballot(run_meets(r0 + lane)); rs; rs &= rs - 1) {
+                const int64_t g0 = (r0 + __builtin_ctzll(rs)) * WAVE * nslice + slice;
+                const bool near = group_meets(g0 + (int64_t)nslice * lane);
+                for (uint64_t gs = __ballot(near); gs; gs &= gs - 1) {
+                    const int64_t e = (g0 + (int64_t)nslice * __builtin_ctzll(gs)) * WAVE + lane;
+                    typename P::F fp;
+                    double inv = 1.0;
+                    bool take = e < count && lane % (DEP_THREADS / WAVE) == wave && P::foot(a, wd.list[first + e], fp);
+                    if (take) {
+                        int lo[3], hi[3];
+                        P::box(fp, lo, hi);
+                        take = P::meets(a, lo, hi, t0);
+                        if (wd.inv) {
+                            inv = wd.inv[e];
+                            take = take && inv != 0.0;
+                        }
                     }
+                    for (uint64_t ps = __ballot(take); ps; ps &= ps - 1)
+                        P::tile_wave(a, fp, inv, __builtin_ctzll(ps), t0, win);
                 }
-                for (uint64_t ps = __ballot(take); ps; ps &= ps - 1)
-                    P::tile_wave(a, fp, inv, __builtin_ctzll(ps), t0, win);
             }
         }
         __syncthreads();
@@ -787,16 +869,26 @@ __global__ __launch_bounds__(DEP_THREADS) void k_wide_tiles(typename P::Args a, 
 // (Map of 1024^2: 2048, 4096, 8192 blocks 2.61, 2.50, 2.62 ms.)
 constexpr int64_t WIDE_BLOCKS = 4096;
 template <class P>
-void wide_deposit(mhip_ctx *ctx, typename P::Args a, const Wide &wd, int64_t ntile) {
+void wide_deposit(mhip_ctx *ctx, typename P::Args a, Wide wd, int64_t ntile) {
     hipStream_t s = ctx->stream;
     const int64_t ng = (a.n + WAVE - 1) / WAVE;
     const int nt = (a.res + P::SIDE - 1) / P::SIDE;
     const int nslice = (int)std::min<int64_t>(ng, std::max<int64_t>(1, WIDE_BLOCKS / ntile));
+    const bool large = ntile >= WIDE_BLOCKS;
+    if (large) wd.cells = (unsigned long long *)(wd.range + 2);
     hipLaunchKernelGGL(k_wide_boxes<P>, dim3((unsigned)std::min<int64_t>(1024, (ng + 3) / 4)), dim3(DEP_THREADS), 0, s,
                        a, wd);
+    if (large) {
+        wd.runs = wd.boxes + ng * 6;
+        hipLaunchKernelGGL(k_wide_runs, dim3((unsigned)std::min<int64_t>(1024, (ng / WAVE + 4) / 4)), dim3(DEP_THREADS),
+                           0, s, wd);
+    }
     if (wd.inv)
         hipLaunchKernelGGL(k_wide_totals<P>, dim3((unsigned)std::min<int64_t>(4096, a.n)), dim3(DEP_THREADS), 0, s, a,
                            wd);
+    if (large)
+        hipLaunchKernelGGL(k_wide_direct<P>, dim3((unsigned)std::min<int64_t>(4096, a.n)), dim3(DEP_THREADS), 0, s, a,
+                           wd, ntile);
     hipLaunchKernelGGL(k_wide_tiles<P>, dim3((unsigned)std::min<int64_t>(1 << 22, ntile * nslice)), dim3(DEP_THREADS),
                        0, s, a, wd, nt, ntile, nslice);
 }
@@ -804,14 +896,14 @@ void wide_deposit(mhip_ctx *ctx, typename P::Args a, const Wide &wd, int64_t nti
 // bits of a sort key in [0, top]
 static int key_bits(uint32_t top) { return 64 - __builtin_clzll((unsigned long long)top | 1ull); }
 
-// words the boxes of n particles take
-static size_t box_words(int64_t n) { return ((size_t)n / WAVE + 1) * 6; }
+// words the boxes of n particles' groups and runs take
+static size_t box_words(int64_t n) { return ((size_t)n / WAVE + 1 + (size_t)n / (WAVE * WAVE) + 1) * 6; }
 // scratch for n particles: keys 16 n, values 8 n (room for the boxes), radix
 // counts, the wide particles' range.  The totals and boxes take the halves of
 // the keys and values that the sort leaves free.
 static size_t val_words(int64_t n) { return std::max((size_t)n, box_words(n)); }
 static size_t bin_scratch_bytes(int64_t n) {
-    return (size_t)n * 16 + val_words(n) * 8 + radix_counts_words(std::max<int64_t>(n, 1)) * 4 + 8 + 64;
+    return (size_t)n * 16 + val_words(n) * 8 + radix_counts_words(std::max<int64_t>(n, 1)) * 4 + 16 + 64;
 }
 
 // the binned path: keys, sort, runs, then the tiles of the wide particles
@@ -820,7 +912,7 @@ int bin_deposit(mhip_ctx *ctx, typename P::Args a, uint32_t skip, int64_t ntile,
     const int64_t n = a.n;
     if (n <= 0) return 0;
     uint64_t *k0 = (uint64_t *)sc, *k1 = k0 + n;
-    uint32_t *v0 = (uint32_t *)(k1 + n), *v1 = v0 + val_words(n), *range = v1 + val_words(n), *counts = range + 2;
+    uint32_t *v0 = (uint32_t *)(k1 + n), *v1 = v0 + val_words(n), *range = v1 + val_words(n), *counts = range + 4;
     hipStream_t s = ctx->stream;
     hipLaunchKernelGGL(k_bin_keys<P>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a, k0, v0);
     uint64_t *ks;
@@ -830,7 +922,8 @@ int bin_deposit(mhip_ctx *ctx, typename P::Args a, uint32_t skip, int64_t ntile,
     hipLaunchKernelGGL(k_bin_deposit<P>, dim3((unsigned)((n + BIN_CHUNK - 1) / BIN_CHUNK)), dim3(DEP_THREADS), 0, s,
                        a, ks, vs);
     hipLaunchKernelGGL(k_wide_range, dim3(1), dim3(WAVE), 0, s, ks, n, skip, range);
-    const Wide wd{vs, range, (int *)(vs == v0 ? v1 : v0), conservative ? (double *)(ks == k0 ? k1 : k0) : nullptr};
+    const Wide wd{vs, range, (int *)(vs == v0 ? v1 : v0), nullptr, conservative ? (double *)(ks == k0 ? k1 : k0) : nullptr,
+                  nullptr};
     wide_deposit<P>(ctx, a, wd, ntile);
     return 0;
 }
@@ -1086,6 +1179,17 @@ struct Vol3 {
     // ---- tiles of WIN3^3 cells; a periodic footprint meets a tile once for
     // each m with cells of it shifted by m res inside
     static constexpr int SIDE = WIN3;
+    // (ms by cells a tile, direct / tiles: 1024^3 450 7.7 / 14.0, 3600 21.5 / 30.0,
+    // 14500 67.5 / 64.2; 512^3 3600 2.7 / 3.1, 29000 16.4 / 12.4)
+    static constexpr int TILE_CELLS = 8000;
+    static MHIP_DEV void spread(const Dep3Args &a, const F &fp, double inv, int thread, int stride) {
+        const double f = fp.f * inv;
+        Walk3 w;
+        for (w.start(thread, stride, fp.g0, fp.g1); w.inside(); w.next()) {
+            const double k = weight3(a, fp, w.x, w.y, w.z);
+            if (k != 0.0) atomicAdd(&a.grid[cell3(a, w.x, w.y, w.z)], k * f);
+        }
+    }
     static MHIP_DEV int floor_div(int x, int d) { return x >= 0 ? x / d : -1 - (-1 - x) / d; }
     static MHIP_DEV void box(const F &fp, int *lo, int *hi) {
         for (int c = 0; c < 3; c++) {
@@ -1242,7 +1346,7 @@ int surface_density(mhip_ctx *ctx, const void *f, int f_f64, const void *pos, in
             hipLaunchKernelGGL(k_range_zero, dim3(1), dim3(WAVE), 0, s, range);
             hipLaunchKernelGGL(k_deposit_tiles, dim3((unsigned)nchunk), dim3(DEP_THREADS), lds, s, a, res, 1,
                                (int)nchunk);
-            const Wide wd{a.big, range, (int *)(a.big + n), conservative ? (double *)sc : nullptr};
+            const Wide wd{a.big, range, (int *)(a.big + n), nullptr, conservative ? (double *)sc : nullptr, nullptr};
             wide_deposit<Map2>(ctx, a, wd, nt * nt);
         } else {
             // binned by 32^2 bricks (per-tile LDS copies of the map would
