@@ -279,7 +279,10 @@ struct MaskStack {
 constexpr int LROWS = 33;                          // staged member rows (k <= 32)
 constexpr int QROWS = QCAP > LROWS ? QCAP : LROWS;  // per-lane LDS rows
 
-template <int KCAP, bool P64>
+// SPLIT: wavefronts whose queries lie far apart are the other kernel's
+// (knn_splits).  An instantiation of its own: the test alone, through the
+// allocation of scalar registers, made whole sets 3.4% slower (2^24, k = 32).
+template <int KCAP, bool P64, bool SPLIT>
 __global__ __launch_bounds__(KNN_BLOCK) void k_knn_main(KnnArgs a) {
     // members are staged in LDS and written as whole rows when they fit
     constexpr bool STAGE = KCAP <= LROWS;
@@ -297,6 +300,7 @@ __global__ __launch_bounds__(KNN_BLOCK) void k_knn_main(KnnArgs a) {
     const bool missed = a.redo && live && (a.st_slot[qs_slot] & ST_RADIUS_MISS);
     if (a.redo && !__any(missed)) return;
     const uint32_t qp = a.qsorted ? a.qsorted[qs_slot] : (uint32_t)qs_slot;
+    if (SPLIT && uniform(__shfl(qp, WAVE - 1)) - uniform(__shfl(qp, 0)) > KNN_SPREAD) return;
     const uint32_t row = a.qrow ? a.qrow[qs_slot] : a.perm[qs_slot];
     // a radius seed starts the k+1 slots at (seed radius)^2 instead of +inf: a
     // lane whose (k+1)-th slot still holds that bound at the end missed
@@ -1064,10 +1068,16 @@ __global__ __launch_bounds__(256) void k_rows_split(const RowRec *__restrict__ r
 
 template <int KCAP>
 static void launch_main(const KnnArgs &a, bool p64, dim3 g, hipStream_t s) {
-    if (p64)
-        hipLaunchKernelGGL((k_knn_main<KCAP, true>), g, dim3(KNN_BLOCK), 0, s, a);
+    // (larger k of a split set are the other kernel's altogether)
+    constexpr bool MAY = KCAP <= 65;
+    if (p64 && MAY && a.split)
+        hipLaunchKernelGGL((k_knn_main<KCAP, true, MAY>), g, dim3(KNN_BLOCK), 0, s, a);
+    else if (MAY && a.split)
+        hipLaunchKernelGGL((k_knn_main<KCAP, false, MAY>), g, dim3(KNN_BLOCK), 0, s, a);
+    else if (p64)
+        hipLaunchKernelGGL((k_knn_main<KCAP, true, false>), g, dim3(KNN_BLOCK), 0, s, a);
     else
-        hipLaunchKernelGGL((k_knn_main<KCAP, false>), g, dim3(KNN_BLOCK), 0, s, a);
+        hipLaunchKernelGGL((k_knn_main<KCAP, false, false>), g, dim3(KNN_BLOCK), 0, s, a);
 }
 
 static void launch_main_k(const KnnArgs &a, bool p64, dim3 g, hipStream_t s) {
@@ -1193,6 +1203,7 @@ int knn_run(mhip_ctx *ctx, const mhip_index *ix, const int64_t *qidx, int64_t nq
     a.stats = ctx->prof >= 2 ? ctx->stats : nullptr;
     a.amb = nl->amb;
     a.defer = nl->defer;
+    a.split = false;
     a.wlcap = (flags & MHIP_KNN_SMALL_RECORD) ? 8u : (uint32_t)WLCAP;
     const bool p64 = ix->pos_f64 != 0;
     const dim3 g((unsigned)((nq + KNN_BLOCK - 1) / KNN_BLOCK));
@@ -1205,7 +1216,10 @@ int knn_run(mhip_ctx *ctx, const mhip_index *ix, const int64_t *qidx, int64_t nq
     if (wave) {
         if ((rc = knn_wave_launch(ctx, a, per, p64, false))) return rc;
     } else {
+        if (!seed_h && !seed_r && !(flags & (MHIP_KNN_SMALL_RECORD | MHIP_KNN_LANE)))
+            a.split = knn_splits(ix->n, nq, k, ix->dim, per);
         launch_main_k(a, p64, g, s);
+        if (a.split && (rc = knn_wave_launch(ctx, a, per, p64, false))) return rc;
         if (seed_r) {
             // second launch: waves with a radius-seed miss are recomputed plainly
             KnnArgs r = a;

@@ -183,6 +183,7 @@ struct KnnArgs {
     unsigned long long *stats;  // work counters, may be null
     uint32_t *amb;              // [0] count, [1..] slots for the resolver: ambiguous, or h not refined
     uint32_t *defer;            // [0] count, [1..] wavefronts (64 slots) left to the one-wavefront-per-query kernel
+    bool split;                 // wavefronts shared out between the kernels (knn_splits)
     uint32_t wlcap;             // leaf-record capacity used (<= WLCAP; smaller only as a test hook)
 };
 

@@ -576,7 +576,12 @@ __global__ __launch_bounds__(64 * KW_WAVES) void k_knn_wave(KnnArgs a, uint32_t 
     constexpr uint32_t PARTS = WAVE / NCOL;
     auto part = [&](uint32_t b) { return (int64_t)a.defer[1 + b / PARTS] * WAVE + b % PARTS * NCOL; };
     if constexpr (MODE == KW_ALL) {
-        serve((int64_t)xcd_remap(blockIdx.x, gridDim.x) * NCOL);
+        const int64_t slot0 = (int64_t)xcd_remap(blockIdx.x, gridDim.x) * NCOL;
+        if (a.split) {  // (qsorted is given then)
+            const int64_t s0 = slot0 & ~(int64_t)(WAVE - 1);
+            if (a.qsorted[min(s0 + WAVE - 1, a.nq - 1)] - a.qsorted[s0] <= KNN_SPREAD) return;
+        }
+        serve(slot0);
     } else if constexpr (MODE == KW_LIST) {
         const uint32_t b = first + blockIdx.x;
         if (b < a.defer[0] * PARTS) serve(part(b));
