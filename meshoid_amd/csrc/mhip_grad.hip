@@ -17,6 +17,7 @@
 #include <type_traits>
 
 #include "mhip_internal.hpp"
+#include "mhip_knn.hpp"
 #include "mhip_linalg.hpp"
 
 namespace mhip {
@@ -57,17 +58,6 @@ MHIP_DEV void pair_offset(const ApplyArgs &a, const float (&c)[3], const float (
 // per query: 1.97 ms, against 2.31 with 2 and 2.42 with 4 per batch).
 template <int ORDER>
 constexpr int apply_nb() { return ORDER == 1 ? 1 : 4; }
-
-// pair_dist by one Newton step on the root (4.1e-15 off at most): the weights of
-// a fit, whose results are float32.  (Against sqrt, apply_D1 2.27 -> 2.05 ms at
-// 2^24 with four lanes per query.)
-MHIP_DEV double fit_dist(double r2) {
-    if (r2 < 1e-280) return sqrt(r2);
-    const double y = __builtin_amdgcn_rsq(r2);
-    const double r = r2 * y;
-    const double res = fma(-r, r, r2);
-    return fma(0.5 * y, res, r);
-}
 
 __global__ __launch_bounds__(256) void k_pack_xyzf(const float *__restrict__ sx, const float *__restrict__ sy,
                                                   const float *__restrict__ sz, const float *__restrict__ f0,

@@ -779,7 +779,7 @@ MHIP_DEV void refine_slot(const KnnArgs &a, const QPos &q, int64_t slot) {
 #pragma unroll
     for (int u = 0; u < 2; u++)
         if (u * WAVE + lane < a.k)
-            r[u] = member_dist<PER, P64>(a.t, q, a.nl_idx[(int64_t)(u * WAVE + lane) * a.nq + slot]);
+            r[u] = member_dist<PER, P64, true>(a.t, q, a.nl_idx[(int64_t)(u * WAVE + lane) * a.nq + slot]);
     const double h = hsml_refine(
         a.h64_slot[slot], a.k, a.dim,
         [&](double x) {
@@ -971,8 +971,12 @@ MHIP_DEV void resolve_slot(const KnnArgs &a, const PT *__restrict__ pos_in, int6
         if (total != a.k) pad_list(a, min(total, a.k), qp, slot);
         a.st_slot[slot] = st;
     }
+    bool flat = false;
+    if (lane == 0 && total == a.k && h0 > 0.f && !(st & ST_HSML_NOCONV))
+        write_h(a, slot, refine_h64<PER, P64>(a, q, (double)h0, flat,
+                                              [&](int j) { return a.nl_idx[(int64_t)j * nq + slot]; }));
     __syncthreads();
-    if (total == a.k && h0 > 0.f && !(st & ST_HSML_NOCONV)) refine_slot<PER, P64>(a, q, slot);
+    if (__any(flat)) refine_slot<PER, P64>(a, q, slot);
 }
 
 // empties the lists of ambiguous slots and of deferred wavefronts (a kernel,

@@ -202,9 +202,8 @@ MHIP_DEV void pad_list(const KnnArgs &a, int cnt, uint32_t qp, int64_t slot) {
 // |d| from r2 = |d|^2 (float64): the hardware reciprocal square root (5.2e-8 off
 // at most) and one third-order step, without the scaling and fix-up
 // instructions of the correctly rounded root: 1.7e-16 off at most over 2^22
-// values (a Newton step is one instruction less and 4.1e-15 off).  Tiny r2
-// (float64 inputs at pathological scales, where the estimate would meet
-// denormals) take sqrt.
+// values.  Tiny r2 (float64 inputs at pathological scales, where the estimate
+// would meet denormals) take sqrt.
 MHIP_DEV double pair_dist(double r2) {
     if (r2 < 1e-280) return sqrt(r2);
     const double y = __builtin_amdgcn_rsq(r2);
@@ -212,10 +211,22 @@ MHIP_DEV double pair_dist(double r2) {
     const double e = fma(-r, y, 1.0);
     return fma(r * e, fma(0.375, e, 0.5), r);
 }
+// The same by one Newton step on the root, 4.1e-15 off at most: the weights of a
+// fit, whose results are float32, and the one step of the smoothing length,
+// which moves by no more than its distances do.  (Against sqrt, apply_D1 2.27 ->
+// 2.05 ms at 2^24 with four lanes per query.)
+MHIP_DEV double fit_dist(double r2) {
+    if (r2 < 1e-280) return sqrt(r2);
+    const double y = __builtin_amdgcn_rsq(r2);
+    const double r = r2 * y;
+    const double res = fma(-r, r, r2);
+    return fma(0.5 * y, res, r);
+}
 
-// float64 offset of member p from the query: exact for float32 positions,
-// hi + lo for float64 inputs, minimum image when periodic
-template <bool PER, bool P64>
+// float64 distance of member p from the query: exact offsets for float32
+// positions, hi + lo for float64 inputs, minimum image when periodic.  FINE: the
+// root by pair_dist (a row's bracket, and rows where n(h) is flat)
+template <bool PER, bool P64, bool FINE>
 MHIP_DEV double member_dist(const TreeView &t, const QPos &q, uint32_t p) {
     double d[3] = {(double)t.sx[p] - ((double)q.x + (double)q.lx), (double)t.sy[p] - ((double)q.y + (double)q.ly),
                    (double)t.sz[p] - ((double)q.z + (double)q.lz)};
@@ -229,7 +240,8 @@ MHIP_DEV double member_dist(const TreeView &t, const QPos &q, uint32_t p) {
 #pragma unroll
         for (int c = 0; c < 3; c++) d[c] = wrap<double>(d[c], box);
     }
-    return pair_dist(d[0] * d[0] + d[1] * d[1] + d[2] * d[2]);
+    const double r2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
+    return FINE ? pair_dist(r2) : fit_dist(r2);
 }
 
 // The float64 smoothing length by one lane, member(j) giving the sorted index of
@@ -240,12 +252,12 @@ template <bool PER, bool P64, typename F>
 MHIP_DEV double refine_h64(const KnnArgs &a, const QPos &q, double hd, bool &flat, F member) {
     if (hsml_rootless(a.k, a.dim)) {
         HsmlRange r;
-        for (int j = 0; j < a.k; j++) r.add(member_dist<PER, P64>(a.t, q, member(j)));
+        for (int j = 0; j < a.k; j++) r.add(member_dist<PER, P64, true>(a.t, q, member(j)));
         return r.r1;
     }
     const double ih = 1.0 / hd;
     HsmlSums s;
-    for (int j = 0; j < a.k; j++) s.add(member_dist<PER, P64>(a.t, q, member(j)) * ih);
+    for (int j = 0; j < a.k; j++) s.add(member_dist<PER, P64, false>(a.t, q, member(j)) * ih);
     const HsmlStep st = hsml_halley(s, a.k, a.dim);
     flat = !hsml_last(st, a.k, a.dim);
     return flat ? hd : hd - hd * st.rel;

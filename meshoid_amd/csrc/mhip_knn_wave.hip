@@ -419,7 +419,7 @@ MHIP_DEV void row_hsml(const KnnArgs &a, bool on, int64_t slot, uint32_t qp, flo
     for (int u = 0; u < MPL; u++) {
         const int j = u * 16 + rl;
         r64[u] = 1e300;
-        if (j < k) r64[u] = member_dist<PER, P64>(t, q, s_out[j * ncol + col]);
+        if (j < k) r64[u] = member_dist<PER, P64, false>(t, q, s_out[j * ncol + col]);
         mn = fminf(mn, fminf((float)r64[u], 3e38f));
     }
     // bracket [r_1, c_d r_(k-1)] of the reference: r_1 is the second smallest
@@ -484,7 +484,7 @@ MHIP_DEV void row_hsml(const KnnArgs &a, bool on, int64_t slot, uint32_t qp, flo
         HsmlRange r;
 #pragma unroll
         for (int u = 0; u < MPL; u++)
-            if (u * 16 + rl < k) r.add(r64[u]);
+            if (u * 16 + rl < k) r.add(member_dist<PER, P64, true>(t, q, s_out[(u * 16 + rl) * ncol + col]));
         row_join(r);
         if (fine) h64 = r.r1;
     } else {
