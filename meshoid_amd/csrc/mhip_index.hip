@@ -542,8 +542,14 @@ int index_build(mhip_ctx *ctx, const void *pos, int pos_f64, int64_t n, int dim,
     const int nbb = 1024;
     size_t off_k0 = 0, off_k1 = off_k0 + n * 8, off_v0 = off_k1 + n * 8, off_v1 = off_v0 + n * 4,
            off_c = off_v1 + n * 4, off_bb = off_c + cw * 4, total = off_bb + (nbb + 2) * 8 * 4;
+    // (a build that fails from here on leaves the index empty: its arrays are
+    // those of the new set, and a caller may hold outputs sized for the old one)
+    auto failed = [&](int code) {
+        ix->n = 0;
+        return code;
+    };
     char *s = (char *)scratch(ctx, total, &rc);
-    if (!s) return rc;
+    if (!s) return failed(rc);
     uint64_t *k0 = (uint64_t *)(s + off_k0), *k1 = (uint64_t *)(s + off_k1);
     uint32_t *v0 = (uint32_t *)(s + off_v0), *v1 = (uint32_t *)(s + off_v1);
     uint32_t *counts = (uint32_t *)(s + off_c);
@@ -575,7 +581,7 @@ int index_build(mhip_ctx *ctx, const void *pos, int pos_f64, int64_t n, int dim,
     uint32_t *vs;
     if ((rc = radix_sort_pairs(ctx, k0, v0, k1, v1, counts, n, KEY_BITS_PER_AXIS * dim, &ks, &vs,
                                key_sort_lo_bit(dim))))
-        return rc;
+        return failed(rc);
     pr_key.end();
     ProfRegion pr_g(ctx, "index_reorder_boxes");
     const dim3 gp((unsigned)((npad + 255) / 256));
@@ -598,7 +604,7 @@ int index_build(mhip_ctx *ctx, const void *pos, int pos_f64, int64_t n, int dim,
                            ix->nodes, x0, cnt);
     }
     pr_g.end();
-    if ((rc = check_hip(ctx, hipGetLastError(), "index build launch"))) return rc;
+    if ((rc = check_hip(ctx, hipGetLastError(), "index build launch"))) return failed(rc);
     if (rec) {
         // deferred: the caller reads the record (bbox, NaN flag, frame) later;
         // the host copies are unknown until then
@@ -610,17 +616,16 @@ int index_build(mhip_ctx *ctx, const void *pos, int pos_f64, int64_t n, int dim,
     float hb[12];
     if ((rc = check_hip(ctx, hipMemcpyAsync(hb, bb, 12 * sizeof(float), hipMemcpyDeviceToHost,
                                             ctx->stream), "bbox readback")))
-        return rc;
-    if ((rc = check_hip(ctx, hipStreamSynchronize(ctx->stream), "index build"))) return rc;
+        return failed(rc);
+    if ((rc = check_hip(ctx, hipStreamSynchronize(ctx->stream), "index build"))) return failed(rc);
     for (int c = 0; c < 6; c++) ix->bbox[c] = hb[c];
     for (int c = 0; c < 4; c++) ix->frame[c] = hb[8 + c];
-    if (hb[6] != 0.f) return fail(ctx, -1, "positions contain NaN");
+    if (hb[6] != 0.f) return failed(fail(ctx, -1, "positions contain NaN"));
     if (box > 0) {
         for (int c = 0; c < dim; c++)
             // float64 data just below box can round up to box in float32
             if (hb[c] < 0.f || hb[3 + c] > (float)box || (hb[3 + c] == (float)box && !pos_f64))
-                return fail(ctx, -1,
-                            "Some input data are greater than the size of the periodic box.");
+                return failed(fail(ctx, -1, "Some input data are greater than the size of the periodic box."));
     }
     return 0;
 }

@@ -1183,7 +1183,10 @@ int knn_run(mhip_ctx *ctx, const mhip_index *ix, const int64_t *qidx, int64_t nq
     // query slots in Hilbert order
     const bool masked = qidx != nullptr;
     nl->masked = masked;
-    if (masked && (rc = query_setup(ctx, ix, qidx, nq, nl))) return rc;
+    if (masked && (rc = query_setup(ctx, ix, qidx, nq, nl))) {
+        nl->nq = 0;
+        return rc;
+    }
     KnnArgs a;
     a.t = tree_view(ix);
     const bool per = ix->box > 0;
@@ -1384,7 +1387,10 @@ int nlist_subset(mhip_ctx *ctx, const mhip_nlist *full, const int64_t *qidx, int
     nl->index = ix;
     nl->has_d2 = full->has_d2;
     nl->masked = true;
-    if ((rc = query_setup(ctx, ix, qidx, nq, nl))) return rc;
+    if ((rc = query_setup(ctx, ix, qidx, nq, nl))) {
+        nl->nq = 0;
+        return rc;
+    }
     ProfRegion pr(ctx, "nlist_subset");
     hipLaunchKernelGGL(k_nl_subset, dim3((unsigned)((nq + 255) / 256)), dim3(256), 0, ctx->stream, full->idx,
                        full->has_d2 ? full->d2 : nullptr, full->tau, full->h, full->h64, full->status,

@@ -56,3 +56,28 @@ def test_storage_alignment_is_checked():
             assert fn(o.h, ctypes.c_void_p(mem.data_ptr() + off), 1 << 16) == -1
         assert fn(o.h, ctypes.c_void_p(mem.data_ptr() + 16), 1 << 16) == 0
         assert fn(o.h, None, 0) == 0
+
+
+@pytest.mark.parametrize("bad", ["nan", "outside"])
+def test_failed_build_leaves_the_index_empty(bad):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from meshoid_amd import engine
+    from meshoid_amd._lib import lib
+
+    p = torch.rand(1000, 3, device="cuda")
+    ix = engine.SpatialIndex().build(p, 1.0)
+    want = engine.knn_hsml(ix, 8)["nlist"].export(f64=True)
+    q = torch.rand(50000, 3, device="cuda")
+    q[77] = float("nan") if bad == "nan" else 1.5
+    with pytest.raises(ValueError):
+        ix.build(q, 1.0)
+    n = ctypes.c_int64(-1)
+    assert lib.mhip_index_info(ix.h, ctypes.byref(n), None, None, None) == 0
+    assert n.value == 0  # (outputs of 1000 rows below: the calls must not reach the device)
+    with pytest.raises(ValueError):
+        engine.knn_hsml(ix, 8)
+    with pytest.raises(ValueError):
+        engine.nearest(ix, torch.rand(10, 3, device="cuda", dtype=torch.float64))
+    got = engine.knn_hsml(ix.build(p, 1.0), 8)["nlist"].export(f64=True)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
