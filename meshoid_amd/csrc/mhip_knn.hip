@@ -32,10 +32,10 @@
 //       not give (rows where n(h) is flat at the root, see hsml_last).
 //   Wavefronts whose queries spread over a large region, and in periodic sets
 //   those whose balls reach a face of the box, are left to the other kernel.
-// It is bound by vector instructions: 27.9k a wavefront at 2^24 clustered
+// It is bound by vector instructions: 28.1k a wavefront at 2^24 clustered
 // particles, k = 32 (70 leaves x 143, 20 runs of 16 through the networks x
 // 306, 3.5 smoothing-length iterations x 415, 16 member steps x 157), the
-// vector units 90% busy; 14.5 ms, against 20.0 ms and 43.3k with one insertion
+// vector units 79% busy; 14.3 ms, against 20.0 ms and 43.3k with one insertion
 // step per queued row, 8 child boxes tested by all lanes per node and
 // compensated branches in the smoothing length.
 #include "../../include/meshoid_hip.h"
